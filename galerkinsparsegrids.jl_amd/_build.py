@@ -24,18 +24,28 @@ HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", f"-I{ROOT / 'include'}", f"-I{CSRC}"]
 HIPFLAGS = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
+# (source, HIP, part): a source with parts is compiled once per part (GSG_PART), the
+# parts side by side
 SOURCES = [
-    ("gsg_setup.cpp", False),
-    ("gsg_capi.cpp", True),
-    ("gsg_kernels.hip", True),
+    ("gsg_setup.cpp", False, None),
+    ("gsg_capi.cpp", True, None),
+    ("gsg_kernels.hip", True, 0),
+    ("gsg_kernels.hip", True, 1),
+    ("gsg_kernels.hip", True, 2),
+    ("gsg_kernels.hip", True, 3),
+    ("gsg_kernels.hip", True, 4),
 ]
 
 
-def _compile(src: str, hip: bool, verbose: bool) -> Path:
-    out = OBJ / (Path(src).stem + ".o")
+def _object(src: str, part) -> Path:
+    return OBJ / (Path(src).stem + ("" if part is None else f"_{part}") + ".o")
+
+
+def _compile(src: str, hip: bool, part, verbose: bool) -> Path:
+    out = _object(src, part)
     cmd = [HIPCC] + COMMON + (HIPFLAGS if hip else ["-x", "c++"]) + ["-c", str(CSRC / src), "-o", str(out)]
-    if not hip:
-        cmd = [HIPCC] + COMMON + ["-x", "c++", "-c", str(CSRC / src), "-o", str(out)]
+    if part is not None:
+        cmd.insert(-4, f"-DGSG_PART={part}")
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
@@ -47,8 +57,8 @@ def _compile(src: str, hip: bool, verbose: bool) -> Path:
 def build(verbose: bool = False) -> Path:
     """Compile every source and link libgsg.so next to this file."""
     OBJ.mkdir(exist_ok=True)
-    with ThreadPoolExecutor(max_workers=len(SOURCES)) as ex:
-        objs = list(ex.map(lambda s: _compile(s[0], s[1], verbose), SOURCES))
+    with ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 1)) as ex:
+        objs = list(ex.map(lambda s: _compile(*s, verbose), SOURCES))
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp)] + [str(o) for o in objs] + ["-lpthread"]
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -2167,17 +2167,39 @@ static hipError_t launch_tk(bool fp32, const LaunchArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+hipError_t launch_any(bool fp32, const LaunchArgs& a, hipStream_t s);  // shapes read at run time
+
 template <int DT>
-static hipError_t launch_d(int K, bool fp32, const LaunchArgs& a, hipStream_t s) {
+hipError_t launch_d(int K, bool fp32, const LaunchArgs& a, hipStream_t s) {
   switch (K) {
     case 1: return launch_tk<DT, 1>(fp32, a, s);
     case 2: return launch_tk<DT, 2>(fp32, a, s);
     case 3: return launch_tk<DT, 3>(fp32, a, s);
     case 4: return launch_tk<DT, 4>(fp32, a, s);
     case 5: return launch_tk<DT, 5>(fp32, a, s);
-    default: return launch_tk<0, 0>(fp32, a, s);
+    default: return launch_any(fp32, a, s);
   }
 }
+
+// The file is compiled once per part, side by side: part D > 0 holds the operator kernels
+// of dimension D (part 1: of 1, 5, 6 and the run-time shapes), part 0 everything else.
+#ifndef GSG_PART
+#define GSG_PART 0
+#endif
+#if GSG_PART == 1
+template hipError_t launch_d<1>(int, bool, const LaunchArgs&, hipStream_t);
+template hipError_t launch_d<5>(int, bool, const LaunchArgs&, hipStream_t);
+template hipError_t launch_d<6>(int, bool, const LaunchArgs&, hipStream_t);
+hipError_t launch_any(bool fp32, const LaunchArgs& a, hipStream_t s) { return launch_tk<0, 0>(fp32, a, s); }
+#elif GSG_PART > 1
+template hipError_t launch_d<GSG_PART>(int, bool, const LaunchArgs&, hipStream_t);
+#else
+extern template hipError_t launch_d<1>(int, bool, const LaunchArgs&, hipStream_t);
+extern template hipError_t launch_d<2>(int, bool, const LaunchArgs&, hipStream_t);
+extern template hipError_t launch_d<3>(int, bool, const LaunchArgs&, hipStream_t);
+extern template hipError_t launch_d<4>(int, bool, const LaunchArgs&, hipStream_t);
+extern template hipError_t launch_d<5>(int, bool, const LaunchArgs&, hipStream_t);
+extern template hipError_t launch_d<6>(int, bool, const LaunchArgs&, hipStream_t);
 
 hipError_t launch_op(int D, int K, bool fp32, const LaunchArgs& a, hipStream_t s) {
   switch (D) {
@@ -2187,7 +2209,7 @@ hipError_t launch_op(int D, int K, bool fp32, const LaunchArgs& a, hipStream_t s
     case 4: return launch_d<4>(K, fp32, a, s);
     case 5: return launch_d<5>(K, fp32, a, s);
     case 6: return launch_d<6>(K, fp32, a, s);
-    default: return launch_tk<0, 0>(fp32, a, s);
+    default: return launch_any(fp32, a, s);
   }
 }
 
@@ -2451,5 +2473,7 @@ hipError_t launch_csr(const DevCsr& A, bool fp32, const void* x, void* y, hipStr
     hipLaunchKernelGGL((k_csr<double>), dim3(unsigned(blocks)), dim3(256), 0, s, A, (const double*)x, (double*)y);
   return hipGetLastError();
 }
+
+#endif  // GSG_PART
 
 }  // namespace gsg
