@@ -34,6 +34,8 @@ SOURCES = [
     ("gsg_kernels.hip", True, 2),
     ("gsg_kernels.hip", True, 3),
     ("gsg_kernels.hip", True, 4),
+    ("gsg_solo64.hip", True, None),
+    ("gsg_solo32.hip", True, None),
 ]
 
 

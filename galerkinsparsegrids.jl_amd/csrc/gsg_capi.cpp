@@ -168,7 +168,7 @@ struct Tables {
   std::vector<Tile> ttiles; // tile-plan tiles (blk = tile index), natural order
   std::vector<Tile> dtiles; // direct-kernel tiles: one cell each, blk = packed list lengths,
                             // aux = device address of the cell's plan entries
-  DevMem blk_lev, blk_off, blk_inoff, row_ptr, ent, val64, val32, val32p, plan_ptr, plan_ent;
+  DevMem blk_lev, blk_off, blk_inoff, row_ptr, ent, val64, val32, val32p, plan_ptr, plan_ent, solo_ent;
   DevMem tile_bptr[2], batch_sptr[2], slot_off[2], slot_dir[2], batch_lptr[2], tile_ent[2];
   DevTables devp[2];        // device tables with the precision's tile plan
   static int64_t ipow_i(int64_t b, int e) {
@@ -180,7 +180,7 @@ struct Tables {
   // device memory the tables hold (every array, both precisions' tile plans)
   size_t device_bytes() const {
     size_t b = blk_lev.bytes + blk_off.bytes + blk_inoff.bytes + row_ptr.bytes + ent.bytes + val64.bytes +
-               val32.bytes + val32p.bytes + plan_ptr.bytes + plan_ent.bytes;
+               val32.bytes + val32p.bytes + plan_ptr.bytes + plan_ent.bytes + solo_ent.bytes;
     for (int f = 0; f < 2; ++f)
       b += tile_bptr[f].bytes + batch_sptr[f].bytes + slot_off[f].bytes + slot_dir[f].bytes + batch_lptr[f].bytes +
            tile_ent[f].bytes;
@@ -341,6 +341,25 @@ static std::shared_ptr<Tables> get_tables(int D, int k, int n, int full, int tki
     upload(T->plan_ent, pe);
   }
   const int64_t kD = Tables::ipow_i(k, D);
+  // grids whose stage vectors and lists fit a workgroup's LDS: the lists packed for the
+  // resident kernel
+  if (tkind == TAB_DERIV && solo_shape_ok(D, k) && T->lt.N / kD <= 65535 && v64.size() / (size_t(k) * k) <= 65535 &&
+      T->lt.N * 8 + int64_t(T->plan.ent.size()) * 2 <= SOLO_LDS) {
+    std::vector<uint32_t> se(T->plan.ent.size() / 2);
+    for (size_t q = 0; q < se.size(); ++q)
+      se[q] = uint32_t(T->plan.ent[2 * q + 1]) << 16 | uint32_t(T->plan.ent[2 * q] / kD);
+    const int32_t* ptr = T->plan.ptr.data();
+    std::vector<uint32_t> lists;
+    for (int64_t g = 0; g < T->lt.N / kD; ++g)
+      for (int d = 0; d < D; ++d) lists.push_back(uint32_t(d) << 16 | uint32_t(g));
+    auto len = [&](uint32_t q) {
+      const int64_t at = int64_t(q & 0xffffu) * D + (q >> 16);
+      return ptr[at + 1] - ptr[at];
+    };
+    std::stable_sort(lists.begin(), lists.end(), [&](uint32_t p, uint32_t q) { return len(p) > len(q); });
+    se.insert(se.end(), lists.begin(), lists.end());
+    upload(T->solo_ent, se);
+  }
   // the shapes with a fiber-kernel instantiation; the others run the plan kernel
   T->tile_ok = tkind == TAB_DERIV && fiber_ok(D, k);
   if (T->tile_ok && !direct_ok(D, k)) {  // the direct kernel needs no tile plan
@@ -372,7 +391,7 @@ static std::shared_ptr<Tables> get_tables(int D, int k, int n, int full, int tki
                            T->val32.as<float>(),         T->plan_ptr.as<int32_t>(),    T->plan_ent.as<int32_t>(),
                            T->tile_bptr[f].as<int32_t>(), T->batch_sptr[f].as<int32_t>(), T->slot_off[f].as<int32_t>(),
                            T->slot_dir[f].as<int32_t>(), T->batch_lptr[f].as<int32_t>(), T->tile_ent[f].as<int32_t>(),
-                           int64_t(v64.size()), T->val32p.as<float>(), int64_t(v32p.size() / 2)};
+                           int64_t(v64.size()), T->solo_ent.as<uint32_t>(), T->val32p.as<float>(), int64_t(v32p.size() / 2)};
   T->tiles = make_tiles(T->lt, 0);
   if (T->tile_ok && (direct_ok(D, k) || seg_ok(D, k))) {
     // one tile per cell; the D list lengths (< 256 each) packed a byte per direction
@@ -590,6 +609,18 @@ static void check_desc(const gsg_op_desc* d) {
   for (int e = 0; e < d->D; ++e) require(std::isfinite(d->coef[e]), "coefficients must be finite");
 }
 
+// Multiplications of one operator application up to which a solve runs resident in one
+// workgroup.  Measured, us an RK4 step on the stage launches / resident (FP64, FP32):
+//   D = 2, k = 3, n = 5 (1,008 coefficients, 42e3)  transport 66 / 16.5, 42 / 17.4
+//                                                   wave 131 / 29.5, 127 / 41.8
+//   D = 3, k = 3, n = 3 (1,026, 37e3)               transport 28 / 13.5, 31 / 15.3
+//   D = 2, k = 4, n = 5 (1,792, 99e3)               transport 39 / 24, 42 / 27
+//   D = 2, k = 3, n = 6 (2,304, 104e3)              transport 82 / 29, 56 / 31
+// With the 1-D blocks left in global memory (they do not fit beside the vectors) it wins
+// only against the FP64 fiber kernel (D = 1, k = 5, n = 7: 465 / 25; FP32, plan kernel:
+// 45 / 55).
+constexpr int64_t SOLO_MACS = 120000;
+constexpr int64_t SOLO_MACS_FIBER = 250000;
 // RK4 stage launches of a set of solves of one (D, K) class.
 // How a grid's launches run: the kernel and, for the LDS fiber kernel, its LDS layout.
 struct LdsShape {
@@ -668,6 +699,50 @@ static void set_lds(LaunchArgs& a, const LdsShape& L) {
   a.lds_xelems = L.xelems;
   a.lds_ments = L.ments;
   a.lds_mslots = L.mslots;
+}
+
+// How a solve's RK4 steps run when they run resident in one workgroup (gsg_solo.hpp).
+struct SoloShape {
+  bool on = false;
+  bool segr = false;  // float: the segmented kernel's roundings
+  bool vals = false;  // the 1-D blocks in LDS beside the vectors
+  bool small = false;  // one output a lane
+  int32_t threads = 0, lds = 0;
+};
+static SoloShape solo_shape(const Tables& T, const LdsShape& L, bool fp32, bool wave) {
+  SoloShape q;
+  if (!T.solo_ent.p || std::getenv("GSG_KERNEL")) return q;  // a forced stage kernel runs as asked
+  if (fp32 && L.kernel == KERNEL_DIRECT) return q;           // its lo correction is the matrix cores' bf16 product
+  const int es = fp32 ? 4 : 8;
+  const int N = int(T.lt.N), ne = int(T.plan.ent.size() / 2);
+  const int64_t base = SoloLds(T.D, T.k, N, es, wave, ne).vals;
+  const int64_t vb = int64_t(T.devp[0].val_elems) * 8;  // FP64, or the two float tables
+  if (base > SOLO_LDS) return q;
+  const int64_t macs = int64_t(ne) * Tables::ipow_i(T.k, T.D + 1);
+  if (base + vb <= SOLO_LDS ? macs > SOLO_MACS : L.kernel != KERNEL_FIBER || macs > SOLO_MACS_FIBER) return q;
+  q.on = true;
+  q.segr = L.kernel == KERNEL_SEG || L.kernel == KERNEL_SEG_ALT;
+  if (!fp32) q.segr = false;
+  q.vals = base + vb <= SOLO_LDS;
+  q.lds = int32_t(q.vals ? base + vb : base);
+  q.small = T.D * N <= 1536;
+  q.threads = int32_t(std::min<int64_t>(SOLO_MAXT, (T.D * N + 63) / 64 * 64));
+  return q;
+}
+// nsteps RK4 steps of nsolve solves of one shape (ids: their indices, null: 0, 1, ...),
+// cut into launches of a few milliseconds
+static void launch_solo_steps(int D, int K, bool fp32, const SoloShape& q, const SolveDesc* solves, const int32_t* ids,
+                              int nsolve, int64_t nsteps, hipStream_t s) {
+  constexpr int64_t STEPS = 256;
+  SoloArgs a{};
+  a.solves = solves;
+  a.ids = ids;
+  a.vals_lds = q.vals ? 1 : 0;
+  a.small_map = q.small ? 1 : 0;
+  for (; nsteps > 0; nsteps -= a.nsteps) {
+    a.nsteps = std::min(nsteps, STEPS);
+    HIPC(launch_solo(D, K, fp32, q.segr, a, nsolve, q.threads, q.lds, s));
+  }
 }
 
 static void launch_rk_step(int D, int K, bool fp32, int sys, const SolveDesc* dsolves, const Tile* dtiles,
@@ -888,6 +963,7 @@ struct gsg_op {
   DevMem d_adesc, d_tiles;  // tiles of the launch shape, XCD-split
   int32_t n_tiles = 0;
   LdsShape shape;  // kernel and LDS layout of the apply and RK launches
+  SoloShape solo;  // RK4 steps in one workgroup (small grids)
   DevMem xbuf, ybuf, x32, wbuf;
   // rk path
   std::unique_ptr<SolveState> rk;
@@ -1209,6 +1285,7 @@ int gsg_op_create(const gsg_op_desc* desc, gsg_op** out) {
                                            tiles_per_wave(op->shape, T.D, T.k));
     op->n_tiles = int32_t(pt.size());
     upload(op->d_tiles, pt);
+    op->solo = solo_shape(T, op->shape, op->fp32, desc->kind == GSG_OP_WAVE);
     const size_t es = op->fp32 ? 4 : 8;
     const bool two_pass = desc->kind == GSG_OP_LAPLACIAN || desc->kind == GSG_OP_WAVE;
     if (op->fp32) op->x32.alloc((op->len + (two_pass ? op->N : 0)) * 4);  // two passes: and u's remainder
@@ -1505,6 +1582,10 @@ static void op_rk_prepare(gsg_op* op, double dt) {
 static void op_rk_steps(gsg_op* op, int64_t nsteps, hipStream_t s) {
   const Tables& T = *op->T;
   const int sys = op->d.kind == GSG_OP_WAVE ? SYS_WAVE : SYS_SUM;
+  if (op->solo.on) {
+    launch_solo_steps(T.D, T.k, op->fp32, op->solo, op->d_rkdesc.as<SolveDesc>(), nullptr, 1, nsteps, s);
+    return;
+  }
   op->rkgraphs.run(nsteps, s, false, [&](int64_t k, hipStream_t st) {
     for (int64_t i = 0; i < k; ++i)
       launch_rk_step(T.D, T.k, op->fp32, sys, op->d_rkdesc.as<SolveDesc>(), op->d_tiles.as<Tile>(), op->n_tiles,
@@ -1542,7 +1623,7 @@ int gsg_op_rk4(gsg_op* op, double* y, int64_t len, double t0, double dt, int64_t
     SolveState& S = *op->rk;
     hipStream_t s = op->stream;
     HIPC(hipMemcpyAsync(S.y.p, y, size_t(len) * 8, hipMemcpyHostToDevice, s));
-    S.to_stage0(s);
+    if (!op->solo.on) S.to_stage0(s);
     int64_t done = 0, snap = 0;
     while (done < nsteps) {
       int64_t chunk = nsteps - done;
@@ -1577,7 +1658,7 @@ int gsg_op_rk4_device(gsg_op* op, double* y_dev, int64_t len, double dt, int64_t
       op_rk_prepare(op, dt);
       SolveState& S = *op->rk;
       HIPC(hipMemcpyAsync(S.y.p, y_dev, size_t(len) * 8, hipMemcpyDeviceToDevice, s));
-      S.to_stage0(s);
+      if (!op->solo.on) S.to_stage0(s);
       op_rk_steps(op, nsteps, s);
       HIPC(hipMemcpyAsync(y_dev, S.y.p, size_t(len) * 8, hipMemcpyDeviceToDevice, s));
     });
@@ -1691,9 +1772,10 @@ int gsg_op_rk4_device_noalloc(gsg_op* op, double* y_dev, int64_t len, double dt,
     on_op_stream(op, stream, [&](hipStream_t s) {
       HIPC(launch_write_desc(dd, d, s));
       HIPC(hipMemcpyAsync(d.y, y_dev, size_t(len) * 8, hipMemcpyDeviceToDevice, s));
-      if (op->fp32)
+      if (op->fp32 && !op->solo.on)
         HIPC(launch_to_f32(d.y, static_cast<float*>(d.xs[0]), len, s, op->d.kind == GSG_OP_WAVE ? op->N : 0));
-      for (int64_t i = 0; i < nsteps; ++i)
+      if (op->solo.on) launch_solo_steps(T.D, T.k, op->fp32, op->solo, dd, nullptr, 1, nsteps, s);
+      for (int64_t i = 0; i < nsteps && !op->solo.on; ++i)
         launch_rk_step(T.D, T.k, op->fp32, sys, dd, op->d_tiles.as<Tile>(), op->n_tiles, op->shape, s);
       HIPC(hipMemcpyAsync(y_dev, d.y, size_t(len) * 8, hipMemcpyDeviceToDevice, s));
     });
@@ -1736,6 +1818,9 @@ struct Group {
   DevMem dtiles;
   int64_t dofs = 0;  // component DoFs covered per launch
   LdsShape lds;      // kernel; for the fiber kernel the LDS layout (maxima over the group)
+  SoloShape solo;    // resident solves: all steps of a call in one launch (maxima over the group)
+  std::vector<int32_t> ids;  // resident: the group's solves
+  DevMem dids;
   bool tiled() const { return lds.kernel != KERNEL_PLAN; }
 };
 
@@ -1831,32 +1916,46 @@ struct Scheduler {
     reset_graph();
     descs.clear();
     groups.clear();
-    std::map<std::tuple<int, int, int, int>, size_t> gidx;
+    std::map<std::tuple<int, int, int, int, int>, size_t> gidx;
     std::vector<std::vector<size_t>> members;
+    auto solo_of = [&](const SolveState& S) {
+      return solo_shape(*S.T, lds_shape(*S.T, fp32), fp32, S.desc.sys == SYS_WAVE);
+    };
     // cells per (D, k, system) class of the solves whose grid runs the segmented kernel:
     // a class launch of too few cells runs the plan kernel instead (FP64, SEG64_MIN_CELLS)
     std::map<std::tuple<int, int, int>, int64_t> seg_cells;
     for (SolveState* S : solves)
-      if (lds_shape(*S->T, fp32).kernel == KERNEL_SEG)
+      if (lds_shape(*S->T, fp32).kernel == KERNEL_SEG && !solo_of(*S).on)
         seg_cells[std::make_tuple(S->T->D, S->T->k, S->desc.sys)] += S->N / Tables::ipow_i(S->T->k, S->T->D);
     for (size_t s = 0; s < solves.size(); ++s) {
       SolveState& S = *solves[s];
       descs.push_back(S.desc);
       const auto ck = std::make_tuple(S.T->D, S.T->k, S.desc.sys);
       const LdsShape L = lds_shape(*S.T, fp32, seg_cells.count(ck) ? seg_cells[ck] : int64_t(1) << 40);
-      auto key = std::make_tuple(S.T->D, S.T->k, S.desc.sys, int(L.kernel));
+      const SoloShape q = solo_of(S);
+      auto key = std::make_tuple(S.T->D, S.T->k, S.desc.sys, int(L.kernel), q.on ? 1 + int(q.vals) + 2 * int(q.small) : 0);
       auto it = gidx.find(key);
       if (it == gidx.end()) {
         gidx[key] = groups.size();
-        groups.push_back(Group{S.T->D, S.T->k, S.desc.sys, {}, {}, 0, L});
+        groups.push_back(Group{S.T->D, S.T->k, S.desc.sys, {}, {}, 0, L, q, {}, {}});
         members.emplace_back();
         it = gidx.find(key);
+      }
+      if (q.on) {
+        Group& g = groups[it->second];
+        g.ids.push_back(int32_t(s));
+        g.solo.threads = std::max(g.solo.threads, q.threads);
+        g.solo.lds = std::max(g.solo.lds, q.lds);
       }
       groups[it->second].dofs += S.N;
       members[it->second].push_back(s);
     }
     for (size_t gi = 0; gi < groups.size(); ++gi) {
       Group& g = groups[gi];
+      if (g.solo.on) {
+        upload(g.dids, g.ids);
+        continue;
+      }
       std::vector<Tile> all;
       for (size_t s : members[gi]) {
         const SolveState& S = *solves[s];
@@ -1901,6 +2000,7 @@ struct Scheduler {
     for (size_t gi : order) {
       const Group& g = groups[gi];
       const bool wave = g.sys == SYS_WAVE;
+      if (g.solo.on) continue;
       if (!fused_ok(g.lds.kernel, g.D, g.K) || fused[0].nseg >= FUSED_MAXSEG || (wave && fused[1].nseg >= FUSED_MAXSEG)) {
         unfused.push_back(gi);
         continue;
@@ -1984,6 +2084,21 @@ struct Scheduler {
     pend.push_back(Pending{g.D, g.K, g.sys, g.tiled(), g.dofs, double(g.dofs) * stage_bytes(g.sys, op, stage, fp32, g.D), e0});
   }
 
+  // all k steps of a resident group
+  void launch_solo_group(const Group& g, int64_t k, hipStream_t st) {
+    const size_t e0 = evused;
+    if (profile) HIPC(hipEventRecord(next_event(), st));
+    launch_solo_steps(g.D, g.K, fp32, g.solo, ddescs.as<SolveDesc>(), g.dids.as<int32_t>(), int(g.ids.size()), k, st);
+    if (!profile) return;
+    HIPC(hipEventRecord(next_event(), st));
+    double b = 0;
+    for (int stage = 1; stage <= 4; ++stage) {
+      if (g.sys == SYS_WAVE) b += stage_bytes(g.sys, OP_RK_WAVE_GRAD, stage, fp32, g.D);
+      b += stage_bytes(g.sys, g.sys == SYS_WAVE ? OP_RK_WAVE_SUM : OP_RK_SUM, stage, fp32, g.D);
+    }
+    pend.push_back(Pending{g.D, g.K, g.sys, g.tiled(), g.dofs, double(g.dofs) * b * double(k), e0});
+  }
+
   // GSG_STREAMS=1 runs every launch on the batch stream (for kernel-trace profiles whose
   // per-kernel durations must not include other classes' concurrent kernels)
   static bool lanes_enabled() {
@@ -2012,6 +2127,8 @@ struct Scheduler {
 
   void enqueue(int64_t n) {
     if (schedule == GSG_SCHEDULE_FUSED && !profile) {
+      for (const Group& g : groups)
+        if (g.solo.on) launch_solo_group(g, n, stream);
       for (int64_t st = 0; st < n; ++st)
         for (int stage = 1; stage <= 4; ++stage) {
           if (fused[0].nseg) HIPC(launch_fused(fused_pass_a, stage, fused[0], fused[0].items, stream));
@@ -2029,9 +2146,12 @@ struct Scheduler {
       HIPC(hipEventRecord(fork, stream));
       for (int l = 0; l < nlanes; ++l) HIPC(hipStreamWaitEvent(lanes[l], fork, 0));
     }
+    for (size_t gi = 0; gi < groups.size(); ++gi)
+      if (groups[gi].solo.on) launch_solo_group(groups[gi], n, par ? lanes[lane_of[gi]] : stream);
     for (int64_t st = 0; st < n; ++st)
       for (size_t gi = 0; gi < groups.size(); ++gi) {
         const Group& g = groups[gi];
+        if (g.solo.on) continue;
         hipStream_t s = par ? lanes[lane_of[gi]] : stream;
         for (int stage = 1; stage <= 4; ++stage) {
           if (g.sys == SYS_WAVE) {

@@ -92,6 +92,8 @@ struct DevTables {
   const int32_t* batch_lptr;
   const int32_t* tile_ent;
   int64_t val_elems;         // elements of val64 (and of each half of val32)
+  const uint32_t* solo_ent;  // resident kernel: the plan entries as (block << 16) | input cell, then
+                             // (direction << 16) | cell of every list, longest first (null: not packed)
   const float* val32p;       // the hi and lo blocks padded to 4 x 4 (k <= 4), (nent + 1) * 16 each,
   int64_t val32p_elems;      // the lo half at val32p + val32p_elems
 };
@@ -260,6 +262,46 @@ hipError_t launch_tensor(const ProjArgs& a, const TensorVecs& tv, int64_t N, dou
 // weighted basis values
 hipError_t launch_proj_pass(const ProjArgs& a, const double* wv, int d, int64_t cell0, int64_t ncell, int64_t R,
                             const double* in, double* out, hipStream_t s);
+
+// ---- small solves, resident in one workgroup (gsg_solo.hpp) -------------------------
+// Advance solves (one workgroup each) by nsteps RK4 steps, TRANSPORT-like or WAVE.
+struct SoloArgs {
+  const SolveDesc* solves;
+  const int32_t* ids;  // workgroup -> solve (null: the workgroup's index)
+  int64_t nsteps;
+  int32_t vals_lds;    // the blocks fit beside the vectors in LDS
+  int32_t small_map;   // one output a lane (SoloMap)
+};
+constexpr int SOLO_MAXT = 1024;       // threads of a workgroup, at most
+constexpr int SOLO_LDS = 160 * 1024;  // LDS a workgroup may take
+// a task's outputs: R block rows of G fibers, U entries in flight
+struct SoloMap {
+  int G, R, U;
+};
+constexpr SoloMap solo_map_small(int, int K) { return SoloMap{1, 1, K <= 3 ? 4 : 2}; }
+constexpr SoloMap solo_map_large(int D, int K) {
+  if (D == 1 || K == 1) return solo_map_small(D, K);
+  if (K == 2) return D == 2 ? SoloMap{2, 1, 4} : SoloMap{2, 2, 2};
+  if (K == 3) return D == 2 ? SoloMap{3, 1, 2} : SoloMap{3, 3, 1};
+  return K == 4 ? SoloMap{2, 1, 2} : SoloMap{5, 1, 1};
+}
+// byte offsets of the LDS areas; vals: the blocks, last (absent when they stay in global memory)
+struct SoloLds {
+  int x, ent, ptr, task, vals;
+  constexpr SoloLds(int D, int K, int N, int es, bool wave, int nent)
+      : x(8 * D * N),
+        ent(x + (wave ? D + 2 + (es == 4 ? 1 : 0) : 1) * N * es),
+        ptr(ent + 4 * nent),
+        task(ptr + 4 * (N / kpow(K, D) * D + 1)),
+        vals((task + 4 * (N / kpow(K, D) * D) + 15) / 16 * 16) {}
+};
+constexpr bool solo_shape_ok(int D, int K) { return D >= 1 && D <= 6 && K >= 1 && K <= 5 && kpow(K, D) <= 1024; }
+// segr: float with the segmented kernel's roundings (seg_ok shapes with several cells a
+// wavefront), else the plan kernel's; lds_bytes: with or without the blocks (vals_lds)
+hipError_t launch_solo(int D, int K, bool fp32, bool segr, const SoloArgs& a, int nsolve, int threads, int lds_bytes,
+                       hipStream_t s);
+hipError_t launch_solo32(int D, int K, bool segr, const SoloArgs& a, int nsolve, int threads, int lds_bytes,
+                         hipStream_t s);
 
 // CSR SpMV y = A x (rows ascending columns), value/vector type per precision.
 struct DevCsr {
