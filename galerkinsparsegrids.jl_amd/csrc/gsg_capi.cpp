@@ -229,6 +229,39 @@ static std::vector<Tile> xcd_split(const std::vector<Tile>& tiles, size_t chunk 
   for (size_t t = 0; t < tiles.size(); ++t) bins[per ? t / per : 0].push_back(tiles[t]);
   return xcd_interleave(bins, chunk);
 }
+// The same for single-cell tiles, with the longest wavefronts of an eighth first: a wavefront
+// (`unit` tiles) takes one round per `per_round` entries of each direction's longest list, up
+// to three times the mean, and one that starts last is waited for.  Four classes of rounds,
+// each in its old order (a full sort loses the L2 reuse of neighbours).  Measured on one
+// solve, us a stage in the old / new order: FP64 D = 4, k = 3, n = 8: 34.3 / 27.9; FP32
+// D = 3, k = 4, n = 9, wave: 29.6 / 23.8; FP32 D = 4, k = 4, n = 8: 33.4 / 30.3.  Launches of
+// more than 64 K wavefronts keep the old order (256-solve batch in FP64: 2% slower in the new).
+constexpr size_t LONG_FIRST_WAVES = 65536;
+static std::vector<Tile> xcd_split_work(const std::vector<Tile>& tiles, int D, size_t chunk, size_t unit, int per_round) {
+  const size_t nu = tiles.size() / unit, per = (nu + NXCD - 1) / NXCD;
+  std::vector<uint8_t> cls(nu);
+  for (size_t u = 0; u < nu; ++u) {
+    int r = 0;
+    for (int d = 0; d < D; ++d) {
+      int m = 0;
+      for (size_t q = 0; q < unit; ++q) m = std::max(m, int((uint32_t(tiles[u * unit + q].blk) >> (8 * d)) & 255u));
+      r += (m + per_round - 1) / per_round;
+    }
+    cls[u] = uint8_t(r >= 20 ? 0 : r >= 15 ? 1 : r >= 11 ? 2 : 3);
+  }
+  // as xcd_interleave: tile j of eighth x goes to workgroup (j / chunk) NXCD + x
+  const Tile& t0 = tiles[0];
+  std::vector<Tile> out((per * unit + chunk - 1) / chunk * NXCD * chunk, Tile{t0.solve, t0.blk, t0.start, t0.start, t0.aux});
+  for (size_t x = 0; x < NXCD; ++x) {
+    const size_t u0 = std::min(nu, x * per), u1 = std::min(nu, u0 + per);
+    size_t j = 0;
+    for (int c = 0; c < 4; ++c)
+      for (size_t u = u0; u < u1; ++u)
+        if (cls[u] == c)
+          for (size_t q = 0; q < unit; ++q, ++j) out[((j / chunk) * NXCD + x) * chunk + j % chunk] = tiles[u * unit + q];
+  }
+  return out;
+}
 // Visit order of single-cell tiles: by the Morton code of the cell centre.  A cell's
 // coupled input cells overlap it in space (at every level), so a spatially coherent
 // order keeps the inputs in flight on an XCD within a small region and lets its L2
@@ -626,6 +659,7 @@ constexpr int64_t SOLO_MACS_FIBER = 250000;
 struct LdsShape {
   int32_t kernel = KERNEL_PLAN;
   int32_t bytes = 0, xelems = 0, ments = 0, mslots = 0;
+  bool dsplit = false;  // direct and segmented kernels: one wavefront per direction
 };
 // LDS layout of the fiber kernel for batches of at most `slots` input cells and `ents`
 // entries: the input region also holds the per-direction results and keeps the
@@ -673,10 +707,32 @@ static LdsShape lds_shape(const Tables& T, bool fp32) {
 // n = 8: 1.7x the plan kernel on 190K cells of copies, 0.8x on one solve's 10.5K.  A launch
 // of fewer cells runs the plan kernel.
 constexpr int64_t SEG64_MIN_CELLS = 65536;
-static LdsShape lds_shape(const Tables& T, bool fp32, int64_t launch_cells) {
-  const LdsShape L = lds_shape(T, fp32);
+// One wavefront per direction (LaunchArgs::dsplit) cuts a cell's serial rounds to its
+// longest direction's and gives a launch D times the wavefronts; the price is a barrier and
+// D readers of a cell's tile.  It pays while a launch has fewer wavefronts (without it) than
+// the chip holds at once, 8192; a launch of more is bound by throughput.  Measured, us a
+// stage without / with: FP32 D = 3, k = 3: 2432 wavefronts 20.1 / 12.4, 9728 29.8 / 30.6;
+// D = 4, k = 3: 5248 25.1 / 21.6, 10496 34.0 / 35.9; D = 4, k = 4: 3040 12.4 / 11.4,
+// 6080 17.1 / 19.3; FP64 D = 4, k = 4: 20992 72.7 / 70.2, 41984 150 / 158; D = 3, k = 4:
+// 688 14.4 / 9.6, 9728 26.5 / 26.5.
+static int64_t dsplit_waves(int32_t kernel, int D, int K, bool fp32) {
+  if (fp32 && (kernel == KERNEL_SEG || kernel == KERNEL_SEG_ALT)) return 8192;
+  if (kernel != KERNEL_DIRECT) return -1;
+  return fp32 ? 4096 : direct_ok(D, K) ? 24576 : 8192;
+}
+// launch_waves: the wavefronts of every launch that runs beside this one
+static LdsShape lds_shape(const Tables& T, bool fp32, int64_t launch_cells, int64_t launch_waves) {
+  LdsShape L = lds_shape(T, fp32);
   if (!fp32 && L.kernel == KERNEL_SEG && launch_cells < SEG64_MIN_CELLS) return LdsShape{};
+  if (T.D > 1) L.dsplit = launch_waves <= dsplit_waves(L.kernel, T.D, T.k, fp32);
   return L;
+}
+static int64_t grid_cells(const Tables& T) { return T.lt.N / Tables::ipow_i(T.k, T.D); }
+// wavefronts of one solve of the grid on the single-cell kernels, one cell group each
+static int64_t grid_waves(const Tables& T, bool fp32) {
+  const int32_t k = lds_shape(T, fp32).kernel;
+  const int64_t per = k == KERNEL_SEG || k == KERNEL_SEG_ALT ? seg_cpw(T.D, T.k) : 1;
+  return (grid_cells(T) + per - 1) / per;
 }
 // tiles of a launch shape: tile-plan tiles for the fiber kernel, TILE-DoF tiles otherwise
 static const std::vector<Tile>& tiles_of(const Tables& T, const LdsShape& L) {
@@ -685,13 +741,19 @@ static const std::vector<Tile>& tiles_of(const Tables& T, const LdsShape& L) {
 }
 // tiles per workgroup of a launch shape
 static size_t tiles_per_wg(const LdsShape& L, int D, int K) {
-  if (L.kernel == KERNEL_DIRECT) return DIRECT_CPW;
-  if (L.kernel == KERNEL_SEG || L.kernel == KERNEL_SEG_ALT) return size_t(SEG_WAVES * seg_cpw(D, K));
+  if (L.kernel == KERNEL_DIRECT) return L.dsplit ? 1 : DIRECT_CPW;
+  if (L.kernel == KERNEL_SEG || L.kernel == KERNEL_SEG_ALT) return size_t((L.dsplit ? 1 : SEG_WAVES) * seg_cpw(D, K));
   return 1;
 }
 // tiles a wavefront takes together (they must belong to one solve)
 static size_t tiles_per_wave(const LdsShape& L, int D, int K) {
   return (L.kernel == KERNEL_SEG || L.kernel == KERNEL_SEG_ALT) ? size_t(seg_cpw(D, K)) : 1;
+}
+// the launch order of a list of tiles of this shape
+static std::vector<Tile> launch_order(const std::vector<Tile>& tiles, const LdsShape& L, int D, int K) {
+  const size_t wg = tiles_per_wg(L, D, K), wave = tiles_per_wave(L, D, K);
+  const bool single = L.kernel == KERNEL_DIRECT || L.kernel == KERNEL_SEG || L.kernel == KERNEL_SEG_ALT;
+  return single && !tiles.empty() && tiles.size() / wave <= LONG_FIRST_WAVES ? xcd_split_work(tiles, D, wg, wave, 4) : xcd_split(tiles, wg, wave);
 }
 static void set_lds(LaunchArgs& a, const LdsShape& L) {
   a.kernel = L.kernel;
@@ -699,6 +761,7 @@ static void set_lds(LaunchArgs& a, const LdsShape& L) {
   a.lds_xelems = L.xelems;
   a.lds_ments = L.ments;
   a.lds_mslots = L.mslots;
+  a.dsplit = L.dsplit ? 1 : 0;
 }
 
 // How a solve's RK4 steps run when they run resident in one workgroup (gsg_solo.hpp).
@@ -708,6 +771,7 @@ struct SoloShape {
   bool vals = false;  // the 1-D blocks in LDS beside the vectors
   bool small = false;  // one output a lane
   int32_t threads = 0, lds = 0;
+  double us = 0;  // about a step's time
 };
 static SoloShape solo_shape(const Tables& T, const LdsShape& L, bool fp32, bool wave) {
   SoloShape q;
@@ -726,6 +790,7 @@ static SoloShape solo_shape(const Tables& T, const LdsShape& L, bool fp32, bool 
   q.vals = base + vb <= SOLO_LDS;
   q.lds = int32_t(q.vals ? base + vb : base);
   q.small = T.D * N <= 1536;
+  q.us = (wave ? 2.0 : 1.0) * (8.0 + double(macs) * 2e-4);
   q.threads = int32_t(std::min<int64_t>(SOLO_MAXT, (T.D * N + 63) / 64 * 64));
   return q;
 }
@@ -1036,7 +1101,8 @@ static void vlasov_rk_steps(gsg_op* op, double dt, int64_t n, hipStream_t s) {
     for (int64_t i = 0; i < k; ++i)
       for (int stage = 1; stage <= 4; ++stage) {
         // the last n2m sweep applies the stage update (no right-hand-side vector)
-        const XRk rk{stage, dt, op->vy.as<double>(), op->vacc.as<double>(), op->vx.as<double>(), x32};
+        const double wa = stage == 1 || stage == 4 ? dt / 6.0 : dt / 3.0, wx = stage <= 2 ? dt / 2.0 : dt;
+        const XRk rk{stage, wa, wx, op->vy.as<double>(), op->vacc.as<double>(), op->vx.as<double>(), x32};
         vlasov_apply(op, stage == 1 ? op->vy.as<double>() : op->vx.as<double>(), op->vr.as<double>(), st,
                      i > 0 || stage > 1, &rk);
       }
@@ -1280,9 +1346,8 @@ int gsg_op_create(const gsg_op_desc* desc, gsg_op** out) {
       HIPC(hipMemcpy(op->d_adesc.p, &a, sizeof(SolveDesc), hipMemcpyHostToDevice));
     }
     // the fiber and direct kernels apply every direction: a single derivative runs the plan kernel
-    if (desc->kind != GSG_OP_DERIV) op->shape = lds_shape(T, op->fp32, T.lt.N / Tables::ipow_i(T.k, T.D));
-    const std::vector<Tile> pt = xcd_split(tiles_of(T, op->shape), tiles_per_wg(op->shape, T.D, T.k),
-                                           tiles_per_wave(op->shape, T.D, T.k));
+    if (desc->kind != GSG_OP_DERIV) op->shape = lds_shape(T, op->fp32, grid_cells(T), grid_waves(T, op->fp32));
+    const std::vector<Tile> pt = launch_order(tiles_of(T, op->shape), op->shape, T.D, T.k);
     op->n_tiles = int32_t(pt.size());
     upload(op->d_tiles, pt);
     op->solo = solo_shape(T, op->shape, op->fp32, desc->kind == GSG_OP_WAVE);
@@ -1472,9 +1537,8 @@ int gsg_vlasov_create(const gsg_vlasov_desc* desc, const double* F_point, int64_
     a.ndir = D;
     for (int e = 0; e < D; ++e) a.coef[e] = 1.0;
     upload(op->d_adesc, std::vector<SolveDesc>{a});
-    op->shape = lds_shape(T, op->fp32, T.lt.N / Tables::ipow_i(k, D));
-    const std::vector<Tile> pt = xcd_split(tiles_of(T, op->shape), tiles_per_wg(op->shape, D, k),
-                                           tiles_per_wave(op->shape, D, k));
+    op->shape = lds_shape(T, op->fp32, grid_cells(T), grid_waves(T, op->fp32));
+    const std::vector<Tile> pt = launch_order(tiles_of(T, op->shape), op->shape, D, k);
     op->n_tiles = int32_t(pt.size());
     upload(op->d_tiles, pt);
     op->m2n.init(D, k, n, scheme, TAB_M2N);
@@ -1572,7 +1636,7 @@ static void op_rk_prepare(gsg_op* op, double dt) {
   // the descriptor (with dt) changes only with dt; its write is ordered on op->stream
   // after the steps of earlier calls, which read it
   if (!op->rk_desc_set || dt != op->rk_dt) {
-    op->rk->desc.dt = dt;
+    op->rk->desc.set_dt(dt);
     HIPC(launch_write_desc(op->d_rkdesc.as<SolveDesc>(), op->rk->desc, op->stream));
     op->rk_dt = dt;
     op->rk_desc_set = true;
@@ -1755,7 +1819,7 @@ int gsg_op_rk4_device_noalloc(gsg_op* op, double* y_dev, int64_t len, double dt,
     std::memcpy(d.coef, op->adesc.coef, sizeof(d.coef));  // the RK right-hand side is the operator
     d.ndir = op->adesc.ndir;
     d.dir0 = op->adesc.dir0;
-    d.dt = dt;
+    d.set_dt(dt);
     const size_t xl = size_t(SolveState::xs_len(op->d.kind, op->N, op->fp32));
     d.y = reinterpret_cast<double*>(take(size_t(len) * 8));
     d.acc = reinterpret_cast<double*>(take(size_t(len) * 8));
@@ -1892,12 +1956,20 @@ struct Scheduler {
     }
   }
 
-  // lanes by estimated cost (DoFs x D x k), largest class first onto the least loaded lane
+  // about the microseconds a step of `dofs` DoFs takes of a busy chip
+  static double stage_us(double dofs, int D, int K, int sys) { return dofs * D * K * (sys == SYS_WAVE ? 5e-6 : 2.5e-6); }
+  static constexpr double SOLO_BATCH_US = 100.0;
+
+  // lanes by estimated cost, largest class first onto the least loaded lane
   void assign_lanes() {
     lane_of.assign(groups.size(), 0);
     std::vector<size_t> order(groups.size());
     for (size_t i = 0; i < order.size(); ++i) order[i] = i;
-    auto cost = [&](size_t i) { return double(groups[i].dofs) * groups[i].D * groups[i].K; };
+    auto cost = [&](size_t i) {  // about microseconds a step
+      const Group& g = groups[i];
+      if (g.solo.on) return g.solo.us * std::max(1.0, double(g.ids.size()) / 256.0);
+      return 30.0 + stage_us(double(g.dofs), g.D, g.K, g.sys);
+    };
     std::sort(order.begin(), order.end(), [&](size_t x, size_t y) { return cost(x) > cost(y); });
     nlanes = tuned_lanes();
     double load[NLANE] = {};
@@ -1921,18 +1993,29 @@ struct Scheduler {
     auto solo_of = [&](const SolveState& S) {
       return solo_shape(*S.T, lds_shape(*S.T, fp32), fp32, S.desc.sys == SYS_WAVE);
     };
-    // cells per (D, k, system) class of the solves whose grid runs the segmented kernel:
-    // a class launch of too few cells runs the plan kernel instead (FP64, SEG64_MIN_CELLS)
-    std::map<std::tuple<int, int, int>, int64_t> seg_cells;
+    // Resident solves only beside little else: every other class's launches of a large batch
+    // cover its small solves as well, and a resident solve holds a compute unit (256 uneven
+    // solves: 1.98 ms a step with the small ones resident, 1.91 without).
+    double busy = 0;
     for (SolveState* S : solves)
-      if (lds_shape(*S->T, fp32).kernel == KERNEL_SEG && !solo_of(*S).on)
+      if (!solo_of(*S).on) busy += stage_us(double(S->N), S->T->D, S->T->k, S->desc.sys);
+    const bool solo_ok = busy <= SOLO_BATCH_US;
+    // cells per (D, k, system) class and wavefronts of all classes: a launch of too few cells
+    // runs the plan kernel (FP64, SEG64_MIN_CELLS), one of few wavefronts splits directions
+    std::map<std::tuple<int, int, int>, int64_t> seg_cells;
+    int64_t waves = 0;
+    for (SolveState* S : solves)
+      if (!(solo_ok && solo_of(*S).on)) {
         seg_cells[std::make_tuple(S->T->D, S->T->k, S->desc.sys)] += S->N / Tables::ipow_i(S->T->k, S->T->D);
+        waves += grid_waves(*S->T, fp32);
+      }
+    if (fp32 && resolve_schedule(schedule_own) == GSG_SCHEDULE_FUSED) waves = int64_t(1) << 40;  // whole wavefronts per cell
     for (size_t s = 0; s < solves.size(); ++s) {
       SolveState& S = *solves[s];
       descs.push_back(S.desc);
       const auto ck = std::make_tuple(S.T->D, S.T->k, S.desc.sys);
-      const LdsShape L = lds_shape(*S.T, fp32, seg_cells.count(ck) ? seg_cells[ck] : int64_t(1) << 40);
-      const SoloShape q = solo_of(S);
+      const SoloShape q = solo_ok ? solo_of(S) : SoloShape{};
+      const LdsShape L = q.on ? lds_shape(*S.T, fp32) : lds_shape(*S.T, fp32, seg_cells[ck], waves);
       auto key = std::make_tuple(S.T->D, S.T->k, S.desc.sys, int(L.kernel), q.on ? 1 + int(q.vals) + 2 * int(q.small) : 0);
       auto it = gidx.find(key);
       if (it == gidx.end()) {
@@ -1946,6 +2029,7 @@ struct Scheduler {
         g.ids.push_back(int32_t(s));
         g.solo.threads = std::max(g.solo.threads, q.threads);
         g.solo.lds = std::max(g.solo.lds, q.lds);
+        g.solo.us = std::max(g.solo.us, q.us);
       }
       groups[it->second].dofs += S.N;
       members[it->second].push_back(s);
@@ -1961,7 +2045,7 @@ struct Scheduler {
         const SolveState& S = *solves[s];
         for (const Tile& t : tiles_of(*S.T, g.lds)) all.push_back(Tile{int32_t(s), t.blk, t.start, t.end, t.aux});
       }
-      g.tiles = xcd_split(all, tiles_per_wg(g.lds, g.D, g.K), tiles_per_wave(g.lds, g.D, g.K));
+      g.tiles = launch_order(all, g.lds, g.D, g.K);
       if (g.lds.kernel == KERNEL_FIBER) {
         int32_t slots = 0, ents = 0;
         for (size_t s : members[gi]) {
@@ -2001,7 +2085,7 @@ struct Scheduler {
       const Group& g = groups[gi];
       const bool wave = g.sys == SYS_WAVE;
       if (g.solo.on) continue;
-      if (!fused_ok(g.lds.kernel, g.D, g.K) || fused[0].nseg >= FUSED_MAXSEG || (wave && fused[1].nseg >= FUSED_MAXSEG)) {
+      if (g.lds.dsplit || !fused_ok(g.lds.kernel, g.D, g.K) || fused[0].nseg >= FUSED_MAXSEG || (wave && fused[1].nseg >= FUSED_MAXSEG)) {
         unfused.push_back(gi);
         continue;
       }
@@ -2219,7 +2303,7 @@ static void batch_build(gsg_batch* b) {
   for (auto& s : b->solves) {
     auto T = get_tables(s->d.D, s->d.k, s->d.n, s->d.scheme);
     s->st.init(T, s->d, b->fp32);
-    s->st.desc.dt = s->dt;
+    s->st.desc.set_dt(s->dt);
     require(int64_t(s->y0.size()) == s->st.len, "initial state length does not match the grid");
     HIPC(hipMemcpyAsync(s->st.y.p, s->y0.data(), s->y0.size() * 8, hipMemcpyHostToDevice, b->stream));
     s->st.to_stage0(b->stream);
@@ -2536,7 +2620,7 @@ static void server_loop(gsg_server* S) {
         auto T = r->tab;
         r->st = std::make_unique<SolveState>();
         r->st->init(T, r->d, S->cfg.precision == GSG_PREC_FP32);
-        r->st->desc.dt = r->dt;
+        r->st->desc.set_dt(r->dt);
         HIPC(hipMemcpyAsync(r->st->y.p, r->y0.data(), r->y0.size() * 8, hipMemcpyHostToDevice, S->stream));
         r->st->to_stage0(S->stream);
         std::lock_guard<std::mutex> g(S->mu);

@@ -10,6 +10,22 @@
 
 namespace gsg {
 
+// loads and stores through the global address space (the pointers are device
+// allocations): global_* instructions instead of flat_* ones, which the compiler picks for
+// a pointer read from memory; a flat access also occupies the LDS counter, so every LDS
+// wait waits for it
+template <typename X>
+__device__ __forceinline__ X gld(const X* p) {
+  return *(const __attribute__((address_space(1))) X*)p;
+}
+__device__ __forceinline__ int2 gld2(const int32_t* p) {  // an aligned pair of words
+  return __builtin_bit_cast(int2, gld(reinterpret_cast<const uint64_t*>(p)));
+}
+template <typename X>
+__device__ __forceinline__ void gst(X* p, X v) {
+  *(__attribute__((address_space(1))) X*)p = v;
+}
+
 constexpr int MAXD = 8;
 constexpr int TILE = 256;  // DoFs per tile == threads per workgroup
 
@@ -107,7 +123,15 @@ struct SolveDesc {
   int32_t dir0;     // first direction in SUM mode
   int32_t pad;
   double coef[MAXD];
-  double dt;
+  // the step and its fractions of the RK stages, divided on the host: a division in every
+  // lane's epilogue cost more than the epilogue's memory accesses
+  double dt, dt2, dt3, dt6;
+  void set_dt(double h) {
+    dt = h;
+    dt2 = h / 2.0;
+    dt3 = h / 3.0;
+    dt6 = h / 6.0;
+  }
   // RK4 state (double) and stage buffers (element type = precision of the launch)
   double* y;
   double* acc;
@@ -153,6 +177,8 @@ struct LaunchArgs {
                        // results); the coefficient blocks follow
   int32_t lds_ments;   // entries per batch the coefficient and entry staging hold
   int32_t lds_mslots;  // slots per batch the offset staging holds
+  int32_t dsplit;      // direct and segmented kernels: one wavefront per direction, one group of
+                       // cells (a wavefront's) a workgroup
 };
 
 // Launch one operation over the given tiles for solves of shape (D, K); fp32 selects
@@ -209,7 +235,7 @@ struct XComb {
 // input x (and its float copy x32 when not null); stage 0: none.
 struct XRk {
   int32_t stage;
-  double dt;
+  double wa, wx;  // the stage's weights: of the accumulator and of the next stage input
   double* y;
   double* acc;
   double* x;

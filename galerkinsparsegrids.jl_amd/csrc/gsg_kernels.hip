@@ -100,7 +100,7 @@ __device__ __forceinline__ void plan_entries(const SolveDesc& S, __amdgpu_buffer
       off[u] = uni(sld(S.t.plan_ent + 2 * (p + u)));
       eb[u] = uni(sld(S.t.plan_ent + 2 * (p + u) + 1));
     } else {
-      const int2 pe = *reinterpret_cast<const int2*>(S.t.plan_ent + 2 * (p + u));
+      const int2 pe = gld2(S.t.plan_ent + 2 * (p + u));
       off[u] = pe.x;
       eb[u] = pe.y;
     }
@@ -113,8 +113,8 @@ __device__ __forceinline__ void plan_entries(const SolveDesc& S, __amdgpu_buffer
 #pragma unroll
     for (int mm = 0; mm < KM; ++mm) {
       if (mm >= K) break;
-      b[u][mm] = vp[mm];
-      if constexpr (HL) bl[u][mm] = vp[S.t.val_elems + mm];
+      b[u][mm] = gld(vp + mm);
+      if constexpr (HL) bl[u][mm] = gld(vp + S.t.val_elems + mm);
     }
   }
 #pragma unroll
@@ -149,8 +149,8 @@ __device__ __forceinline__ double plan_dir(const SolveDesc& S, __amdgpu_buffer_r
     p0 = uni(sld(ptr));
     p1 = uni(sld(ptr + 1));
   } else {
-    p0 = ptr[0];
-    p1 = ptr[1];
+    p0 = gld(ptr);
+    p1 = gld(ptr + 1);
   }
   T acc = T(0), acl = T(0);
   int32_t p = p0;
@@ -182,8 +182,8 @@ struct RkIn {
 };
 __device__ __forceinline__ RkIn rk_pre(const SolveDesc& S, int stage, int64_t idx) {
   RkIn v;
-  v.y = stage <= 3 ? S.y[idx] : 0.0;
-  v.acc = stage >= 2 ? S.acc[idx] : 0.0;
+  v.y = stage <= 3 ? gld(S.y + idx) : 0.0;
+  v.acc = stage >= 2 ? gld(S.acc + idx) : 0.0;
   return v;
 }
 // the next stage input x at out[idx] (and, with lo >= 0 in float, its rounding remainder
@@ -191,26 +191,25 @@ __device__ __forceinline__ RkIn rk_pre(const SolveDesc& S, int stage, int64_t id
 template <typename T>
 __device__ __forceinline__ void put_stage(T* out, int64_t idx, int64_t lo, double x) {
   const T h = T(x);
-  out[idx] = h;
-  if (sizeof(T) == 4 && lo >= 0) out[lo] = T(x - double(h));
+  gst(out + idx, h);
+  if (sizeof(T) == 4 && lo >= 0) gst(out + lo, T(x - double(h)));
 }
 template <typename T>
 __device__ __forceinline__ void rk_post(const SolveDesc& S, int stage, int64_t idx, const RkIn& v, double r,
                                         int64_t lo = -1) {
-  const double dt = S.dt;
   T* out = stage_out<T>(S, stage);
   if (stage == 1) {
-    S.acc[idx] = v.y + (dt / 6.0) * r;
-    put_stage(out, idx, lo, v.y + (dt / 2.0) * r);
+    gst(S.acc + idx, v.y + S.dt6 * r);
+    put_stage(out, idx, lo, v.y + S.dt2 * r);
   } else if (stage == 2) {
-    S.acc[idx] = v.acc + (dt / 3.0) * r;
-    put_stage(out, idx, lo, v.y + (dt / 2.0) * r);
+    gst(S.acc + idx, v.acc + S.dt3 * r);
+    put_stage(out, idx, lo, v.y + S.dt2 * r);
   } else if (stage == 3) {
-    S.acc[idx] = v.acc + (dt / 3.0) * r;
-    put_stage(out, idx, lo, v.y + dt * r);
+    gst(S.acc + idx, v.acc + S.dt3 * r);
+    put_stage(out, idx, lo, v.y + S.dt * r);
   } else {
-    const double yn = v.acc + (dt / 6.0) * r;
-    S.y[idx] = yn;
+    const double yn = v.acc + S.dt6 * r;
+    gst(S.y + idx, yn);
     if (out) put_stage(out, idx, lo, yn);
   }
 }
@@ -271,7 +270,7 @@ __device__ __forceinline__ void plan_body(const LaunchArgs& a, int wg) {
       kd *= K;
     }
     if (a.op == OP_APPLY_SUM)
-      ((double*)a.yout)[i] = s;
+      gst((double*)a.yout + i, s);
     else
       rk_update<T>(S, a.stage, i, s);
     return;
@@ -291,7 +290,7 @@ __device__ __forceinline__ void plan_body(const LaunchArgs& a, int wg) {
       const uint32_t mb = uint32_t(ml - md * kd);
       double r = plan_dir<KT, T, UNI>(S, xr, 0u, g, d, D, K, md, mb, kd);
       if (lo) r += plan_dir<KT, T, UNI>(S, xr, uint32_t(lo * int64_t(sizeof(T))), g, d, D, K, md, mb, kd);
-      w[int64_t(d) * N + i] = T(r);
+      gst(w + int64_t(d) * N + i, T(r));
       kd *= K;
     }
     return;
@@ -311,11 +310,11 @@ __device__ __forceinline__ void plan_body(const LaunchArgs& a, int wg) {
   }
   if (a.op == OP_APPLY_WAVE_SUM) {
     const T* x = (const T*)a.xin;
-    ((double*)a.yout)[i] = double(x[N + i]);
-    ((double*)a.yout)[N + i] = s;
+    gst((double*)a.yout + i, double(gld(x + N + i)));
+    gst((double*)a.yout + N + i, s);
   } else {
     const T* xin = stage_in<T>(S, a.stage);
-    rk_update<T>(S, a.stage, i, double(xin[N + i]), 2 * N + i);  // float: u's lo part too
+    rk_update<T>(S, a.stage, i, double(gld(xin + N + i)), 2 * N + i);  // float: u's lo part too
     rk_update<T>(S, a.stage, N + i, s);
   }
 }
@@ -452,9 +451,9 @@ __global__ __launch_bounds__(TILE) void k_fiber(LaunchArgs a) {
     const int32_t E0 = uni(sld(lb));
     const int32_t ne = uni(sld(lb + CPT * D)) - E0;
     for (int32_t q = tid; q < ns; q += TILE)
-      soff[q] = uint32_t(S.t.slot_off[s0 + q]) + uint32_t(S.t.slot_dir[s0 + q] * dstride);
-    for (int32_t q = tid; q < ne; q += TILE) entl[q] = S.t.tile_ent[E0 + q];
-    for (int32_t q = tid; q <= CPT * D; q += TILE) lptl[q] = lb[q] - E0;
+      soff[q] = uint32_t(gld(S.t.slot_off + s0 + q)) + uint32_t(gld(S.t.slot_dir + s0 + q) * dstride);
+    for (int32_t q = tid; q < ne; q += TILE) entl[q] = gld(S.t.tile_ent + E0 + q);
+    for (int32_t q = tid; q <= CPT * D; q += TILE) lptl[q] = gld(lb + q) - E0;
     __syncthreads();
     // input cells: chunk w of the batch -> chunk w % XCH of slot w / XCH, from the
     // 16-byte boundary at or below the slot's cell
@@ -532,24 +531,24 @@ __global__ __launch_bounds__(TILE) void k_fiber(LaunchArgs a) {
 #pragma unroll
       for (int e = 0; e < D; ++e) s += T(S.coef[e]) * yq[e * KD];
       if (a.op == OP_APPLY_SUM)
-        ((double*)a.yout)[i] = double(s);
+        gst((double*)a.yout + i, double(s));
       else
         rk_update<T>(S, a.stage, i, double(s));
     } else if (a.op == OP_APPLY_GRAD || a.op == OP_RK_WAVE_GRAD) {
       T* w = a.op == OP_RK_WAVE_GRAD ? (T*)S.w : (T*)a.yout;
 #pragma unroll
-      for (int e = 0; e < D; ++e) w[int64_t(e) * N + i] = yq[e * KD];
+      for (int e = 0; e < D; ++e) gst(w + int64_t(e) * N + i, yq[e * KD]);
     } else {
       T s = T(0);
 #pragma unroll
       for (int e = 0; e < D; ++e) s += yq[e * KD];
       if (a.op == OP_APPLY_WAVE_SUM) {
         const T* x = (const T*)a.xin;
-        ((double*)a.yout)[i] = double(x[N + i]);
-        ((double*)a.yout)[N + i] = double(s);
+        gst((double*)a.yout + i, double(gld(x + N + i)));
+        gst((double*)a.yout + N + i, double(s));
       } else {
         const T* xin = stage_in<T>(S, a.stage);
-        rk_update<T>(S, a.stage, i, double(xin[N + i]));
+        rk_update<T>(S, a.stage, i, double(gld(xin + N + i)));
         rk_update<T>(S, a.stage, N + i, double(s));
       }
     }
@@ -625,17 +624,6 @@ __device__ __forceinline__ double lane_bcast(double v, int q) {
   return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_readlane(w.x, q), __builtin_amdgcn_readlane(w.y, q)));
 }
 
-// loads and stores through the global address space (the pointers are device
-// allocations): global_* instructions instead of flat_* ones
-template <typename X>
-__device__ __forceinline__ X gld(const X* p) {
-  return *(const __attribute__((address_space(1))) X*)p;
-}
-template <typename X>
-__device__ __forceinline__ void gst(X* p, X v) {
-  *(__attribute__((address_space(1))) X*)p = v;
-}
-
 template <typename P>
 __device__ __forceinline__ P sldp(P const* p) {  // scalar load of a pointer field
   return reinterpret_cast<P>(sld(reinterpret_cast<const int64_t*>(p)));
@@ -647,7 +635,7 @@ template <typename T, int D>
 struct SolveView {
   int64_t N, val_elems;
   int32_t active;
-  double dt;
+  double dt, dt2, dt3, dt6;
   double coef[D];
   double *y, *acc;
   const T* vals;
@@ -657,6 +645,9 @@ struct SolveView {
     val_elems = sld(&S.t.val_elems);
     active = sld(&S.active);
     dt = sld(&S.dt);
+    dt2 = sld(&S.dt2);
+    dt3 = sld(&S.dt3);
+    dt6 = sld(&S.dt6);
 #pragma unroll
     for (int e = 0; e < D; ++e) coef[e] = sld(&S.coef[e]);
     y = sldp(&S.y);
@@ -688,19 +679,19 @@ struct SolveView {
     const d2 ai = stage >= 2 ? *(const gd2*)(acc + idx) : d2{0.0, 0.0};
     T* o = out(stage);
     if (stage == 1) {
-      *(gd2*)(acc + idx) = yi + (dt / 6.0) * r;
-      const d2 x = yi + (dt / 2.0) * r;
+      *(gd2*)(acc + idx) = yi + dt6 * r;
+      const d2 x = yi + dt2 * r;
       *(gt2*)(o + idx) = t2{T(x.x), T(x.y)};
     } else if (stage == 2) {
-      *(gd2*)(acc + idx) = ai + (dt / 3.0) * r;
-      const d2 x = yi + (dt / 2.0) * r;
+      *(gd2*)(acc + idx) = ai + dt3 * r;
+      const d2 x = yi + dt2 * r;
       *(gt2*)(o + idx) = t2{T(x.x), T(x.y)};
     } else if (stage == 3) {
-      *(gd2*)(acc + idx) = ai + (dt / 3.0) * r;
+      *(gd2*)(acc + idx) = ai + dt3 * r;
       const d2 x = yi + dt * r;
       *(gt2*)(o + idx) = t2{T(x.x), T(x.y)};
     } else {
-      const d2 yn = ai + (dt / 6.0) * r;
+      const d2 yn = ai + dt6 * r;
       *(gd2*)(y + idx) = yn;
       if (o) *(gt2*)(o + idx) = t2{T(yn.x), T(yn.y)};
     }
@@ -715,16 +706,16 @@ struct SolveView {
   __device__ __forceinline__ void rk(int stage, int64_t idx, double yi, double ai, double r, int64_t lo = -1) const {
     T* o = out(stage);
     if (stage == 1) {
-      gst(acc + idx, yi + (dt / 6.0) * r);
-      put(o, idx, lo, yi + (dt / 2.0) * r);
+      gst(acc + idx, yi + dt6 * r);
+      put(o, idx, lo, yi + dt2 * r);
     } else if (stage == 2) {
-      gst(acc + idx, ai + (dt / 3.0) * r);
-      put(o, idx, lo, yi + (dt / 2.0) * r);
+      gst(acc + idx, ai + dt3 * r);
+      put(o, idx, lo, yi + dt2 * r);
     } else if (stage == 3) {
-      gst(acc + idx, ai + (dt / 3.0) * r);
+      gst(acc + idx, ai + dt3 * r);
       put(o, idx, lo, yi + dt * r);
     } else {
-      const double yn = ai + (dt / 6.0) * r;
+      const double yn = ai + dt6 * r;
       gst(y + idx, yn);
       if (o) put(o, idx, lo, yn);
     }
@@ -756,8 +747,16 @@ struct SolveView {
 #ifndef GSG_DIRECT64_EB
 #define GSG_DIRECT64_EB 1
 #endif
-template <typename T>
-constexpr int direct_eb() { return sizeof(T) == 4 ? DIRECT_EB : GSG_DIRECT64_EB; }
+#ifndef GSG_DSPLIT_EB
+#define GSG_DSPLIT_EB 4
+#endif
+#ifndef GSG_DSPLIT64_EB
+#define GSG_DSPLIT64_EB 1
+#endif
+template <typename T, bool DS = false>
+constexpr int direct_eb() {
+  return DS ? (sizeof(T) == 4 ? GSG_DSPLIT_EB : GSG_DSPLIT64_EB) : sizeof(T) == 4 ? DIRECT_EB : GSG_DIRECT64_EB;
+}
 // elements of an LDS input slot: a cell (D = 4, k = 4), or the 1 KiB window one
 // 16-byte-a-lane DMA fills (FP64: an 81-double cell from the 16-byte boundary at or below
 // it, or a 64-double cell at D = 3)
@@ -768,15 +767,22 @@ constexpr int direct_lds_bytes() {
   return int(sizeof(T)) * DIRECT_CPW * (direct_eb<T>() * direct_slot<T, D, K>() + kpow(K, D));
 }
 
+// LDS of the split form: per wavefront EB input slots, then the D directions' results
+template <typename T, int D, int K>
+constexpr int direct_split_lds_bytes() {
+  return int(sizeof(T)) * D * direct_eb<T, true>() * direct_slot<T, D, K>() + 8 * D * kpow(K, D);
+}
+
 // wg: the workgroup's group of DIRECT_CPW tiles (blockIdx.x of k_direct, an item of the
-// fused kernel); lds: direct_lds_bytes<T, D, K>() bytes of LDS, 16-byte aligned.
-template <int DT, int KT, typename T, int OPT, int STG>
+// fused kernel), or with DS (one wavefront per direction) its one tile; lds:
+// direct_lds_bytes<T, D, K>() (direct_split_lds_bytes) bytes of LDS, 16-byte aligned.
+template <int DT, int KT, typename T, int OPT, int STG, bool DS = false>
 __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigned char* lds) {
   constexpr int D = DT, K = KT;
   constexpr int KD = ipow_c(K, D);
   constexpr int F = KD / K;  // fibers per direction: lanes f >= F (k = 3) read fiber 0 and discard it
   constexpr int KK = K * K;
-  constexpr int EB = direct_eb<T>();  // LDS slots per wavefront
+  constexpr int EB = direct_eb<T, DS>();  // LDS slots per wavefront
   constexpr int SL = direct_slot<T, D, K>();
   constexpr uint32_t es = sizeof(T);
   constexpr bool FULL = D == 4 && K == 4;              // 256-value cells
@@ -794,19 +800,25 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
   static_assert((FULL && direct_ok(D, K)) || (sizeof(T) == 8 && direct64_ok(D, K) && KD * 8 + 8 <= 1024),
                 "shape not served by the direct kernel");
   T(*Xs)[EB][SL] = reinterpret_cast<T(*)[EB][SL]>(lds);
-  T(*Yw)[KD] = reinterpret_cast<T(*)[KD]>(lds + sizeof(T) * DIRECT_CPW * EB * SL);
+  constexpr int NW = DS ? D : DIRECT_CPW;  // wavefronts
+  T(*Yw)[KD] = reinterpret_cast<T(*)[KD]>(lds + sizeof(T) * NW * EB * SL);
+  double(*P)[KD] = reinterpret_cast<double(*)[KD]>(lds + sizeof(T) * NW * EB * SL);  // DS: direction d's results
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = uni(tid >> 6);
-  T* Y = Yw[wave];
+  T* Y = Yw[DS ? 0 : wave];
   // first scalar loads: this wavefront's tile (padding tiles repeat a real tile with an empty
   // range, so every address below is readable)
-  const Tile* tp = a.tiles + int64_t(wg) * DIRECT_CPW + wave;
+  const Tile* tp = a.tiles + (DS ? int64_t(wg) : int64_t(wg) * DIRECT_CPW + wave);
   const int64_t start = sld(&tp->start);
   const int64_t end = sld(&tp->end);
   const int32_t solve = uni(sld(&tp->solve));
   const uint32_t lens = uint32_t(uni(sld(&tp->blk)));
   const int32_t* ep = reinterpret_cast<const int32_t*>(sld(&tp->aux));
+  if constexpr (DS) {  // this wavefront's direction's entries
+#pragma unroll
+    for (int e = 0; e + 1 < D; ++e) ep += e < wave ? 2 * int((lens >> (8 * e)) & 255u) : 0;
+  }
   // second scalar loads: the first entries and the solve descriptor
   int32_t ew[2 * EB];
 #pragma unroll
@@ -850,9 +862,25 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
   T* w = nullptr;
   if constexpr (OPT == OP_APPLY_GRAD) w = (T*)a.yout;
   if constexpr (OPT == OP_RK_WAVE_GRAD) w = (T*)V.w;
+  // DS: the RK state of output tid, in flight during the gathers
+  double dy = 0.0, da = 0.0, dyn = 0.0, dan = 0.0;
+  T dvn = T(0);
+  if constexpr (DS && (OPT == OP_RK_SUM || OPT == OP_RK_WAVE_SUM)) {
+    if (valid && tid < KD) {
+      const int64_t i = start + tid;
+      if (STG <= 3) dy = V.y_at(i);
+      if (STG >= 2) da = V.acc_at(i);
+      if constexpr (OPT == OP_RK_WAVE_SUM) {
+        if (STG <= 3) dyn = V.y_at(N + i);
+        if (STG >= 2) dan = V.acc_at(N + i);
+        dvn = gld(V.in(STG) + N + i);
+      }
+    }
+  }
   int p0 = 0;  // first entry of direction d in the cell's list
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
+  for (int dd = 0; dd < (DS ? 1 : D); ++dd) {
+    const int d = DS ? wave : dd;
     const int sd = ipow_rt(K, d);
     const bool fib = lane < F;
     const int fc = fib ? lane : 0;
@@ -957,8 +985,11 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
       if constexpr (OPT == OP_APPLY_GRAD || OPT == OP_RK_WAVE_GRAD) {
         if (valid) {
 #pragma unroll
-          for (int q = 0; q < K; ++q) w[int64_t(d) * N + start + vbd + q * sd] = T(r[q]);
+          for (int q = 0; q < K; ++q) gst(w + int64_t(d) * N + start + vbd + q * sd, T(r[q]));
         }
+      } else if constexpr (DS) {
+#pragma unroll
+        for (int q = 0; q < K; ++q) P[d][vbd + q * sd] = r[q];
       } else {
         const double ce = (OPT == OP_APPLY_SUM || OPT == OP_RK_SUM) ? V.coef[d] : 1.0;
 #pragma unroll
@@ -970,7 +1001,12 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
     } else if constexpr (OPT == OP_APPLY_GRAD || OPT == OP_RK_WAVE_GRAD) {
       if (valid && fib) {
 #pragma unroll
-        for (int q = 0; q < K; ++q) w[int64_t(d) * N + start + vbd + q * sd] = acc[q];
+        for (int q = 0; q < K; ++q) gst(w + int64_t(d) * N + start + vbd + q * sd, acc[q]);
+      }
+    } else if constexpr (DS) {
+      if (fib) {
+#pragma unroll
+        for (int q = 0; q < K; ++q) P[d][vbd + q * sd] = acc[q];
       }
     } else if (fib) {
       // sum over directions in direction order (as the other kernels) in this
@@ -986,8 +1022,34 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
       }
     }
   }
-  if (!valid) return;  // whole wavefront; no barrier follows
+  if (!valid) return;  // whole wavefront (DS: whole workgroup); without DS no barrier follows
   if constexpr (OPT == OP_APPLY_GRAD || OPT == OP_RK_WAVE_GRAD) return;
+  if constexpr (DS) {
+    __syncthreads();
+    // one output a lane: the direction sums in direction order
+#pragma unroll
+    for (int m = tid; m < KD; m += 64 * D) {
+      T sum = T(0);
+#pragma unroll
+      for (int e = 0; e < D; ++e) {
+        const double ce = (OPT == OP_APPLY_SUM || OPT == OP_RK_SUM) ? V.coef[e] : 1.0;
+        sum = e == 0 ? T(ce * P[e][m]) : T(__builtin_fma(ce, P[e][m], double(sum)));
+      }
+      const int64_t i = start + m;
+      if constexpr (OPT == OP_APPLY_SUM) {
+        gst((double*)a.yout + i, double(sum));
+      } else if constexpr (OPT == OP_RK_SUM) {
+        V.rk(STG, i, dy, da, double(sum));
+      } else if constexpr (OPT == OP_APPLY_WAVE_SUM) {
+        gst((double*)a.yout + i, double(gld((const T*)a.xin + N + i)));
+        gst((double*)a.yout + N + i, double(sum));
+      } else {
+        V.rk(STG, i, dy, da, double(dvn), 2 * N + i);
+        V.rk(STG, N + i, dyn, dan, double(sum));
+      }
+    }
+    return;
+  }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   if constexpr (OPT == OP_RK_SUM && FULL) {
@@ -1010,15 +1072,15 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
     const int64_t i = start + m;
     const T sum = Y[m];
     if constexpr (OPT == OP_APPLY_SUM) {
-      ((double*)a.yout)[i] = double(sum);
+      gst((double*)a.yout + i, double(sum));
     } else if constexpr (OPT == OP_RK_SUM) {
       V.rk(STG, i, STG <= 3 ? V.y_at(i) : 0.0, STG >= 2 ? V.acc_at(i) : 0.0, double(sum));
     } else if constexpr (OPT == OP_APPLY_WAVE_SUM) {
       const T* x = (const T*)a.xin;
-      ((double*)a.yout)[i] = double(x[N + i]);
-      ((double*)a.yout)[N + i] = double(sum);
+      gst((double*)a.yout + i, double(gld(x + N + i)));
+      gst((double*)a.yout + N + i, double(sum));
     } else {
-      const T vN = V.in(STG)[N + i];
+      const T vN = gld(V.in(STG) + N + i);
       V.rk(STG, i, STG <= 3 ? V.y_at(i) : 0.0, STG >= 2 ? V.acc_at(i) : 0.0, double(vN), 2 * N + i);
       V.rk(STG, N + i, STG <= 3 ? V.y_at(N + i) : 0.0, STG >= 2 ? V.acc_at(N + i) : 0.0, double(sum));
     }
@@ -1029,6 +1091,12 @@ template <int DT, int KT, typename T, int OPT, int STG>
 __global__ __launch_bounds__(TILE) void k_direct(LaunchArgs a) {
   __shared__ __align__(16) unsigned char lds[direct_lds_bytes<T, DT, KT>()];
   direct_body<DT, KT, T, OPT, STG>(a, int(blockIdx.x), lds);
+}
+// one cell a workgroup, one wavefront per direction
+template <int DT, int KT, typename T, int OPT, int STG>
+__global__ __launch_bounds__(64 * DT) void k_direct_ds(LaunchArgs a) {
+  __shared__ __align__(16) unsigned char lds[direct_split_lds_bytes<T, DT, KT>()];
+  direct_body<DT, KT, T, OPT, STG, true>(a, int(blockIdx.x), lds);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1062,7 +1130,17 @@ constexpr int seg_lds_bytes(int D, int K) { return seg_lds_bytes(D, K, seg_eb(D,
 // wg: the workgroup's tiles (blockIdx.x of k_seg, an item of the fused kernel); dsel:
 // the one direction an OP_APPLY_GRAD workgroup runs (-1: all); lds: seg_lds_bytes(D, K)
 // bytes of LDS, 16-byte aligned.
-template <int DT, int KT, int OPT, int STG, int EBX = 0>
+// With DS (one wavefront per direction) wg is the workgroup's one group of seg_cpw cells
+// and lds holds seg_split_lds_bytes(D, K) bytes: D wavefronts' input slots, then the D
+// directions' results in double.
+#ifndef GSG_SSPLIT_EB
+#define GSG_SSPLIT_EB seg_eb(D, K)
+#endif
+constexpr int seg_split_eb(int D, int K) { return GSG_SSPLIT_EB; }
+constexpr int seg_split_lds_bytes(int D, int K) {
+  return 1024 * D * seg_split_eb(D, K) + 8 * D * seg_cpw(D, K) * kpow(K, D);
+}
+template <int DT, int KT, int OPT, int STG, int EBX = 0, bool DS = false>
 __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, unsigned char* lds) {
   typedef float T;
   typedef float v4f __attribute__((ext_vector_type(4)));
@@ -1071,7 +1149,7 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
   constexpr int F = KD / K;
   constexpr int S = seg_lanes(D, K);
   constexpr int CPW = seg_cpw(D, K);
-  constexpr int EB = EBX ? EBX : seg_eb(D, K);  // entries a round (EBX: the tuned alternative)
+  constexpr int EB = DS ? seg_split_eb(D, K) : EBX ? EBX : seg_eb(D, K);  // entries a round (EBX: the tuned alternative)
   static_assert(EB >= 1 && EB <= 8, "the block broadcast addresses at most 8 slots");
   constexpr uint32_t es = 4;
   constexpr int NOUT = CPW * KD;  // outputs of a wavefront
@@ -1096,16 +1174,18 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
   static_assert(seg_ok(D, K) && KD * 4 + (ALN ? 0 : 12) <= 16 * S && S % 4 == 0,
                 "shape not served by the segmented kernel");
   float(*Xs)[EB][SLOT] = reinterpret_cast<float(*)[EB][SLOT]>(lds);
-  float(*Yw)[NOUT] = reinterpret_cast<float(*)[NOUT]>(lds + 4 * SEG_WAVES * EB * SLOT);
+  constexpr int NW = DS ? D : SEG_WAVES;  // wavefronts
+  float(*Yw)[NOUT] = reinterpret_cast<float(*)[NOUT]>(lds + 4 * NW * EB * SLOT);
+  double(*P)[NOUT] = reinterpret_cast<double(*)[NOUT]>(lds + 4 * NW * EB * SLOT);  // DS: direction d's results
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = uni(tid >> 6);
   const int seg = lane / S;
   const int fl = lane - seg * S;
   const bool fib = fl < F;  // a real fiber
-  float* Y = Yw[wave];
+  float* Y = Yw[DS ? 0 : wave];
   // this lane's cell (all tiles of a wavefront belong to one solve)
-  const int64_t t0 = (int64_t(wg) * SEG_WAVES + wave) * CPW;
+  const int64_t t0 = (DS ? int64_t(wg) : int64_t(wg) * SEG_WAVES + wave) * CPW;
   const Tile* tp = a.tiles + t0 + seg;
   const int64_t start = tp->start;
   const int64_t end = tp->end;
@@ -1155,12 +1235,18 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
   if constexpr (OPT == OP_APPLY_GRAD) w = (T*)a.yout;
   if constexpr (OPT == OP_RK_WAVE_GRAD) w = (T*)V.w;
   // per direction: this cell's list length and first entry, and the wavefront's rounds
-  int lraw[D], p0v[D], nrd[D];
+  // (DS: of this wavefront's direction, as index 0)
+  constexpr int ND = DS ? 1 : D;
+  int lraw[ND], p0v[ND], nrd[ND];
   {
     int c = 0;
+    if constexpr (DS) {
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      lraw[d] = int((lens >> (8 * d)) & 255u);
+      for (int e = 0; e + 1 < D; ++e) c += e < wave ? int((lens >> (8 * e)) & 255u) : 0;
+    }
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      lraw[d] = int((lens >> (8 * (DS ? wave : d))) & 255u);
       p0v[d] = c;
       c += lraw[d];
       const int lv = valid ? lraw[d] : 0;
@@ -1182,7 +1268,7 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
   // SEW: every cell's entry address, list lengths and first entries as wave-uniform
   // values, read from the cell's first lane once
   const int32_t* epq[SEW ? CPW : 1];
-  int lqd[SEW ? CPW : 1][D], pqd[SEW ? CPW : 1][D];
+  int lqd[SEW ? CPW : 1][ND], pqd[SEW ? CPW : 1][ND];
   if constexpr (SEW) {
     const uint64_t epa = reinterpret_cast<uintptr_t>(ep);
 #pragma unroll
@@ -1191,7 +1277,7 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
       const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(epa >> 32)), q * S));
       epq[q] = reinterpret_cast<const int32_t*>(uintptr_t((uint64_t(hi) << 32) | lo));
 #pragma unroll
-      for (int e = 0; e < D; ++e) {
+      for (int e = 0; e < ND; ++e) {
         lqd[q][e] = __builtin_amdgcn_readlane(lraw[e], q * S);
         pqd[q][e] = __builtin_amdgcn_readlane(p0v[e], q * S);
       }
@@ -1216,14 +1302,37 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
 #pragma unroll
       for (int u = 0; u < EB; ++u) {
         const bool in = c0 + u < lraw[dd];
-        dst[u] = *reinterpret_cast<const int2*>(ep + 2 * (in ? p0v[dd] + c0 + u : 0));
+        dst[u] = gld2(ep + 2 * (in ? p0v[dd] + c0 + u : 0));
       }
     }
   };
+  // DS: the RK state of outputs tid and tid + 64 D, in flight during the gathers
+  constexpr int NO = DS ? (NOUT + 64 * D - 1) / (64 * D) : 1;
+  double dy[NO], da[NO], dyn[NO], dan[NO];
+  T dvn[NO];
+  if constexpr (DS && (OPT == OP_RK_SUM || OPT == OP_RK_WAVE_SUM)) {
+#pragma unroll
+    for (int t = 0; t < NO; ++t) {
+      const int m = tid + t * 64 * D;
+      dy[t] = da[t] = dyn[t] = dan[t] = 0.0;
+      dvn[t] = T(0);
+      if (m < NOUT && ((cmask >> ((m / KD) * S)) & 1u)) {
+        const int64_t i = start0 + m;
+        if (STG <= 3) dy[t] = V.y_at(i);
+        if (STG >= 2) da[t] = V.acc_at(i);
+        if constexpr (OPT == OP_RK_WAVE_SUM) {
+          if (STG <= 3) dyn[t] = V.y_at(N + i);
+          if (STG >= 2) dan[t] = V.acc_at(N + i);
+          dvn[t] = gld(V.in(STG) + N + i);
+        }
+      }
+    }
+  }
   fetch(ewc, 0, 0);
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
-    if constexpr (OPT == OP_APPLY_GRAD) {
+  for (int dd = 0; dd < (DS ? 1 : D); ++dd) {
+    const int d = DS ? wave : dd;  // the lists' index is dd
+    if constexpr (OPT == OP_APPLY_GRAD && !DS) {
       if (dsel >= 0 && d != dsel) {  // wave-uniform
         if (d < dsel) fetch(ewc, d + 1 < D ? d + 1 : d, 0);  // the next direction's first entries
         continue;
@@ -1232,8 +1341,8 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
     const int sdd = ipow_rt(K, d);
     const int flc = fib ? fl : 0;  // padding lanes read (and discard) fiber 0
     const int vbd = flc % sdd + (flc / sdd) * sdd * K;  // the fiber's element with digit d = 0
-    const int len = lraw[d];
-    const int nr = nrd[d];
+    const int len = lraw[dd];
+    const int nr = nrd[dd];
     const uint32_t xbase = uint32_t(int64_t(d) * dstride * 4);
     v4f accv = {0.f, 0.f, 0.f, 0.f}, accl = {0.f, 0.f, 0.f, 0.f};
     for (int part = 0; part < npart; ++part)
@@ -1289,11 +1398,11 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
       // the next round's entry words (this direction's next round or the next
       // direction's first), in flight with this round's loads
       if (c0 + EB < nr)
-        fetch(ewn, d, c0 + EB);
+        fetch(ewn, dd, c0 + EB);
       else if (part + 1 < npart)
-        fetch(ewn, d, 0);  // the direction's first entries again, for the second part
-      else if (d + 1 < D)
-        fetch(ewn, d + 1 < D ? d + 1 : d, 0);
+        fetch(ewn, dd, 0);  // the direction's first entries again, for the second part
+      else if (!DS && d + 1 < D)
+        fetch(ewn, d + 1 < ND ? d + 1 : 0, 0);
       __builtin_amdgcn_s_waitcnt(0);  // the DMA into LDS (and everything else) has landed
 #pragma unroll
       for (int u = 0; u < EB; ++u) {
@@ -1334,7 +1443,7 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
       // the next round's DMA rewrites the slots only after these reads (the MFMAs above
       // consumed them)
     }
-    if (nr == 0 && d + 1 < D) fetch(ewc, d + 1 < D ? d + 1 : d, 0);  // no round ran
+    if (!DS && nr == 0 && d + 1 < D) fetch(ewc, d + 1 < ND ? d + 1 : 0, 0);  // no round ran
     // the hi and lo sums and the coefficient in double
     double r[K];
 #pragma unroll
@@ -1342,7 +1451,12 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
     if constexpr (OPT == OP_APPLY_GRAD || OPT == OP_RK_WAVE_GRAD) {
       if (valid && fib) {
 #pragma unroll
-        for (int q = 0; q < K; ++q) w[int64_t(d) * N + start + vbd + q * sdd] = T(r[q]);
+        for (int q = 0; q < K; ++q) gst(w + int64_t(d) * N + start + vbd + q * sdd, T(r[q]));
+      }
+    } else if constexpr (DS) {
+      if (fib) {
+#pragma unroll
+        for (int q = 0; q < K; ++q) P[d][seg * KD + vbd + q * sdd] = r[q];
       }
     } else {
       // sum over directions in direction order in the wavefront's LDS row (float)
@@ -1357,6 +1471,33 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
     }
   }
   if constexpr (OPT == OP_APPLY_GRAD || OPT == OP_RK_WAVE_GRAD) return;
+  if constexpr (DS) {
+    __syncthreads();  // every wavefront of the workgroup gets here
+#pragma unroll
+    for (int t = 0; t < NO; ++t) {
+      const int m = tid + t * 64 * D;
+      if (m >= NOUT || !((cmask >> ((m / KD) * S)) & 1u)) continue;
+      T sum = T(0);
+#pragma unroll
+      for (int e = 0; e < D; ++e) {
+        const double ce = (OPT == OP_APPLY_SUM || OPT == OP_RK_SUM) ? V.coef[e] : 1.0;
+        sum = e == 0 ? T(ce * P[e][m]) : T(__builtin_fma(ce, P[e][m], double(sum)));
+      }
+      const int64_t i = start0 + m;
+      if constexpr (OPT == OP_APPLY_SUM) {
+        gst((double*)a.yout + i, double(sum));
+      } else if constexpr (OPT == OP_RK_SUM) {
+        V.rk(STG, i, dy[t], da[t], double(sum));
+      } else if constexpr (OPT == OP_APPLY_WAVE_SUM) {
+        gst((double*)a.yout + i, double(gld((const T*)a.xin + N + i)));
+        gst((double*)a.yout + N + i, double(sum));
+      } else {
+        V.rk(STG, i, dy[t], da[t], double(dvn[t]), 2 * N + i);
+        V.rk(STG, N + i, dyn[t], dan[t], double(sum));
+      }
+    }
+    return;
+  }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   if constexpr (OPT == OP_RK_SUM) {
@@ -1392,15 +1533,15 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
     const int64_t i = start0 + m;
     const T sum = Y[m];
     if constexpr (OPT == OP_APPLY_SUM) {
-      ((double*)a.yout)[i] = double(sum);
+      gst((double*)a.yout + i, double(sum));
     } else if constexpr (OPT == OP_RK_SUM) {
       V.rk(STG, i, STG <= 3 ? V.y_at(i) : 0.0, STG >= 2 ? V.acc_at(i) : 0.0, double(sum));
     } else if constexpr (OPT == OP_APPLY_WAVE_SUM) {
       const T* x = (const T*)a.xin;
-      ((double*)a.yout)[i] = double(x[N + i]);
-      ((double*)a.yout)[N + i] = double(sum);
+      gst((double*)a.yout + i, double(gld(x + N + i)));
+      gst((double*)a.yout + N + i, double(sum));
     } else {
-      const T vN = V.in(STG)[N + i];
+      const T vN = gld(V.in(STG) + N + i);
       V.rk(STG, i, STG <= 3 ? V.y_at(i) : 0.0, STG >= 2 ? V.acc_at(i) : 0.0, double(vN), 2 * N + i);
       V.rk(STG, N + i, STG <= 3 ? V.y_at(N + i) : 0.0, STG >= 2 ? V.acc_at(N + i) : 0.0, double(sum));
     }
@@ -1416,14 +1557,32 @@ __global__ __launch_bounds__(TILE) void k_seg(LaunchArgs a) {
   seg_body<DT, KT, OPT, STG, EBX>(a, int(blockIdx.x), dsel, lds);
 }
 
+// seg_cpw cells a workgroup, one wavefront per direction
+template <int DT, int KT, int OPT, int STG>
+__global__ __launch_bounds__(64 * DT) void k_seg_ds(LaunchArgs a) {
+  __shared__ __align__(16) unsigned char lds[seg_split_lds_bytes(DT, KT)];
+  seg_body<DT, KT, OPT, STG, 0, true>(a, int(blockIdx.x), -1, lds);
+}
+
+template <int DT, int KT, int OPT, int STG, int EBX = 0>
+static void launch_seg_op(const LaunchArgs& a, hipStream_t s) {
+  const dim3 grid(unsigned(a.ntiles / (SEG_WAVES * seg_cpw(DT, KT))));
+  // without the split, the gradient of a grid of fewer than 1024 workgroups (4 per CU)
+  // runs one direction per grid row: measured on the 2 + 2 dimensional Vlasov derivative
+  // (k = 2, n = 8)
+  const dim3 ggrid(grid.x, OPT == OP_APPLY_GRAD && grid.x < 1024 ? unsigned(DT) : 1u);
+  if (a.dsplit)
+    hipLaunchKernelGGL((k_seg_ds<DT, KT, OPT, STG>), dim3(unsigned(a.ntiles / seg_cpw(DT, KT))), dim3(64 * DT), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_seg<DT, KT, OPT, STG, EBX>), ggrid, dim3(TILE), 0, s, a);
+}
 template <int DT, int KT, int OPT, int EBX = 0>
 static void launch_seg_stage(const LaunchArgs& a, hipStream_t s) {
-  const dim3 grid(unsigned(a.ntiles / (SEG_WAVES * seg_cpw(DT, KT))));
   switch (a.stage) {
-    case 1: hipLaunchKernelGGL((k_seg<DT, KT, OPT, 1, EBX>), grid, dim3(TILE), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((k_seg<DT, KT, OPT, 2, EBX>), grid, dim3(TILE), 0, s, a); break;
-    case 3: hipLaunchKernelGGL((k_seg<DT, KT, OPT, 3, EBX>), grid, dim3(TILE), 0, s, a); break;
-    default: hipLaunchKernelGGL((k_seg<DT, KT, OPT, 4, EBX>), grid, dim3(TILE), 0, s, a); break;
+    case 1: launch_seg_op<DT, KT, OPT, 1, EBX>(a, s); break;
+    case 2: launch_seg_op<DT, KT, OPT, 2, EBX>(a, s); break;
+    case 3: launch_seg_op<DT, KT, OPT, 3, EBX>(a, s); break;
+    default: launch_seg_op<DT, KT, OPT, 4, EBX>(a, s); break;
   }
 }
 
@@ -1431,7 +1590,7 @@ static void launch_seg_stage(const LaunchArgs& a, hipStream_t s) {
 // the rule's)
 template <int DT, int KT>
 static hipError_t launch_seg_alt(const LaunchArgs& a, hipStream_t s) {
-  if (a.ntiles % (SEG_WAVES * seg_cpw(DT, KT))) return hipErrorInvalidValue;  // the host pads
+  if (a.ntiles % ((a.dsplit ? 1 : SEG_WAVES) * seg_cpw(DT, KT))) return hipErrorInvalidValue;  // the host pads
   constexpr int E = seg_eb_alt(DT, KT);
   switch (a.op) {
     case OP_RK_SUM: launch_seg_stage<DT, KT, OP_RK_SUM, E>(a, s); break;
@@ -1444,15 +1603,11 @@ static hipError_t launch_seg_alt(const LaunchArgs& a, hipStream_t s) {
 
 template <int DT, int KT>
 static hipError_t launch_seg(const LaunchArgs& a, hipStream_t s) {
-  if (a.ntiles % (SEG_WAVES * seg_cpw(DT, KT))) return hipErrorInvalidValue;  // the host pads
-  const dim3 grid(unsigned(a.ntiles / (SEG_WAVES * seg_cpw(DT, KT))));
-  // the gradient of a grid of fewer than 1024 workgroups (4 per CU) runs one direction
-  // per grid row: measured on the 2 + 2 dimensional Vlasov derivative (k = 2, n = 8)
-  const dim3 ggrid(grid.x, grid.x < 1024 ? unsigned(DT) : 1u);
+  if (a.ntiles % ((a.dsplit ? 1 : SEG_WAVES) * seg_cpw(DT, KT))) return hipErrorInvalidValue;  // the host pads
   switch (a.op) {
-    case OP_APPLY_SUM: hipLaunchKernelGGL((k_seg<DT, KT, OP_APPLY_SUM, 0>), grid, dim3(TILE), 0, s, a); break;
-    case OP_APPLY_GRAD: hipLaunchKernelGGL((k_seg<DT, KT, OP_APPLY_GRAD, 0>), ggrid, dim3(TILE), 0, s, a); break;
-    case OP_APPLY_WAVE_SUM: hipLaunchKernelGGL((k_seg<DT, KT, OP_APPLY_WAVE_SUM, 0>), grid, dim3(TILE), 0, s, a); break;
+    case OP_APPLY_SUM: launch_seg_op<DT, KT, OP_APPLY_SUM, 0>(a, s); break;
+    case OP_APPLY_GRAD: launch_seg_op<DT, KT, OP_APPLY_GRAD, 0>(a, s); break;
+    case OP_APPLY_WAVE_SUM: launch_seg_op<DT, KT, OP_APPLY_WAVE_SUM, 0>(a, s); break;
     case OP_RK_SUM: launch_seg_stage<DT, KT, OP_RK_SUM>(a, s); break;
     case OP_RK_WAVE_GRAD: launch_seg_stage<DT, KT, OP_RK_WAVE_GRAD>(a, s); break;
     case OP_RK_WAVE_SUM: launch_seg_stage<DT, KT, OP_RK_WAVE_SUM>(a, s); break;
@@ -1547,7 +1702,7 @@ __device__ __forceinline__ void seg64_body(const LaunchArgs& a, int wg, unsigned
   }
   // this lane's cell's entry words of round c0 of direction dd (its first entry past the list)
   auto fetch = [&](int dd, int c0) {
-    return *reinterpret_cast<const int2*>(ep + 2 * (c0 < lraw[dd] ? p0v[dd] + c0 : 0));
+    return gld2(ep + 2 * (c0 < lraw[dd] ? p0v[dd] + c0 : 0));
   };
   int2 ewc = fetch(0, 0);
 #pragma unroll
@@ -1586,7 +1741,7 @@ __device__ __forceinline__ void seg64_body(const LaunchArgs& a, int wg, unsigned
     if constexpr (OPT == OP_APPLY_GRAD || OPT == OP_RK_WAVE_GRAD) {
       if (valid && fib) {
 #pragma unroll
-        for (int q = 0; q < K; ++q) w[int64_t(d) * N + start + vbd + q * sd] = acc[q];
+        for (int q = 0; q < K; ++q) gst(w + int64_t(d) * N + start + vbd + q * sd, acc[q]);
       }
     } else if (fib) {
       // sum over directions in direction order: Y = c_0 a_0, then Y = fma(c_d, a_d, Y)
@@ -1611,15 +1766,15 @@ __device__ __forceinline__ void seg64_body(const LaunchArgs& a, int wg, unsigned
     const int64_t i = start0 + m;
     const T sum = Y[m];
     if constexpr (OPT == OP_APPLY_SUM) {
-      ((double*)a.yout)[i] = double(sum);
+      gst((double*)a.yout + i, double(sum));
     } else if constexpr (OPT == OP_RK_SUM) {
       V.rk(STG, i, STG <= 3 ? V.y_at(i) : 0.0, STG >= 2 ? V.acc_at(i) : 0.0, double(sum));
     } else if constexpr (OPT == OP_APPLY_WAVE_SUM) {
       const T* x = (const T*)a.xin;
-      ((double*)a.yout)[i] = double(x[N + i]);
-      ((double*)a.yout)[N + i] = double(sum);
+      gst((double*)a.yout + i, double(gld(x + N + i)));
+      gst((double*)a.yout + N + i, double(sum));
     } else {
-      const T vN = V.in(STG)[N + i];
+      const T vN = gld(V.in(STG) + N + i);
       V.rk(STG, i, STG <= 3 ? V.y_at(i) : 0.0, STG >= 2 ? V.acc_at(i) : 0.0, double(vN));
       V.rk(STG, N + i, STG <= 3 ? V.y_at(N + i) : 0.0, STG >= 2 ? V.acc_at(N + i) : 0.0, double(sum));
     }
@@ -1658,29 +1813,30 @@ static hipError_t launch_seg64(const LaunchArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <int DT, int KT, typename T, int OPT, int STG>
+static void launch_direct_op(const LaunchArgs& a, hipStream_t s) {
+  if (a.dsplit)
+    hipLaunchKernelGGL((k_direct_ds<DT, KT, T, OPT, STG>), dim3(a.ntiles), dim3(64 * DT), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_direct<DT, KT, T, OPT, STG>), dim3(a.ntiles / DIRECT_CPW), dim3(TILE), 0, s, a);
+}
 template <int DT, int KT, typename T, int OPT>
 static void launch_direct_stage(const LaunchArgs& a, hipStream_t s) {
   switch (a.stage) {
-    case 1: hipLaunchKernelGGL((k_direct<DT, KT, T, OPT, 1>), dim3(a.ntiles / DIRECT_CPW), dim3(TILE), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((k_direct<DT, KT, T, OPT, 2>), dim3(a.ntiles / DIRECT_CPW), dim3(TILE), 0, s, a); break;
-    case 3: hipLaunchKernelGGL((k_direct<DT, KT, T, OPT, 3>), dim3(a.ntiles / DIRECT_CPW), dim3(TILE), 0, s, a); break;
-    default: hipLaunchKernelGGL((k_direct<DT, KT, T, OPT, 4>), dim3(a.ntiles / DIRECT_CPW), dim3(TILE), 0, s, a); break;
+    case 1: launch_direct_op<DT, KT, T, OPT, 1>(a, s); break;
+    case 2: launch_direct_op<DT, KT, T, OPT, 2>(a, s); break;
+    case 3: launch_direct_op<DT, KT, T, OPT, 3>(a, s); break;
+    default: launch_direct_op<DT, KT, T, OPT, 4>(a, s); break;
   }
 }
 
 template <int DT, int KT, typename T>
 static hipError_t launch_direct(const LaunchArgs& a, hipStream_t s) {
-  if (a.ntiles % DIRECT_CPW) return hipErrorInvalidValue;  // the host pads to whole workgroups
+  if (!a.dsplit && a.ntiles % DIRECT_CPW) return hipErrorInvalidValue;  // the host pads to whole workgroups
   switch (a.op) {
-    case OP_APPLY_SUM:
-      hipLaunchKernelGGL((k_direct<DT, KT, T, OP_APPLY_SUM, 0>), dim3(a.ntiles / DIRECT_CPW), dim3(TILE), 0, s, a);
-      break;
-    case OP_APPLY_GRAD:
-      hipLaunchKernelGGL((k_direct<DT, KT, T, OP_APPLY_GRAD, 0>), dim3(a.ntiles / DIRECT_CPW), dim3(TILE), 0, s, a);
-      break;
-    case OP_APPLY_WAVE_SUM:
-      hipLaunchKernelGGL((k_direct<DT, KT, T, OP_APPLY_WAVE_SUM, 0>), dim3(a.ntiles / DIRECT_CPW), dim3(TILE), 0, s, a);
-      break;
+    case OP_APPLY_SUM: launch_direct_op<DT, KT, T, OP_APPLY_SUM, 0>(a, s); break;
+    case OP_APPLY_GRAD: launch_direct_op<DT, KT, T, OP_APPLY_GRAD, 0>(a, s); break;
+    case OP_APPLY_WAVE_SUM: launch_direct_op<DT, KT, T, OP_APPLY_WAVE_SUM, 0>(a, s); break;
     case OP_RK_SUM: launch_direct_stage<DT, KT, T, OP_RK_SUM>(a, s); break;
     case OP_RK_WAVE_GRAD: launch_direct_stage<DT, KT, T, OP_RK_WAVE_GRAD>(a, s); break;
     case OP_RK_WAVE_SUM: launch_direct_stage<DT, KT, T, OP_RK_WAVE_SUM>(a, s); break;
@@ -1916,24 +2072,20 @@ __device__ __forceinline__ RkIn rk_stage_in(int stage, int64_t i, const double* 
 // (the stage epilogue of the fused kernels, rk_update), applied by the last sweep of the
 // Vlasov right-hand side; x receives the next stage input (stage < 4) or the new state's
 // copy, and x32 (when not null) its float copy for an FP32 operator.
-__device__ __forceinline__ void rk_stage_at(int stage, int64_t i, double dt, RkIn in, double* y, double* acc,
-                                            double ri, double* x, float* x32) {
+__device__ __forceinline__ void rk_stage_at(const XRk& rk, int64_t i, RkIn in, double ri) {
   double xn;
-  if (stage == 1) {
-    gst(acc + i, in.y + (dt / 6.0) * ri);
-    xn = in.y + (dt / 2.0) * ri;
-  } else if (stage == 2) {
-    gst(acc + i, in.acc + (dt / 3.0) * ri);
-    xn = in.y + (dt / 2.0) * ri;
-  } else if (stage == 3) {
-    gst(acc + i, in.acc + (dt / 3.0) * ri);
-    xn = in.y + dt * ri;
+  if (rk.stage == 1) {
+    gst(rk.acc + i, in.y + rk.wa * ri);
+    xn = in.y + rk.wx * ri;
+  } else if (rk.stage <= 3) {
+    gst(rk.acc + i, in.acc + rk.wa * ri);
+    xn = in.y + rk.wx * ri;
   } else {
-    xn = in.acc + (dt / 6.0) * ri;
-    gst(y + i, xn);
+    xn = in.acc + rk.wa * ri;
+    gst(rk.y + i, xn);
   }
-  gst(x + i, xn);
-  if (x32) gst(x32 + i, float(xn));
+  gst(rk.x + i, xn);
+  if (rk.x32) gst(rk.x32 + i, float(xn));
 }
 
 // One direction sweep of a sparse-grid basis transform (the 1-D transform along
@@ -1990,7 +2142,7 @@ __global__ __launch_bounds__(TILE) void k_xsweep(LaunchArgs a, XComb cb, XRk rk,
       }
       gst((double*)a.yout + i, cb.F ? -c1 + c2 : -c1);
     } else if (rk.stage) {
-      rk_stage_at(rk.stage, i, rk.dt, in, rk.y, rk.acc, r[0], rk.x, rk.x32);
+      rk_stage_at(rk, i, in, r[0]);
     } else {
 #pragma unroll
       for (int v = 0; v < NV; ++v) gst((double*)a.yout + int64_t(v0 + v) * N + i, r[v]);
@@ -2191,9 +2343,9 @@ template hipError_t launch_d<1>(int, bool, const LaunchArgs&, hipStream_t);
 template hipError_t launch_d<5>(int, bool, const LaunchArgs&, hipStream_t);
 template hipError_t launch_d<6>(int, bool, const LaunchArgs&, hipStream_t);
 hipError_t launch_any(bool fp32, const LaunchArgs& a, hipStream_t s) { return launch_tk<0, 0>(fp32, a, s); }
-#elif GSG_PART > 1
+#elif GSG_PART > 1 && GSG_PART < 9
 template hipError_t launch_d<GSG_PART>(int, bool, const LaunchArgs&, hipStream_t);
-#else
+#elif GSG_PART == 0
 extern template hipError_t launch_d<1>(int, bool, const LaunchArgs&, hipStream_t);
 extern template hipError_t launch_d<2>(int, bool, const LaunchArgs&, hipStream_t);
 extern template hipError_t launch_d<3>(int, bool, const LaunchArgs&, hipStream_t);
@@ -2235,7 +2387,7 @@ hipError_t launch_xsweep(int K, int nvec, const LaunchArgs& a, hipStream_t s, bo
   if (a.ntiles <= 0 || nvec <= 0) return hipSuccess;
   if (ell && K != 2) return hipErrorInvalidValue;  // the table exists for k = 2 only
   const XComb none{nullptr, nullptr, 0, 1};
-  const XRk nork{0, 0.0, nullptr, nullptr, nullptr, nullptr};
+  const XRk nork{0, 0.0, 0.0, nullptr, nullptr, nullptr, nullptr};
   if (rk && rk->stage && (comb || nvec != 1)) return hipErrorInvalidValue;  // one plain vector only
   const XRk& r = rk ? *rk : nork;
   if (comb) {

@@ -39,7 +39,7 @@ struct Tab<float> {
 // the blocks (LDS or global), vlo: elements from the hi to the lo table; off[q]: fiber q's
 // element with the direction's mode digit 0, sd the digit's stride.  U entries a round.
 // HI2: the hi table into accl only.
-template <int K, int KD, int G, int R, int U, bool HI2, typename T>
+template <int K, int KD, int G, int R, int U, bool HI2, bool VL, typename T>
 __device__ __forceinline__ void round_of(const uint32_t (&e)[U], const T* v, int vlo, const T* x, const int (&off)[G],
                                          int sd, T (&acc)[G][R], T (&accl)[G][R]) {
   constexpr bool HL = sizeof(T) == 4;
@@ -50,8 +50,8 @@ __device__ __forceinline__ void round_of(const uint32_t (&e)[U], const T* v, int
     const T* xp = x + int(e[u] & 0xffffu) * KD;
 #pragma unroll
     for (int q = 0; q < R * K; ++q) {
-      b[u][q] = vp[q];
-      if constexpr (HL && !HI2) bl[u][q] = vp[vlo + q];
+      b[u][q] = VL ? vp[q] : gld(vp + q);
+      if constexpr (HL && !HI2) bl[u][q] = VL ? vp[vlo + q] : gld(vp + vlo + q);
     }
 #pragma unroll
     for (int q = 0; q < G; ++q)
@@ -74,7 +74,7 @@ __device__ __forceinline__ void round_of(const uint32_t (&e)[U], const T* v, int
           }
         }
 }
-template <int K, int KD, int G, int R, int U, bool HI2, typename T>
+template <int K, int KD, int G, int R, int U, bool HI2, bool VL, typename T>
 __device__ __forceinline__ void list(const uint32_t* ent, int p0, int p1, const T* v, int vlo, const T* x,
                                      const int (&off)[G], int sd, T (&acc)[G][R], T (&accl)[G][R]) {
   int p = p0;
@@ -89,13 +89,13 @@ __device__ __forceinline__ void list(const uint32_t* ent, int p0, int p1, const 
       p += U;
 #pragma unroll
       for (int u = 0; u < U; ++u) e[u] = ent[min(p + u, p1 - 1)];  // the next round's words
-      round_of<K, KD, G, R, U, HI2>(c, v, vlo, x, off, sd, acc, accl);
+      round_of<K, KD, G, R, U, HI2, VL>(c, v, vlo, x, off, sd, acc, accl);
     } while (p + U <= p1);
   }
   if constexpr (U > 1)
     for (; p < p1; ++p) {
       const uint32_t c[1] = {ent[p]};
-      round_of<K, KD, G, R, 1, HI2>(c, v, vlo, x, off, sd, acc, accl);
+      round_of<K, KD, G, R, 1, HI2, VL>(c, v, vlo, x, off, sd, acc, accl);
     }
 }
 
@@ -112,28 +112,28 @@ struct RkRegs {
 };
 __device__ __forceinline__ RkRegs rk_load(int stage, const double* y, const double* acc, int64_t i) {
   RkRegs q;
-  q.y = stage <= 3 ? y[i] : 0.0;
-  q.acc = stage >= 2 ? acc[i] : 0.0;
+  q.y = stage <= 3 ? gld(y + i) : 0.0;
+  q.acc = stage >= 2 ? gld(acc + i) : 0.0;
   return q;
 }
 // the classical RK4 stage update of state entry i with derivative r; returns the next
 // stage input
-__device__ __forceinline__ double rk_stage(int stage, double dt, double* y, double* acc, int64_t i, const RkRegs& q,
+__device__ __forceinline__ double rk_stage(int stage, const SolveDesc& S, double* y, double* acc, int64_t i, const RkRegs& q,
                                            double r) {
   if (stage == 1) {
-    acc[i] = q.y + (dt / 6.0) * r;
-    return q.y + (dt / 2.0) * r;
+    gst(acc + i, q.y + S.dt6 * r);
+    return q.y + S.dt2 * r;
   }
   if (stage == 2) {
-    acc[i] = q.acc + (dt / 3.0) * r;
-    return q.y + (dt / 2.0) * r;
+    gst(acc + i, q.acc + S.dt3 * r);
+    return q.y + S.dt2 * r;
   }
   if (stage == 3) {
-    acc[i] = q.acc + (dt / 3.0) * r;
-    return q.y + dt * r;
+    gst(acc + i, q.acc + S.dt3 * r);
+    return q.y + S.dt * r;
   }
-  const double yn = q.acc + (dt / 6.0) * r;
-  y[i] = yn;
+  const double yn = q.acc + S.dt6 * r;
+  gst(y + i, yn);
   return yn;
 }
 
@@ -149,7 +149,7 @@ __device__ __forceinline__ void run(const SoloArgs& a, const SolveDesc& S, unsig
   const int NT = int(blockDim.x), tid = int(threadIdx.x);
   const bool wave = S.sys == SYS_WAVE;
   const int ncell = N / KD;
-  const int ne = S.t.plan_ptr[int64_t(ncell) * D];
+  const int ne = gld(S.t.plan_ptr + int64_t(ncell) * D);
   // LDS (SoloLds): the D direction sums in double; the stage input x, or for the wave u,
   // v, the D gradient vectors and (float) u's remainder; the lists, the tasks' words, the
   // blocks
@@ -166,11 +166,11 @@ __device__ __forceinline__ void run(const SoloArgs& a, const SolveDesc& S, unsig
   const int nv = int(S.t.val_elems);
   const T* vg = Tab<T>::vals(S.t);
   const int ntask = ncell * D;  // (direction, cell) words, NG fiber groups each
-  for (int q = tid; q < ne; q += NT) ent[q] = S.t.solo_ent[q];
-  for (int q = tid; q <= ntask; q += NT) ptr[q] = S.t.plan_ptr[q];
-  for (int q = tid; q < ntask; q += NT) task[q] = S.t.solo_ent[ne + q];
+  for (int q = tid; q < ne; q += NT) ent[q] = gld(S.t.solo_ent + q);
+  for (int q = tid; q <= ntask; q += NT) ptr[q] = gld(S.t.plan_ptr + q);
+  for (int q = tid; q < ntask; q += NT) task[q] = gld(S.t.solo_ent + ne + q);
   if constexpr (VL)
-    for (int q = tid; q < nv * (HL ? 2 : 1); q += NT) vl[q] = vg[q];
+    for (int q = tid; q < nv * (HL ? 2 : 1); q += NT) vl[q] = gld(vg + q);
   const T* v;
   if constexpr (VL)
     v = vl;
@@ -178,7 +178,6 @@ __device__ __forceinline__ void run(const SoloArgs& a, const SolveDesc& S, unsig
     v = vg;
   double* const y = S.y;
   double* const acc = S.acc;
-  const double dt = S.dt;
   const int d0 = S.dir0, d1 = S.dir0 + S.ndir;
   double coef[D];
 #pragma unroll
@@ -212,15 +211,15 @@ __device__ __forceinline__ void run(const SoloArgs& a, const SolveDesc& S, unsig
           for (int r = 0; r < R; ++r) ac[q][r] = al[q][r] = T(0);
       };
       clear();
-      list<K, KD, G, R, U, false>(ent, p0, p1, vr, nv, xin + d * xs, off, sd, ac, al);
-      if (HL && SEGR && grad) list<K, KD, G, R, U, true>(ent, p0, p1, vr, nv, ulo, off, sd, ac, al);
+      list<K, KD, G, R, U, false, VL>(ent, p0, p1, vr, nv, xin + d * xs, off, sd, ac, al);
+      if (HL && SEGR && grad) list<K, KD, G, R, U, true, VL>(ent, p0, p1, vr, nv, ulo, off, sd, ac, al);
 #pragma unroll
       for (int q = 0; q < G; ++q)
 #pragma unroll
         for (int r = 0; r < R; ++r) s[q][r] = HL ? double(ac[q][r]) + double(al[q][r]) : double(ac[q][r]);
       if (HL && !SEGR && grad) {
         clear();
-        list<K, KD, G, R, U, false>(ent, p0, p1, vr, nv, ulo, off, sd, ac, al);
+        list<K, KD, G, R, U, false, VL>(ent, p0, p1, vr, nv, ulo, off, sd, ac, al);
 #pragma unroll
         for (int q = 0; q < G; ++q)
 #pragma unroll
@@ -257,11 +256,11 @@ __device__ __forceinline__ void run(const SoloArgs& a, const SolveDesc& S, unsig
   };
 
   for (int i = tid; i < N; i += NT) {
-    const double yu = y[i];
+    const double yu = gld(y + i);
     x[i] = T(yu);
     if (wave) {
       if constexpr (HL) ulo[i] = T(yu - double(T(yu)));
-      vv[i] = T(y[N + i]);
+      vv[i] = T(gld(y + N + i));
     }
   }
   lds_barrier();
@@ -283,12 +282,12 @@ __device__ __forceinline__ void run(const SoloArgs& a, const SolveDesc& S, unsig
         const double s = total(i, !wave);
         if (wave) {
           const RkRegs qv = i == tid ? f1 : rk_load(stage, y, acc, int64_t(N) + i);
-          const double un = rk_stage(stage, dt, y, acc, i, qu, double(vv[i]));
+          const double un = rk_stage(stage, S, y, acc, i, qu, double(vv[i]));
           x[i] = T(un);
           if constexpr (HL) ulo[i] = T(un - double(T(un)));
-          vv[i] = T(rk_stage(stage, dt, y, acc, int64_t(N) + i, qv, s));
+          vv[i] = T(rk_stage(stage, S, y, acc, int64_t(N) + i, qv, s));
         } else {
-          x[i] = T(rk_stage(stage, dt, y, acc, i, qu, s));
+          x[i] = T(rk_stage(stage, S, y, acc, i, qu, s));
         }
       }
       lds_barrier();
