@@ -1038,7 +1038,7 @@ struct gsg_op {
   StepGraphs rkgraphs;  // the launches read dt and the state through the descriptor, so
                         // captured steps stay valid for every later call
   // csr
-  DevMem rp, ci, v64, v32;
+  DevMem rp, ci, v64, v32, blk;
   DevCsr csr{};
   // basis transform (kind GSG_OP_TRANSFORM) / the Vlasov right-hand side (GSG_OP_VLASOV)
   XForm xf;
@@ -1141,12 +1141,7 @@ static void op_apply_dev(gsg_op* op, const double* x, double* y, hipStream_t s) 
     return;
   }
   if (op->is_csr) {
-    const void* xin = x;
-    if (op->fp32) {
-      HIPC(launch_to_f32(x, op->x32.as<float>(), op->csr.n, s));
-      xin = op->x32.p;
-    }
-    HIPC(launch_csr(op->csr, op->fp32, xin, y, s));
+    HIPC(launch_csr(op->csr, op->fp32, x, y, s));
     return;
   }
   const Tables& T = *op->T;
@@ -1406,8 +1401,20 @@ int gsg_csc_create(int64_t m, int64_t n, const int64_t* colptr, const int64_t* r
       v32[v.size() + i] = float(v[i] - double(v32[i]));
     }
     upload(op->v32, v32);
-    if (op->fp32) op->x32.alloc(size_t(n) * 4);
-    op->csr = DevCsr{m, n, nnz, op->rp.as<int64_t>(), op->ci.as<int32_t>(), op->v64.as<double>(), op->v32.as<float>()};
+    // row blocks of k_csr: consecutive rows, at most 256 of them and CSR_ENT entries, or one row
+    std::vector<int32_t> blk{0};
+    for (int64_t i = 1; i <= m; ++i)
+      if (i == m || i - blk.back() == 256 || rp[i + 1] - rp[blk.back()] > CSR_ENT) blk.push_back(int32_t(i));
+    upload(op->blk, blk);
+    op->csr = DevCsr{m,
+                     n,
+                     nnz,
+                     op->rp.as<int64_t>(),
+                     op->ci.as<int32_t>(),
+                     op->v64.as<double>(),
+                     op->v32.as<float>(),
+                     op->blk.as<int32_t>(),
+                     int32_t(blk.size() - 1)};
     *out = op.release();
   });
 }

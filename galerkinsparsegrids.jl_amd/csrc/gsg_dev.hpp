@@ -329,6 +329,7 @@ hipError_t launch_solo(int D, int K, bool fp32, bool segr, const SoloArgs& a, in
 hipError_t launch_solo32(int D, int K, bool segr, const SoloArgs& a, int nsolve, int threads, int lds_bytes,
                          hipStream_t s);
 
+constexpr int CSR_ENT = 1024;  // entries of a row block: 4 a thread, 16 KiB of LDS
 // CSR SpMV y = A x (rows ascending columns), value/vector type per precision.
 struct DevCsr {
   int64_t m, n, nnz;
@@ -336,7 +337,9 @@ struct DevCsr {
   const int32_t* ci;
   const double* v64;
   const float* v32;  // 2 nnz: hi values, then lo values (v64 - hi)
+  const int32_t* blk;  // nblk + 1 first rows of the row blocks (csr_blocks)
+  int32_t nblk;
 };
-hipError_t launch_csr(const DevCsr& A, bool fp32, const void* x, void* y, hipStream_t s);
+hipError_t launch_csr(const DevCsr& A, bool fp32, const double* x, double* y, hipStream_t s);
 
 }  // namespace gsg
