@@ -1017,10 +1017,11 @@ struct gsg_op {
   bool fp32 = false;
   bool is_csr = false;
   int device = 0;
-  // every device launch of the handle runs on its own stream; ev_in / ev_out order that
-  // stream after the caller's stream and the caller's stream after it
+  // RK steps run on the handle's own stream, single applications on the caller's; ev_in
+  // orders the handle's stream after the caller's, ev_out (ev_cap under capture) marks the
+  // end of the last call
   hipStream_t stream = nullptr;
-  hipEvent_t ev_in = nullptr, ev_out = nullptr;
+  hipEvent_t ev_in = nullptr, ev_out = nullptr, ev_cap = nullptr;
   std::shared_ptr<Tables> T;
   int64_t N = 0, len = 0;
   // apply path
@@ -1109,18 +1110,53 @@ static void vlasov_rk_steps(gsg_op* op, double dt, int64_t n, hipStream_t s) {
   });
 }
 
+// Whether cs is being captured into a graph.  A captured call keeps to events of its own: one
+// recorded inside a capture must not be waited for outside, nor the other way round.
+static bool capturing(hipStream_t cs) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(cs, &st) != hipSuccess) {
+    (void)hipGetLastError();  // the null stream while another stream captures
+    return false;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
 // Runs fn(op->stream) ordered after the work already enqueued on the caller's stream cs
-// (NULL: the null stream) and before the work the caller enqueues on cs afterwards.  The
-// handle's scratch buffers and captured steps are only touched on op->stream, so calls
-// made on different caller streams are also ordered among themselves.
+// (NULL: the null stream) and before the work the caller enqueues on cs afterwards.  Every
+// call, this way or on the caller's stream (on_caller_stream), starts after ev_out, the end
+// of the call before it, so the handle's scratch buffers and captured steps are ordered
+// whatever streams the calls are made on.
 template <typename F>
 static void on_op_stream(gsg_op* op, void* cs, F&& fn) {
   hipStream_t c = static_cast<hipStream_t>(cs);
+  const bool cap = capturing(c);
+  hipEvent_t out = cap ? op->ev_cap : op->ev_out;
   HIPC(hipEventRecord(op->ev_in, c));
   HIPC(hipStreamWaitEvent(op->stream, op->ev_in, 0));
+  if (!cap) HIPC(hipStreamWaitEvent(op->stream, op->ev_out, 0));
   fn(op->stream);
-  HIPC(hipEventRecord(op->ev_out, op->stream));
+  HIPC(hipEventRecord(out, op->stream));
+  HIPC(hipStreamWaitEvent(c, out, 0));
+}
+// Runs fn on the caller's stream itself, after the handle's earlier calls.  For work without
+// stream capture of its own (one application): the hop to the handle's stream and back cost
+// more than a small operator (two event records, two waits on the host and two
+// cross-stream dependencies on the device).
+template <typename F>
+static void on_caller_stream(gsg_op* op, void* cs, F&& fn) {
+  hipStream_t c = static_cast<hipStream_t>(cs);
+  if (capturing(c)) {
+    on_op_stream(op, cs, fn);
+    return;
+  }
   HIPC(hipStreamWaitEvent(c, op->ev_out, 0));
+  fn(c);
+  HIPC(hipEventRecord(op->ev_out, c));
+}
+// The handle's stream after the device calls made so far (for the calls with host vectors,
+// which end with a synchronisation).
+static hipStream_t host_call_stream(gsg_op* op) {
+  HIPC(hipStreamWaitEvent(op->stream, op->ev_out, 0));
+  return op->stream;
 }
 
 static void op_common_init(gsg_op* op) {
@@ -1129,6 +1165,7 @@ static void op_common_init(gsg_op* op) {
   HIPC(hipStreamCreateWithFlags(&op->stream, hipStreamNonBlocking));
   HIPC(hipEventCreateWithFlags(&op->ev_in, hipEventDisableTiming));
   HIPC(hipEventCreateWithFlags(&op->ev_out, hipEventDisableTiming));
+  HIPC(hipEventCreateWithFlags(&op->ev_cap, hipEventDisableTiming));
 }
 
 static void op_apply_dev(gsg_op* op, const double* x, double* y, hipStream_t s) {
@@ -1593,7 +1630,7 @@ int gsg_op_apply_device(gsg_op* op, const double* x, double* y, int64_t len, voi
   return guarded([&] {
     require(op && x && y, "NULL argument");
     require(len == op->len, "len does not match the operator");
-    on_op_stream(op, stream, [&](hipStream_t s) { op_apply_dev(op, x, y, s); });
+    on_caller_stream(op, stream, [&](hipStream_t s) { op_apply_dev(op, x, y, s); });
   });
 }
 
@@ -1605,10 +1642,11 @@ int gsg_op_apply(gsg_op* op, const double* x, double* y, int64_t len) {
       op->xbuf.alloc(size_t(len) * 8);
       op->ybuf.alloc(size_t(len) * 8);
     }
-    HIPC(hipMemcpyAsync(op->xbuf.p, x, size_t(len) * 8, hipMemcpyHostToDevice, op->stream));
-    op_apply_dev(op, op->xbuf.as<double>(), op->ybuf.as<double>(), op->stream);
-    HIPC(hipMemcpyAsync(y, op->ybuf.p, size_t(len) * 8, hipMemcpyDeviceToHost, op->stream));
-    HIPC(hipStreamSynchronize(op->stream));
+    hipStream_t s = host_call_stream(op);
+    HIPC(hipMemcpyAsync(op->xbuf.p, x, size_t(len) * 8, hipMemcpyHostToDevice, s));
+    op_apply_dev(op, op->xbuf.as<double>(), op->ybuf.as<double>(), s);
+    HIPC(hipMemcpyAsync(y, op->ybuf.p, size_t(len) * 8, hipMemcpyDeviceToHost, s));
+    HIPC(hipStreamSynchronize(s));
   });
 }
 
@@ -1673,7 +1711,7 @@ int gsg_op_rk4(gsg_op* op, double* y, int64_t len, double t0, double dt, int64_t
     require(nsteps >= 0, "nsteps must be >= 0");
     if (op->d.kind == GSG_OP_VLASOV) {
       vlasov_rk_prepare(op, dt);
-      hipStream_t s = op->stream;
+      hipStream_t s = host_call_stream(op);
       HIPC(hipMemcpyAsync(op->vy.p, y, size_t(len) * 8, hipMemcpyHostToDevice, s));
       int64_t done = 0, snap = 0;
       while (done < nsteps) {
@@ -1692,7 +1730,7 @@ int gsg_op_rk4(gsg_op* op, double* y, int64_t len, double t0, double dt, int64_t
     }
     op_rk_prepare(op, dt);
     SolveState& S = *op->rk;
-    hipStream_t s = op->stream;
+    hipStream_t s = host_call_stream(op);
     HIPC(hipMemcpyAsync(S.y.p, y, size_t(len) * 8, hipMemcpyHostToDevice, s));
     if (!op->solo.on) S.to_stage0(s);
     int64_t done = 0, snap = 0;
@@ -1779,11 +1817,13 @@ int gsg_op_destroy(gsg_op* op) {
   return guarded([&] {
     if (op->stream) {
       (void)hipStreamSynchronize(op->stream);
+      if (op->ev_out) (void)hipEventSynchronize(op->ev_out);  // calls on the callers' streams
       {
         CaptureGuard cg(g_capture_mu);
         (void)hipStreamDestroy(op->stream);
         if (op->ev_in) (void)hipEventDestroy(op->ev_in);
         if (op->ev_out) (void)hipEventDestroy(op->ev_out);
+        if (op->ev_cap) (void)hipEventDestroy(op->ev_cap);
       }
     }
     delete op;
