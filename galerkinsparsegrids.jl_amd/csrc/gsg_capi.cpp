@@ -643,17 +643,20 @@ static void check_desc(const gsg_op_desc* d) {
 }
 
 // Multiplications of one operator application up to which a solve runs resident in one
-// workgroup.  Measured, us an RK4 step on the stage launches / resident (FP64, FP32):
-//   D = 2, k = 3, n = 5 (1,008 coefficients, 42e3)  transport 66 / 16.5, 42 / 17.4
-//                                                   wave 131 / 29.5, 127 / 41.8
-//   D = 3, k = 3, n = 3 (1,026, 37e3)               transport 28 / 13.5, 31 / 15.3
-//   D = 2, k = 4, n = 5 (1,792, 99e3)               transport 39 / 24, 42 / 27
-//   D = 2, k = 3, n = 6 (2,304, 104e3)              transport 82 / 29, 56 / 31
-// With the 1-D blocks left in global memory (they do not fit beside the vectors) it wins
-// only against the FP64 fiber kernel (D = 1, k = 5, n = 7: 465 / 25; FP32, plan kernel:
-// 45 / 55).
-constexpr int64_t SOLO_MACS = 120000;
-constexpr int64_t SOLO_MACS_FIBER = 250000;
+// workgroup.  Measured, us a transport step on the stage launches (directions split) /
+// resident, FP64 then FP32:
+//   D = 2, k = 3: n = 5 (1,008 coefficients, 42e3) 28 / 16.5, 29 / 17.4; n = 6 (2,304, 104e3)
+//   33 / 31, 37 / 32;  k = 2: n = 6 (1,024, 32e3) 30 / 14.4, 28 / 17; n = 7 (2,304, 74e3)
+//   32 / 35, 31 / 39
+//   D = 3: k = 2, n = 5 (2,176, 61e3) 28 / 25, 29 / 27; k = 4, n = 3 (2,432, 87e3) 23 / 26, 21 / 27
+//   D = 4: k = 3, n = 2 (1,539, 46e3) 23 / 12, 17 / 14; k = 2, n = 4 (3,072, 74e3) 26 / 26, 23 / 31
+// (wave systems gain more).  At D = 2 the lists are longer, and so are the stages.  With the
+// 1-D blocks left in global memory (they do not fit beside the vectors) it wins only in FP64 at
+// D = 1, where a stage is one long list: k = 5, n = 8 57 / 42, n = 9 57 / 72.
+static int64_t solo_macs(int D, int K, bool vals, bool fp32) {
+  if (!vals) return !fp32 && D == 1 ? 90000 : -1;
+  return D <= 2 && K >= 3 ? 105000 : 70000;
+}
 // RK4 stage launches of a set of solves of one (D, K) class.
 // How a grid's launches run: the kernel and, for the LDS fiber kernel, its LDS layout.
 struct LdsShape {
@@ -717,22 +720,35 @@ constexpr int64_t SEG64_MIN_CELLS = 65536;
 // 688 14.4 / 9.6, 9728 26.5 / 26.5.
 static int64_t dsplit_waves(int32_t kernel, int D, int K, bool fp32) {
   if (fp32 && (kernel == KERNEL_SEG || kernel == KERNEL_SEG_ALT)) return 8192;
+  if (kernel == KERNEL_PLAN) return D <= 6 && K <= 5 ? 8192 : -1;
   if (kernel != KERNEL_DIRECT) return -1;
   return fp32 ? 4096 : direct_ok(D, K) ? 24576 : 8192;
 }
+// The FP64 fiber kernel walks its tile's batches with barriers between them: it wins in
+// launches bound by throughput at D = 3 and on the coarse grids of D = 2, and loses where the
+// chain of batches is what is waited for.  Measured, us a stage on the plan / fiber kernel:
+// 3 M DoFs of copies: D = 3, k = 5, n = 5 206 / 126; D = 2, k = 3, n = 6 169 / 147, n = 9 186 /
+// 244; D = 1, k = 5, n = 9 254 / 1177; D = 5, k = 2, n = 6 137 / 202.  One solve (the plan
+// kernel with its directions split): D = 3, k = 5, n = 6 15.4 / 29.2; D = 2, k = 5, n = 9
+// 17.5 / 154; D = 6, k = 2, n = 5 10.8 / 12.8.
+constexpr int64_t FIBER_MIN_WAVES = 8192;
 // launch_waves: the wavefronts of every launch that runs beside this one
 static LdsShape lds_shape(const Tables& T, bool fp32, int64_t launch_cells, int64_t launch_waves) {
   LdsShape L = lds_shape(T, fp32);
-  if (!fp32 && L.kernel == KERNEL_SEG && launch_cells < SEG64_MIN_CELLS) return LdsShape{};
+  if (!fp32 && L.kernel == KERNEL_SEG && launch_cells < SEG64_MIN_CELLS) L = LdsShape{};
+  if (L.kernel == KERNEL_FIBER && !std::getenv("GSG_KERNEL") &&
+      (launch_waves <= FIBER_MIN_WAVES || T.D == 1 || T.D > 3 || (T.D == 2 && T.n > 6)))
+    L = LdsShape{};
   if (T.D > 1) L.dsplit = launch_waves <= dsplit_waves(L.kernel, T.D, T.k, fp32);
   return L;
 }
 static int64_t grid_cells(const Tables& T) { return T.lt.N / Tables::ipow_i(T.k, T.D); }
-// wavefronts of one solve of the grid on the single-cell kernels, one cell group each
+// wavefronts of one solve of the grid's launch without the direction split
 static int64_t grid_waves(const Tables& T, bool fp32) {
   const int32_t k = lds_shape(T, fp32).kernel;
-  const int64_t per = k == KERNEL_SEG || k == KERNEL_SEG_ALT ? seg_cpw(T.D, T.k) : 1;
-  return (grid_cells(T) + per - 1) / per;
+  if (k == KERNEL_DIRECT) return grid_cells(T);
+  if (fp32 && (k == KERNEL_SEG || k == KERNEL_SEG_ALT)) return (grid_cells(T) + seg_cpw(T.D, T.k) - 1) / seg_cpw(T.D, T.k);
+  return (T.lt.N + 63) / 64;
 }
 // tiles of a launch shape: tile-plan tiles for the fiber kernel, TILE-DoF tiles otherwise
 static const std::vector<Tile>& tiles_of(const Tables& T, const LdsShape& L) {
@@ -783,7 +799,7 @@ static SoloShape solo_shape(const Tables& T, const LdsShape& L, bool fp32, bool 
   const int64_t vb = int64_t(T.devp[0].val_elems) * 8;  // FP64, or the two float tables
   if (base > SOLO_LDS) return q;
   const int64_t macs = int64_t(ne) * Tables::ipow_i(T.k, T.D + 1);
-  if (base + vb <= SOLO_LDS ? macs > SOLO_MACS : L.kernel != KERNEL_FIBER || macs > SOLO_MACS_FIBER) return q;
+  if (macs > solo_macs(T.D, T.k, base + vb <= SOLO_LDS, fp32)) return q;
   q.on = true;
   q.segr = L.kernel == KERNEL_SEG || L.kernel == KERNEL_SEG_ALT;
   if (!fp32) q.segr = false;

@@ -324,6 +324,84 @@ __global__ __launch_bounds__(TILE) void k_plan(LaunchArgs a) {
   plan_body<DT, KT, T>(a, int(blockIdx.x));
 }
 
+// The plan kernel with one wavefront per direction: a workgroup owns a quarter of a tile (64
+// DoFs), wavefront d walks their lists of direction d, the direction sums meet in LDS and
+// are added in direction order (k_plan's sums bit for bit).  A small launch is as long as
+// its longest lists, which this cuts to one direction's.
+template <int DT, int KT, typename T>
+__global__ __launch_bounds__(64 * DT) void k_plan_ds(LaunchArgs a) {
+  constexpr int D = DT, K = KT;
+  constexpr int KD = ipow_c(K, D);
+  constexpr bool UNI = KD % 64 == 0;
+  __shared__ double P[D][64];
+  const Tile* tp = a.tiles + (blockIdx.x >> 2);
+  const int32_t solve = uni(sld(&tp->solve));
+  const SolveDesc& S = a.solves[solve];
+  const int64_t i0 = sld(&tp->start) + (blockIdx.x & 3) * 64;
+  const int64_t end = sld(&tp->end);
+  if (!sld(&S.active) || i0 >= end) return;  // the whole workgroup
+  const int lane = int(threadIdx.x) & 63;
+  const int d = uni(int(threadIdx.x) >> 6);
+  const bool real = i0 + lane < end;
+  const int64_t i = real ? i0 + lane : i0;
+  const int32_t g = UNI ? uni(int32_t(i0 / KD)) : int32_t(i / KD);
+  const int32_t ml = int32_t(i - int64_t(g) * KD);
+  const int64_t N = S.N;
+  int kd = 1;
+#pragma unroll
+  for (int e = 0; e + 1 < D; ++e) kd = e < d ? kd * K : kd;
+  const int md = (ml / kd) % K;
+  const uint32_t mb = uint32_t(ml - md * kd);
+  const bool rk = a.op == OP_RK_SUM || a.op == OP_RK_WAVE_SUM;
+  const bool wsum = a.op == OP_RK_WAVE_SUM || a.op == OP_APPLY_WAVE_SUM;
+  // the state of the entry this lane updates, in flight during the gathers
+  const int64_t idx = wsum && d == 1 ? N + i : i;
+  RkIn v{0.0, 0.0};
+  if (rk && d <= (wsum ? 1 : 0)) v = rk_pre(S, a.stage, idx);
+  double r = 0.0;
+  if (a.op == OP_APPLY_SUM || a.op == OP_RK_SUM) {
+    const T* x0 = a.op == OP_RK_SUM ? stage_in<T>(S, a.stage) : (const T*)a.xin;
+    const int64_t stride = a.op == OP_RK_SUM ? 0 : a.instride;
+    const int64_t elems = stride ? stride * S.ndir : N;
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(x0, uint32_t(elems * int64_t(sizeof(T))));
+    if (d >= S.dir0 && d < S.dir0 + S.ndir)
+      r = plan_dir<KT, T, UNI>(S, xr, uint32_t((d - S.dir0) * stride * int64_t(sizeof(T))), g, d, D, K, md, mb, kd);
+  } else if (a.op == OP_APPLY_GRAD || a.op == OP_RK_WAVE_GRAD) {
+    const T* x0 = a.op == OP_RK_WAVE_GRAD ? stage_in<T>(S, a.stage) : (const T*)a.xin;
+    T* w = a.op == OP_RK_WAVE_GRAD ? (T*)S.w : (T*)a.yout;
+    const int64_t lo = sizeof(T) == 4 ? (a.op == OP_RK_WAVE_GRAD ? 2 * N : a.split) : 0;
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(x0, uint32_t((lo ? lo + N : N) * int64_t(sizeof(T))));
+    r = plan_dir<KT, T, UNI>(S, xr, 0u, g, d, D, K, md, mb, kd);
+    if (lo) r += plan_dir<KT, T, UNI>(S, xr, uint32_t(lo * int64_t(sizeof(T))), g, d, D, K, md, mb, kd);
+    if (real) gst(w + int64_t(d) * N + i, T(r));
+    return;  // every wavefront: no barrier
+  } else {
+    const T* w = a.op == OP_RK_WAVE_SUM ? (const T*)S.w : (const T*)a.xin2;
+    const __amdgpu_buffer_rsrc_t wr = make_rsrc(w, uint32_t(int64_t(D) * N * int64_t(sizeof(T))));
+    r = plan_dir<KT, T, UNI>(S, wr, uint32_t(int64_t(d) * N * int64_t(sizeof(T))), g, d, D, K, md, mb, kd);
+  }
+  P[d][lane] = r;
+  __syncthreads();
+  if (d > (wsum ? 1 : 0) || !real) return;
+  if (wsum && d == 0) {  // u' = v
+    const T* x = a.op == OP_RK_WAVE_SUM ? stage_in<T>(S, a.stage) : (const T*)a.xin;
+    const double vn = double(gld(x + N + i));
+    if (rk)
+      rk_post<T>(S, a.stage, i, v, vn, 2 * N + i);
+    else
+      gst((double*)a.yout + i, vn);
+    return;
+  }
+  double s = 0.0;
+#pragma unroll
+  for (int e = 0; e < D; ++e)
+    if (wsum || (e >= S.dir0 && e < S.dir0 + S.ndir)) s = __builtin_fma(wsum ? 1.0 : S.coef[e], P[e][lane], s);
+  if (rk)
+    rk_post<T>(S, a.stage, idx, v, s);
+  else
+    gst((double*)a.yout + idx, s);
+}
+
 
 // ---------------------------------------------------------------------------------
 // LDS fiber kernel (fiber_ok shapes).  A workgroup owns fiber_cpt(D, K) consecutive
@@ -2342,6 +2420,16 @@ static hipError_t launch_tk(bool fp32, const LaunchArgs& a, hipStream_t s) {
     }
   }
   if (a.kernel != KERNEL_PLAN) return hipErrorInvalidValue;  // tile-plan tiles need the fiber kernel
+  if constexpr (DT >= 2 && KT > 0) {
+    if (a.dsplit) {
+      if (fp32)
+        hipLaunchKernelGGL((k_plan_ds<DT, KT, float>), dim3(unsigned(a.ntiles) * 4), dim3(64 * DT), 0, s, a);
+      else
+        hipLaunchKernelGGL((k_plan_ds<DT, KT, double>), dim3(unsigned(a.ntiles) * 4), dim3(64 * DT), 0, s, a);
+      return hipGetLastError();
+    }
+  }
+  if (a.dsplit) return hipErrorInvalidValue;  // no such instantiation
   if (fp32)
     hipLaunchKernelGGL((k_plan<DT, KT, float>), dim3(a.ntiles), dim3(TILE), 0, s, a);
   else
