@@ -574,7 +574,17 @@ struct SolveState {
   int kind = GSG_OP_TRANSPORT;
   bool fp32 = false;
   int64_t N = 0, len = 0;
-  DevMem y, acc, xs0, xs1, xs2, w;
+  // the vectors, each on 256 bytes, in one allocation: an allocation and its release cost
+  // tens of microseconds (and a device synchronisation) whatever their size
+  struct Span {
+    void* p = nullptr;
+    template <typename T>
+    T* as() const {
+      return static_cast<T*>(p);
+    }
+  };
+  DevMem mem;
+  Span y, acc, xs0, xs1, xs2, w;
   SolveDesc desc{};
 
   // entries of a stage-input buffer: the state length, plus u's rounding remainder in
@@ -596,7 +606,6 @@ struct SolveState {
   void to_stage0(hipStream_t s) {
     if (fp32) HIPC(launch_to_f32(y.as<double>(), xs0.as<float>(), len, s, kind == GSG_OP_WAVE ? N : 0));
   }
-  size_t bytes() const { return y.bytes + acc.bytes + xs0.bytes + xs1.bytes + xs2.bytes + w.bytes; }
 
   void init(std::shared_ptr<Tables> tab, const gsg_op_desc& d, bool f32) {
     T = std::move(tab);
@@ -606,12 +615,26 @@ struct SolveState {
     len = kind == GSG_OP_WAVE ? 2 * N : N;
     const size_t es = fp32 ? 4 : 8;
     const size_t xl = size_t(xs_len(kind, N, fp32));
-    y.alloc(len * 8);
-    acc.alloc(len * 8);
-    if (fp32) xs0.alloc(xl * es);
-    xs1.alloc(xl * es);
-    xs2.alloc(xl * es);
-    if (kind == GSG_OP_WAVE) w.alloc(size_t(T->D) * N * es);
+    size_t at = 0;
+    auto take = [&](Span& v, size_t bytes) {
+      v.p = reinterpret_cast<void*>(at);  // the offset until the allocation exists
+      at += (bytes + 255) / 256 * 256;
+    };
+    std::vector<Span*> all{&y, &acc, &xs1, &xs2};
+    take(y, size_t(len) * 8);
+    take(acc, size_t(len) * 8);
+    take(xs1, xl * es);
+    take(xs2, xl * es);
+    if (fp32) {
+      take(xs0, xl * es);
+      all.push_back(&xs0);
+    }
+    if (kind == GSG_OP_WAVE) {
+      take(w, size_t(T->D) * N * es);
+      all.push_back(&w);
+    }
+    mem.alloc(at);
+    for (Span* v : all) v->p = mem.as<unsigned char>() + reinterpret_cast<size_t>(v->p);
     std::memset(&desc, 0, sizeof(desc));
     desc.t = T->devp[fp32 ? 1 : 0];
     desc.D = T->D; desc.K = T->k; desc.n = T->n; desc.full = T->full;
@@ -2200,6 +2223,13 @@ struct Scheduler {
                    &descs[s].active, sizeof(int32_t), hipMemcpyHostToDevice));
   }
 
+  // the same, ordered on the batch's stream after the steps enqueued so far
+  void switch_off(size_t s) {
+    if (s >= descs.size() || !descs[s].active) return;
+    descs[s].active = 0;
+    HIPC(launch_switch_off(ddescs.as<SolveDesc>() + s, stream));
+  }
+
   hipEvent_t next_event() {
     if (evused == evpool.size()) {
       hipEvent_t e;
@@ -2347,7 +2377,8 @@ struct gsg_batch {
   std::vector<std::unique_ptr<BatchSolve>> solves;
   bool built = false;
   Scheduler sched;
-  std::vector<size_t> active;  // indices of solves in the current schedule
+  std::vector<size_t> active;     // indices of the unfinished solves
+  std::vector<size_t> scheduled;  // indices of the solves in the current schedule, in its order
 };
 
 static void batch_reschedule(gsg_batch* b) {
@@ -2358,6 +2389,7 @@ static void batch_reschedule(gsg_batch* b) {
       act.push_back(&b->solves[i]->st);
       b->active.push_back(i);
     }
+  b->scheduled = b->active;
   b->sched.build(act);
 }
 
@@ -2379,7 +2411,9 @@ static void batch_build(gsg_batch* b) {
 }
 
 // Advance all unfinished solves by up to `steps` steps, in phases so that no solve
-// overshoots its own step count.
+// overshoots its own step count.  A solve that finishes is switched off on the device, in
+// stream order; the batch is built anew (tiles, uploads, captured steps: milliseconds) only
+// when the solves that have finished since hold a quarter of its DoFs.
 static void batch_advance(gsg_batch* b, int64_t steps) {
   batch_build(b);
   while (steps > 0 && !b->active.empty()) {
@@ -2391,12 +2425,19 @@ static void batch_advance(gsg_batch* b, int64_t steps) {
       b->sched.collect();
     }
     steps -= phase;
-    bool finished = false;
-    for (size_t i : b->active) {
-      b->solves[i]->done += phase;
-      finished |= b->solves[i]->done >= b->solves[i]->nsteps;
+    int64_t built = 0, idle = 0;
+    for (size_t q = 0; q < b->scheduled.size(); ++q) {
+      BatchSolve& s = *b->solves[b->scheduled[q]];
+      if (s.done < s.nsteps) s.done += phase;
+      built += s.st.len;
+      if (s.done < s.nsteps) continue;
+      idle += s.st.len;
+      b->sched.switch_off(q);
     }
-    if (finished) {
+    b->active.erase(std::remove_if(b->active.begin(), b->active.end(),
+                                   [&](size_t i) { return b->solves[i]->done >= b->solves[i]->nsteps; }),
+                    b->active.end());
+    if (4 * idle > built && !b->active.empty()) {
       HIPC(hipStreamSynchronize(b->stream));
       batch_reschedule(b);
     }

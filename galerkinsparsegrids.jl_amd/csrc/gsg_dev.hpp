@@ -255,6 +255,8 @@ hipError_t launch_xsweep(int K, int nvec, const LaunchArgs& a, hipStream_t s, bo
 // *dst = v, written by a one-thread kernel (stream-ordered; the value travels as a kernel
 // argument, so the caller's copy may change as soon as this returns)
 hipError_t launch_write_desc(SolveDesc* dst, const SolveDesc& v, hipStream_t s);
+// d->active = 0, stream-ordered
+hipError_t launch_switch_off(SolveDesc* d, hipStream_t s);
 
 // y[i] = (float) x[i] for i < n, and the rounding remainders y[n + i] = (float)(x[i] -
 // y[i]) for i < nlo (the lo part of the wave system's u, read by its gradient pass)

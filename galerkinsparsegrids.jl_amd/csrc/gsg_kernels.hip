@@ -2326,6 +2326,10 @@ __global__ void k_write_desc(SolveDesc* dst, SolveDesc v) {
   if (threadIdx.x == 0) *dst = v;
 }
 
+__global__ void k_switch_off(SolveDesc* d) {
+  if (threadIdx.x == 0) gst(&d->active, 0);
+}
+
 __global__ void k_to_f32(const double* __restrict__ x, float* __restrict__ y, int64_t n, int64_t nlo) {
   for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
     const float h = float(x[i]);
@@ -2553,6 +2557,11 @@ hipError_t launch_fused(int pass, int stage, const FusedArgs& f, int grid, hipSt
 
 hipError_t launch_write_desc(SolveDesc* dst, const SolveDesc& v, hipStream_t s) {
   hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(64), 0, s, dst, v);
+  return hipGetLastError();
+}
+
+hipError_t launch_switch_off(SolveDesc* d, hipStream_t s) {
+  hipLaunchKernelGGL(k_switch_off, dim3(1), dim3(64), 0, s, d);
   return hipGetLastError();
 }
 
