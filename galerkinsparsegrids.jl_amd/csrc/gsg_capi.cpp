@@ -888,9 +888,9 @@ static bool graphs_enabled() {
 
 // Captured RK4 steps: a graph of CHUNK steps and one of a single step, replayed to cover
 // any step count (CHUNK steps per graph launch amortise the launch cost of small
-// grids).  With `lazy`, the first call after a reset runs eagerly and captures nothing,
-// so a launch set that is used once (a short-lived batch composition) pays no capture;
-// otherwise a call of at least 2 CHUNK steps captures at once.  The graphs hold kernel
+// grids).  The first call after a reset captures at once when it has at least `first_min`
+// steps and runs eagerly otherwise.  For a batch that is CHUNK steps: 17 classes on four
+// streams took 1.9 ms to capture and 0.83 ms a replayed step, 1.40 an eager one.  The graphs hold kernel
 // and event nodes only (no memset or copy nodes).
 struct StepGraphs {
   static constexpr int CHUNK = 8;
@@ -910,11 +910,11 @@ struct StepGraphs {
   ~StepGraphs() { reset(); }
   // run `n` steps on stream s; enqueue(k, stream) issues k steps eagerly
   template <typename F>
-  void run(int64_t n, hipStream_t s, bool lazy, F&& enqueue) {
+  void run(int64_t n, hipStream_t s, int64_t first_min, F&& enqueue) {
     if (n <= 0) return;
     const bool first = !used;
     used = true;
-    if (!graphs_enabled() || (first && (lazy || n < 2 * CHUNK))) {
+    if (!graphs_enabled() || (first && n < first_min)) {
       enqueue(n, s);
       return;
     }
@@ -1137,7 +1137,7 @@ static void vlasov_rk_steps(gsg_op* op, double dt, int64_t n, hipStream_t s) {
   // FP32: the stage update also writes the float copy of the next stage input (and of
   // the new state), so only the first stage of a run converts
   float* x32 = op->fp32 ? op->x32.as<float>() : nullptr;
-  op->vgraphs.run(n, s, false, [&](int64_t k, hipStream_t st) {
+  op->vgraphs.run(n, s, 2 * StepGraphs::CHUNK, [&](int64_t k, hipStream_t st) {
     for (int64_t i = 0; i < k; ++i)
       for (int stage = 1; stage <= 4; ++stage) {
         // the last n2m sweep applies the stage update (no right-hand-side vector)
@@ -1734,7 +1734,7 @@ static void op_rk_steps(gsg_op* op, int64_t nsteps, hipStream_t s) {
     launch_solo_steps(T.D, T.k, op->fp32, op->solo, op->d_rkdesc.as<SolveDesc>(), nullptr, 1, nsteps, s);
     return;
   }
-  op->rkgraphs.run(nsteps, s, false, [&](int64_t k, hipStream_t st) {
+  op->rkgraphs.run(nsteps, s, 2 * StepGraphs::CHUNK, [&](int64_t k, hipStream_t st) {
     for (int64_t i = 0; i < k; ++i)
       launch_rk_step(T.D, T.k, op->fp32, sys, op->d_rkdesc.as<SolveDesc>(), op->d_tiles.as<Tile>(), op->n_tiles,
                      op->shape, st);
@@ -2086,22 +2086,24 @@ struct Scheduler {
     for (SolveState* S : solves)
       if (!solo_of(*S).on) busy += stage_us(double(S->N), S->T->D, S->T->k, S->desc.sys);
     const bool solo_ok = busy <= SOLO_BATCH_US;
-    // cells per (D, k, system) class and wavefronts of all classes: a launch of too few cells
-    // runs the plan kernel (FP64, SEG64_MIN_CELLS), one of few wavefronts splits directions
-    std::map<std::tuple<int, int, int>, int64_t> seg_cells;
-    int64_t waves = 0;
+    // cells and wavefronts per (D, k, system) class: a launch of too few cells runs the plan
+    // kernel (FP64, SEG64_MIN_CELLS), one of few wavefronts splits directions (a class's own
+    // count, its launches follow each other whatever runs beside them, but doubled: what
+    // runs beside them fills the chip as well)
+    std::map<std::tuple<int, int, int>, std::pair<int64_t, int64_t>> launch_of;
+    const bool whole = fp32 && resolve_schedule(schedule_own) == GSG_SCHEDULE_FUSED;  // fused launches do not split
     for (SolveState* S : solves)
       if (!(solo_ok && solo_of(*S).on)) {
-        seg_cells[std::make_tuple(S->T->D, S->T->k, S->desc.sys)] += S->N / Tables::ipow_i(S->T->k, S->T->D);
-        waves += grid_waves(*S->T, fp32);
+        auto& q = launch_of[std::make_tuple(S->T->D, S->T->k, S->desc.sys)];
+        q.first += grid_cells(*S->T);
+        q.second += whole ? int64_t(1) << 40 : 2 * grid_waves(*S->T, fp32);
       }
-    if (fp32 && resolve_schedule(schedule_own) == GSG_SCHEDULE_FUSED) waves = int64_t(1) << 40;  // whole wavefronts per cell
     for (size_t s = 0; s < solves.size(); ++s) {
       SolveState& S = *solves[s];
       descs.push_back(S.desc);
       const auto ck = std::make_tuple(S.T->D, S.T->k, S.desc.sys);
       const SoloShape q = solo_ok ? solo_of(S) : SoloShape{};
-      const LdsShape L = q.on ? lds_shape(*S.T, fp32) : lds_shape(*S.T, fp32, seg_cells[ck], waves);
+      const LdsShape L = q.on ? lds_shape(*S.T, fp32) : lds_shape(*S.T, fp32, launch_of[ck].first, launch_of[ck].second);
       auto key = std::make_tuple(S.T->D, S.T->k, S.desc.sys, int(L.kernel), q.on ? 1 + int(q.vals) + 2 * int(q.small) : 0);
       auto it = gidx.find(key);
       if (it == gidx.end()) {
@@ -2299,7 +2301,7 @@ struct Scheduler {
     }
     if (groups.size() > 1 && lanes_enabled() && schedule != GSG_SCHEDULE_FUSED)
       init_lanes();  // no stream creation inside a capture
-    graphs.run(n, stream, true, [&](int64_t k, hipStream_t) { enqueue(k); });
+    graphs.run(n, stream, StepGraphs::CHUNK, [&](int64_t k, hipStream_t) { enqueue(k); });
   }
 
   void enqueue(int64_t n) {
