@@ -205,7 +205,6 @@ static std::vector<Tile> make_tiles(const Layout& lt, int solve) {
 // XCD has its own L2.  Interleave per-XCD tile lists so that bin x runs on XCD x; short
 // bins are padded with empty tiles that repeat a real tile with an empty range (so the
 // addresses a kernel reads before it sees the empty range stay valid).
-constexpr int NXCD = 8;
 // chunk: tiles per workgroup (the direct kernel runs DIRECT_CPW tiles per workgroup);
 // bin x's chunks go to workgroups x, x + 8, ...
 static std::vector<Tile> xcd_interleave(const std::vector<std::vector<Tile>>& bins, size_t chunk) {
@@ -946,86 +945,64 @@ struct StepGraphs {
 // along direction 0, then 1, ..., each sweep one k_xsweep launch over the grid (and over
 // several vectors at once).  FP64.  Per direction, cells whose entry list is long (the
 // coarse output cells of m2n / n2m couple to every finer nested cell) get a workgroup
-// each and go first; the other cells are cut into TILE-DoF ranges.
+// each and go first; the other cells' lists stand in a fixed-width table.  Where k^D is more
+// than half a workgroup no cell is split and the lanes walk the lists.
 struct XForm {
-  // entries above which a cell is split over a workgroup; measured on the 2 + 2
-  // dimensional Vlasov right-hand side (k = 2, n = 8): 8 beats 32 by 6%, 4 loses 14%
+  // entries above which a cell is split over a workgroup, us a sweep for 8 / 12 / 16 / 32 (a
+  // longer list takes further rounds from the list itself): m2n D = 4, k = 2, n = 8: 3.7 / 4.5 /
+  // 4.8 / 5.6; m2n D = 3, k = 3, n = 7: 3.6 / 4.0 / 4.5 / 5.8; n2p the same or faster at 8 too
   static constexpr int32_t LONG = 8;
   static_assert(LONG == XELL, "the fixed-width table holds every short list");
   std::shared_ptr<Tables> T;
-  DevMem descs;  // D SolveDescs, sweep d uses descs[d]
-  DevMem tiles;  // the D directions' tile lists, one after another
-  // k = 2 with long lists split over workgroups (so every short list has at most LONG
-  // entries): per direction, XELL (input cell offset, block) pairs a cell, the cell's list
-  // and then block -1 (long-list cells: all -1), so a lane reads its entries without
-  // waiting on the list bounds
-  DevMem ell;
-  int64_t ncell = 0;
-  std::vector<int32_t> toff, tcnt;
+  DevMem ell;    // the D directions' fixed-width tables (XDir::ell), one after another
+  DevMem heavy;  // the D directions' long-list cells
+  std::vector<XDir> dirs;
   void init(int D, int k, int n, int full, int tkind) {
     T = get_tables(D, k, n, full, tkind);
-    std::vector<SolveDesc> ds(static_cast<size_t>(D));
-    for (int d = 0; d < D; ++d) {
-      SolveDesc& a = ds[size_t(d)];
-      std::memset(&a, 0, sizeof(a));
-      a.t = T->devp[0];
-      a.D = D; a.K = k; a.n = n; a.full = full;
-      a.N = T->lt.N;
-      a.sys = SYS_SUM;
-      a.active = 1;
-      a.ndir = 1;
-      a.dir0 = d;
-      a.coef[d] = 1.0;
-    }
-    upload(descs, ds);
-    const int64_t KD = Tables::ipow_i(k, D);
-    ncell = T->lt.N / KD;
-    const std::vector<int32_t>& ptr = T->plan.ptr;
+    const DevTables& t = T->devp[0];
+    const int64_t KD = Tables::ipow_i(k, D), ncell = T->lt.N / KD;
+    const std::vector<int32_t>&ptr = T->plan.ptr, &ent = T->plan.ent;
     const int32_t maxparts = KD <= TILE / 2 ? int32_t(TILE / KD) : 1;
-    if (k == 2 && maxparts > 1) {
-      const std::vector<int32_t>& ent = T->plan.ent;
-      std::vector<int32_t> e(size_t(D) * size_t(ncell) * 2 * XELL);
-      for (int d = 0; d < D; ++d)
-        for (int64_t g = 0; g < ncell; ++g) {
-          const int32_t p0 = ptr[size_t(g * D + d)];
-          const int32_t len = ptr[size_t(g * D + d + 1)] - p0;
-          int32_t* row = e.data() + (size_t(d) * size_t(ncell) + size_t(g)) * 2 * XELL;
-          for (int u = 0; u < XELL; ++u) {
-            const bool in = len <= LONG && u < len;
-            row[2 * u] = in ? ent[size_t(2 * (p0 + u))] : 0;
-            row[2 * u + 1] = in ? ent[size_t(2 * (p0 + u) + 1)] : -1;
-          }
-        }
-      upload(ell, e);
-    }
-    std::vector<Tile> all;
+    std::vector<int32_t> e(maxparts > 1 ? size_t(D) * size_t(ncell) * 2 * XELL : 0);
+    std::vector<int4> all;
+    std::vector<size_t> hoff;
     for (int d = 0; d < D; ++d) {
-      std::vector<Tile> heavy, light;
-      int64_t run = -1;  // first DoF of the current run of short-list cells
-      auto flush = [&](int64_t stop) {
-        for (int64_t a0 = run; run >= 0 && a0 < stop; a0 += TILE)
-          light.push_back(Tile{0, 0, a0, std::min<int64_t>(a0 + TILE, stop), 1});
-        run = -1;
-      };
-      for (int64_t g = 0; g < ncell; ++g) {
-        const int32_t len = ptr[size_t(g * D + d + 1)] - ptr[size_t(g * D + d)];
-        if (maxparts > 1 && len > LONG) {
-          flush(g * KD);
-          const int32_t parts = std::min<int32_t>(maxparts, (len + 3) / 4);  // about 4 entries a lane
-          heavy.push_back(Tile{0, 0, g * KD, (g + 1) * KD, parts});
-        } else if (run < 0) {
-          run = g * KD;
+      std::vector<int4> hv;
+      for (int64_t g = 0; maxparts > 1 && g < ncell; ++g) {
+        const int32_t p0 = ptr[size_t(g * D + d)], p1 = ptr[size_t(g * D + d + 1)], len = p1 - p0;
+        int32_t* row = e.data() + (size_t(d) * size_t(ncell) + size_t(g)) * 2 * XELL;
+        for (int u = 0; u < XELL; ++u) {
+          const bool in = len <= LONG && u < len;
+          row[2 * u] = in ? ent[size_t(2 * (p0 + u))] : 0;
+          row[2 * u + 1] = in ? ent[size_t(2 * (p0 + u) + 1)] : len > LONG ? -2 : -1;
         }
+        if (len > LONG)  // about 4 entries a lane
+          hv.push_back(int4{int32_t(g), p0, p1, std::min<int32_t>(maxparts, (len + 3) / 4)});
       }
-      flush(ncell * KD);
-      while (heavy.size() % NXCD) heavy.push_back(Tile{0, 0, 0, 0, 2});  // keeps the XCD runs aligned
-      const std::vector<Tile> pl = xcd_split(light);
-      toff.push_back(int32_t(all.size()));
-      tcnt.push_back(int32_t(heavy.size() + pl.size()));
-      all.insert(all.end(), heavy.begin(), heavy.end());
-      all.insert(all.end(), pl.begin(), pl.end());
+      while (hv.size() % NXCD) hv.push_back(int4{0, 0, 0, 0});  // keeps the XCDs' eighths aligned
+      XDir x{};
+      x.N = uint32_t(T->lt.N);
+      x.D = D;
+      x.KD = uint32_t(KD);
+      x.kd = uint32_t(Tables::ipow_i(k, d));
+      x.mKD = uint32_t((uint64_t(1) << 32) / x.KD);
+      x.mkd = x.kd == 1 ? 0u : uint32_t(((uint64_t(1) << 32) + x.kd - 1) / x.kd);
+      x.nheavy = uint32_t(hv.size());
+      x.per = uint32_t(((T->lt.N + TILE - 1) / TILE + NXCD - 1) / NXCD);
+      x.vbytes = uint32_t(t.val_elems * int64_t(sizeof(double)));
+      x.val = t.val64;
+      x.ptr = t.plan_ptr + d;
+      x.ent = t.plan_ent;
+      hoff.push_back(all.size());
+      all.insert(all.end(), hv.begin(), hv.end());
+      dirs.push_back(x);
     }
-    upload(tiles, all);
+    if (!e.empty()) upload(ell, e);
+    if (!all.empty()) upload(heavy, all);
+    for (int d = 0; d < D; ++d) {
+      if (!e.empty()) dirs[size_t(d)].ell = ell.as<int32_t>() + size_t(d) * size_t(ncell) * 2 * XELL;
+      if (!all.empty()) dirs[size_t(d)].heavy = heavy.as<int4>() + hoff[size_t(d)];
+    }
   }
   // y = T x for nvec vectors of N elements stored one after another, with two scratch
   // areas of as many doubles vectors (all distinct from x and y).  x32: the inputs are
@@ -1037,15 +1014,8 @@ struct XForm {
     const void* cur = x;
     for (int d = 0; d < D; ++d) {
       double* next = d == D - 1 ? y : (d % 2 ? tb : ta);
-      LaunchArgs a{};
-      a.solves = descs.as<SolveDesc>() + d;
-      a.tiles = tiles.as<Tile>() + toff[size_t(d)];
-      a.ntiles = tcnt[size_t(d)];
-      a.xin = cur;
-      a.yout = next;
-      const int32_t* el = ell.p ? ell.as<int32_t>() + size_t(d) * size_t(ncell) * 2 * XELL : nullptr;
-      HIPC(launch_xsweep(T->k, nvec, a, s, x32 && d == 0, d == D - 1 ? comb : nullptr, d == D - 1 ? rk : nullptr,
-                         el));
+      HIPC(launch_xsweep(T->k, nvec, dirs[size_t(d)], cur, next, s, x32 && d == 0, d == D - 1 ? comb : nullptr,
+                         d == D - 1 ? rk : nullptr));
       cur = next;
     }
   }

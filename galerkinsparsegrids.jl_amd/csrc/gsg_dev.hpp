@@ -241,16 +241,33 @@ struct XRk {
   double* x;
   float* x32;
 };
-// entries a row of a sweep's fixed-width table (k = 2): the longest list a one-lane-per-DoF
-// tile takes
+// entries a row of a sweep's fixed-width table: the longest list a lane takes alone where a
+// cell can have a workgroup
 constexpr int XELL = 8;
+constexpr int NXCD = 8;  // workgroup b of a launch runs on XCD b % NXCD
+// One direction's sweep of a basis transform, passed by value: a lane goes from its block
+// index to its entries without loading a descriptor or a tile, and without a division.
+struct XDir {
+  uint32_t N;          // elements of a vector
+  uint32_t KD, kd;     // K^D, K^d
+  uint32_t mKD, mkd;   // floor(2^32 / KD), and ceil(2^32 / kd) (0 for kd = 1)
+  uint32_t nheavy;     // workgroups of the cells with long lists, a multiple of NXCD, first in the grid
+  uint32_t per;        // workgroups of TILE DoFs in an XCD's eighth of the grid
+  uint32_t vbytes;     // of val
+  const double* val;   // the 1-D blocks
+  const int32_t* ptr;  // the direction's list bounds: cell g's list is [ptr[D g], ptr[D g + 1])
+  const int32_t* ent;  // 2 per entry: input cell offset, block
+  // XELL (input cell offset, block) pairs a cell: the cell's list, then block -1; block -2
+  // first: a cell with a workgroup of its own.  Null: no cell has one.
+  const int32_t* ell;
+  const int4* heavy;   // a workgroup's cell, list bounds and lanes per DoF (0: padding)
+  int32_t D;
+};
 // one transform direction sweep over nvec vectors (k_xsweep; K in {2, 3, 5}); in_f32: the
 // inputs are float; comb: write the combination of the nvec results (one vector); rk: the
-// RK stage update instead of the result (one vector); ell (K = 2 only, or null): the sweep
-// direction's fixed-width table, XELL (input cell offset, block) pairs a cell, the cell's
-// list first and block -1 after it, for every cell whose list has at most XELL entries
-hipError_t launch_xsweep(int K, int nvec, const LaunchArgs& a, hipStream_t s, bool in_f32 = false,
-                         const XComb* comb = nullptr, const XRk* rk = nullptr, const int32_t* ell = nullptr);
+// RK stage update instead of the result (one vector)
+hipError_t launch_xsweep(int K, int nvec, const XDir& x, const void* xin, double* yout, hipStream_t s,
+                         bool in_f32 = false, const XComb* comb = nullptr, const XRk* rk = nullptr);
 
 // *dst = v, written by a one-thread kernel (stream-ordered; the value travels as a kernel
 // argument, so the caller's copy may change as soon as this returns)

@@ -2005,31 +2005,39 @@ static void launch_fused_pass(int stage, const FusedArgs& f, int grid, hipStream
 // loads its operands for the rest at offsets past the buffers' ends, which the hardware
 // answers with 0 and no memory access.  No branch separates the loads (a branch makes the
 // compiler wait on every load before the next).
+// k = 5 keeps to 4: 8 took 165 registers and n2p (D = 2, n = 9) 6.8 us a sweep against 6.6.
 template <int KT>
 constexpr int xround_len() {
-  return KT == 2 ? 8 : 4;
+  return KT == 5 ? XELL / 2 : XELL;
 }
 // the operands of entries (off[u], eb[u]), u < NR, applied to the NV vectors
 template <int KT, typename TX, int NV, int NR>
-__device__ __forceinline__ void xround_ops(const SolveDesc& S, __amdgpu_buffer_rsrc_t vr, const TX* xin, int64_t N,
+__device__ __forceinline__ void xround_ops(const XDir& S, __amdgpu_buffer_rsrc_t vr, const TX* xin,
                                            int v0, const uint32_t (&off)[xround_len<KT>()],
                                            const int32_t (&eb)[xround_len<KT>()], int nvalid, int md, uint32_t mb,
                                            int kd, double (&r)[NV]) {
   constexpr uint32_t es = sizeof(TX);
-  const uint32_t vend = uint32_t(S.t.val_elems * int64_t(sizeof(double)));
+  const uint32_t N = S.N, vend = S.vbytes;
   uint32_t xo[NR];
   double b[NR][KT];
 #pragma unroll
   for (int u = 0; u < NR; ++u) {
-    xo[u] = u < nvalid ? off[u] : uint32_t(N);  // N: past every vector's end
-    const uint32_t vo = uint32_t(((int64_t(eb[u]) * KT + md) * KT) * int64_t(sizeof(double)));
+    xo[u] = u < nvalid ? off[u] : N;  // N: past every vector's end
+    const uint32_t vo = uint32_t((eb[u] * KT + md) * KT) * uint32_t(sizeof(double));
+    // the row of KT doubles in loads of two
+    const uint32_t o = u < nvalid ? vo : vend;
 #pragma unroll
-    for (int mm = 0; mm < KT; ++mm)
-      b[u][mm] = buf_load<double>(vr, u < nvalid ? vo + uint32_t(mm * sizeof(double)) : vend, 0u);
+    for (int mm = 0; mm + 1 < KT; mm += 2) {
+      typedef double d2 __attribute__((ext_vector_type(2)));
+      const d2 q = __builtin_bit_cast(d2, __builtin_amdgcn_raw_buffer_load_b128(vr, int(o), mm * int(sizeof(double)), 0));
+      b[u][mm] = q.x;
+      b[u][mm + 1] = q.y;
+    }
+    if constexpr (KT % 2) b[u][KT - 1] = buf_load<double>(vr, o, uint32_t((KT - 1) * sizeof(double)));
   }
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const __amdgpu_buffer_rsrc_t xr = make_rsrc(xin + int64_t(v0 + v) * N, uint32_t(N * int64_t(es)));
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(xin + int64_t(v0 + v) * N, N * es);
     TX xv[NR][KT];
     if (KT == 2 && kd == 1) {
       // direction 0 at k = 2: a lane's two operands of an entry are adjacent, and aligned
@@ -2081,7 +2089,7 @@ __device__ __forceinline__ void xround_ops(const SolveDesc& S, __amdgpu_buffer_r
 }
 // entries p, p + stride, ... of the plan list (p itself inside the list), then their operands
 template <int KT, typename TX, int NV, int NR>
-__device__ __forceinline__ void xround(const SolveDesc& S, __amdgpu_buffer_rsrc_t vr, const TX* xin, int64_t N, int v0,
+__device__ __forceinline__ void xround(const XDir& S, __amdgpu_buffer_rsrc_t vr, const TX* xin, int v0,
                                        int32_t p, int32_t stride, int nvalid, int md, uint32_t mb, int kd,
                                        double (&r)[NV]) {
   constexpr int XR = xround_len<KT>();
@@ -2094,40 +2102,40 @@ __device__ __forceinline__ void xround(const SolveDesc& S, __amdgpu_buffer_rsrc_
     if (u < NR) {  // compile time
       const int32_t q = u < nvalid ? p + u * stride : p;
       // the (offset, block) pair as one 64-bit global load (little endian: offset low)
-      const uint64_t e = gld(reinterpret_cast<const uint64_t*>(S.t.plan_ent + 2 * q));
+      const uint64_t e = gld(reinterpret_cast<const uint64_t*>(S.ent + 2 * q));
       off[u] = uint32_t(e);
       eb[u] = int32_t(uint32_t(e >> 32));
     }
   }
-  xround_ops<KT, TX, NV, NR>(S, vr, xin, N, v0, off, eb, nvalid, md, mb, kd, r);
+  xround_ops<KT, TX, NV, NR>(S, vr, xin, v0, off, eb, nvalid, md, mb, kd, r);
 }
 // the round for nw = the wavefront's largest nvalid (1 <= nw <= NR), one straight-line
 // instantiation per length
 template <int KT, typename TX, int NV, int NR>
-__device__ __forceinline__ void xround_pick(int nw, const SolveDesc& S, __amdgpu_buffer_rsrc_t vr, const TX* xin,
-                                            int64_t N, int v0, int32_t p, int32_t stride, int nvalid, int md,
+__device__ __forceinline__ void xround_pick(int nw, const XDir& S, __amdgpu_buffer_rsrc_t vr, const TX* xin,
+                                            int v0, int32_t p, int32_t stride, int nvalid, int md,
                                             uint32_t mb, int kd, double (&r)[NV]) {
   if constexpr (NR > 1) {
     if (nw < NR) {
-      xround_pick<KT, TX, NV, NR - 1>(nw, S, vr, xin, N, v0, p, stride, nvalid, md, mb, kd, r);
+      xround_pick<KT, TX, NV, NR - 1>(nw, S, vr, xin, v0, p, stride, nvalid, md, mb, kd, r);
       return;
     }
   }
-  xround<KT, TX, NV, NR>(S, vr, xin, N, v0, p, stride, nvalid, md, mb, kd, r);
+  xround<KT, TX, NV, NR>(S, vr, xin, v0, p, stride, nvalid, md, mb, kd, r);
 }
 // the same for entries already in registers (a row of the fixed-width table)
 template <int KT, typename TX, int NV, int NR>
-__device__ __forceinline__ void xround_ops_pick(int nw, const SolveDesc& S, __amdgpu_buffer_rsrc_t vr, const TX* xin,
-                                                int64_t N, int v0, const uint32_t (&off)[xround_len<KT>()],
+__device__ __forceinline__ void xround_ops_pick(int nw, const XDir& S, __amdgpu_buffer_rsrc_t vr, const TX* xin,
+                                                int v0, const uint32_t (&off)[xround_len<KT>()],
                                                 const int32_t (&eb)[xround_len<KT>()], int nvalid, int md,
                                                 uint32_t mb, int kd, double (&r)[NV]) {
   if constexpr (NR > 1) {
     if (nw < NR) {
-      xround_ops_pick<KT, TX, NV, NR - 1>(nw, S, vr, xin, N, v0, off, eb, nvalid, md, mb, kd, r);
+      xround_ops_pick<KT, TX, NV, NR - 1>(nw, S, vr, xin, v0, off, eb, nvalid, md, mb, kd, r);
       return;
     }
   }
-  xround_ops<KT, TX, NV, NR>(S, vr, xin, N, v0, off, eb, nvalid, md, mb, kd, r);
+  xround_ops<KT, TX, NV, NR>(S, vr, xin, v0, off, eb, nvalid, md, mb, kd, r);
 }
 // the largest n over the wavefront's active lanes, for 1 <= n <= XR
 template <int XR>
@@ -2167,7 +2175,7 @@ __device__ __forceinline__ void rk_stage_at(const XRk& rk, int64_t i, RkIn in, d
 }
 
 // One direction sweep of a sparse-grid basis transform (the 1-D transform along
-// direction S.dir0, each row cut to its fiber's admissible levels), FP64 arithmetic on
+// one direction, each row cut to its fiber's admissible levels), FP64 arithmetic on
 // TX inputs (float: the FP32 derivative output read directly), over vectors of S.N
 // elements stored one after another.  NC = 0: vectors v0 .. v0 + NL - 1, v0 = NL blockIdx.y,
 // go from xin + v N to yout + v N, each lane running the NL vectors on the entries it
@@ -2175,35 +2183,28 @@ __device__ __forceinline__ void rk_stage_at(const XRk& rk, int64_t i, RkIn in, d
 // right-hand side, cb.nv = NC vectors): every lane runs the NC vectors for its DoF on the
 // entries it loaded once, and writes only their combination
 // -sum_{v<Dx} vpt_v y_v + sum_{v>=Dx} F_{v-Dx} y_v (the pointwise products of the
-// steprule: -(sum_d v_d P_d) + (sum_d F_d Q_d), each sum in d order).  A tile with
-// aux <= 1 is a DoF range, one lane per DoF.  A tile with aux = P > 1 is one cell with a
-// long entry list (a coarse cell coupled to every finer nested cell): P lanes per DoF take
-// every P-th entry and the partial sums are added in a fixed order through LDS.  ell (k = 2,
-// when every short list of the sweep has at most XELL entries): the sweep direction's
-// fixed-width table, XELL (offset, block) pairs a cell, the cell's list first and block -1
-// after it, which the one-lane-per-DoF tiles read in place of the list bounds and entries.
+// steprule: -(sum_d v_d P_d) + (sum_d F_d Q_d), each sum in d order).  The first S.nheavy
+// workgroups are one cell with a long list each (a coarse cell coupled to every finer
+// nested cell): P lanes per DoF take every P-th entry and the partial sums are added in a
+// fixed order through LDS.  The others are TILE DoFs each, one lane per DoF, with the entries
+// from the fixed-width table; the lanes of a cell with a workgroup of its own leave at once.
+// A sweep is a chain of dependent loads in few wavefronts (the smallest launch takes 2.0 us),
+// so the chain is kept short: what a descriptor and a tile held travels as a kernel argument,
+// quotients are multiplications, the table needs no list bounds, and a row of a 1-D block
+// comes in loads of two values.  us a sweep before and after (m2n, n2p, p2n, n2m): D = 4, k = 2,
+// n = 8: 4.7 4.7 3.7 5.8 / 3.7 3.6 3.1 4.8; D = 3, k = 3, n = 7: 4.5 4.4 3.5 6.7 / 3.6 3.3
+// 2.9 5.4.  The long lists bound n2m (D = 2, k = 5, n = 9, 512 entries: 21 / 18.5).
 template <int KT, typename TX, int NC, int NL = 1>
-__global__ __launch_bounds__(TILE) void k_xsweep(LaunchArgs a, XComb cb, XRk rk, const int32_t* ell) {
+__global__ __launch_bounds__(TILE) void k_xsweep(XDir S, const void* xv, double* yout, XComb cb, XRk rk) {
   static_assert(NC == 0 || NL == 1, "a combination sweep runs its NC vectors");
   constexpr int NV = NC ? NC : NL;  // vectors a lane sums
   constexpr int XR = xround_len<KT>();
   __shared__ double part[NV * TILE];
-  const Tile* tp = a.tiles + blockIdx.x;
-  const SolveDesc& S = a.solves[0];
-  const int D = S.D;
-  const int d = S.dir0;
-  int KD = 1, kd = 1;
-  for (int e = 0; e < D; ++e) {
-    if (e < d) kd *= KT;
-    KD *= KT;
-  }
   const int64_t N = S.N;
-  const int64_t start = sld(&tp->start);
-  const int64_t end = sld(&tp->end);
-  const int parts = int(sld(&tp->aux));
+  const uint32_t KD = S.KD, kd = S.kd;
   const int v0 = NC ? 0 : NL * int(blockIdx.y);
-  const TX* xin = (const TX*)a.xin;
-  const __amdgpu_buffer_rsrc_t vr = make_rsrc(S.t.val64, uint32_t(S.t.val_elems * int64_t(sizeof(double))));
+  const TX* xin = (const TX*)xv;
+  const __amdgpu_buffer_rsrc_t vr = make_rsrc(S.val, S.vbytes);
   // the results at DoF i: the combination of the NC vectors' sums (each sum in vector
   // order, the pointwise factors loaded with the sums' operands), the RK stage update,
   // or the sum itself
@@ -2218,12 +2219,12 @@ __global__ __launch_bounds__(TILE) void k_xsweep(LaunchArgs a, XComb cb, XRk rk,
         else
           c2 = v == cb.Dx ? t : c2 + t;
       }
-      gst((double*)a.yout + i, cb.F ? -c1 + c2 : -c1);
+      gst(yout + i, cb.F ? -c1 + c2 : -c1);
     } else if (rk.stage) {
       rk_stage_at(rk, i, in, r[0]);
     } else {
 #pragma unroll
-      for (int v = 0; v < NV; ++v) gst((double*)a.yout + int64_t(v0 + v) * N + i, r[v]);
+      for (int v = 0; v < NV; ++v) gst(yout + int64_t(v0 + v) * N + i, r[v]);
     }
   };
   auto pointwise = [&](int64_t i, double (&w)[NV]) {
@@ -2235,62 +2236,89 @@ __global__ __launch_bounds__(TILE) void k_xsweep(LaunchArgs a, XComb cb, XRk rk,
         w[v] = 0.0;
     }
   };
-  if (parts <= 1) {
-    const int64_t i = start + threadIdx.x;
-    if (i >= end) return;
-    const int32_t g = int32_t(i / KD);
-    const int ml = int(i - int64_t(g) * KD);
-    const int md = (ml / kd) % KT;
-    const uint32_t mb = uint32_t(ml - md * kd);
-    double w[NV];
-    pointwise(i, w);
-    const RkIn in = rk.stage ? rk_stage_in(rk.stage, i, rk.y, rk.acc) : RkIn{0.0, 0.0};
-    double r[NV];
+  if (blockIdx.x >= S.nheavy) {
+    const uint32_t j = blockIdx.x - S.nheavy;  // XCD j % NXCD: its own eighth of the grid
+    const uint32_t i = ((j % NXCD) * S.per + j / NXCD) * TILE + threadIdx.x;
+    if (i >= S.N) return;
+    // the quotients by multiplication: of i one short at most, of ml exact (ml < 2^14)
+    uint32_t g, ml;
+    int md;
+    if constexpr (KT == 2) {
+      ml = i & (KD - 1);
+      g = i >> S.D;
+      md = (ml & kd) ? 1 : 0;
+    } else {
+      g = __umulhi(i, S.mKD);
+      ml = i - g * KD;
+      if (ml >= KD) {
+        ml -= KD;
+        ++g;
+      }
+      md = int((kd == 1 ? ml : __umulhi(ml, S.mkd)) % KT);
+    }
+    const uint32_t mb = ml - uint32_t(md) * kd;
+    double w[NV], r[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) r[v] = 0.0;
-    if constexpr (XR == XELL) {
-      if (ell) {
-        // the cell's row of the direction's fixed-width table (its list, then block -1):
-        // the entries load without waiting on the list bounds
-        typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-        const __attribute__((address_space(1))) u4* row =
-            (const __attribute__((address_space(1))) u4*)(ell + int64_t(g) * (2 * XELL));
-        uint32_t off[XR];
-        int32_t eb[XR];
-        int nvalid = 0;
+    if (S.ell) {
+      // the cell's row of the fixed-width table: the entries load without waiting on the
+      // list bounds
+      typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+      const __attribute__((address_space(1))) u4* row =
+          (const __attribute__((address_space(1))) u4*)(S.ell + int64_t(g) * (2 * XELL));
+      uint32_t off[XELL];
+      int32_t eb[XELL];
+      int len = 0;
 #pragma unroll
-        for (int j = 0; j < XR / 2; ++j) {
-          const u4 q = row[j];
-          off[2 * j] = q.x;
-          eb[2 * j] = int32_t(q.y);
-          off[2 * j + 1] = q.z;
-          eb[2 * j + 1] = int32_t(q.w);
-        }
-#pragma unroll
-        for (int u = 0; u < XR; ++u) nvalid += eb[u] >= 0 ? 1 : 0;
-        xround_ops_pick<KT, TX, NV, XR>(wave_max_count<XR>(nvalid), S, vr, xin, N, v0, off, eb, nvalid, md, mb, kd,
-                                        r);
-        finish(i, r, w, in);
-        return;
+      for (int q = 0; q < XELL / 2; ++q) {
+        const u4 e = row[q];
+        off[2 * q] = e.x;
+        eb[2 * q] = int32_t(e.y);
+        off[2 * q + 1] = e.z;
+        eb[2 * q + 1] = int32_t(e.w);
       }
+      pointwise(i, w);
+      const RkIn in = rk.stage ? rk_stage_in(rk.stage, i, rk.y, rk.acc) : RkIn{0.0, 0.0};
+      if (eb[0] == -2) return;  // the whole cell
+#pragma unroll
+      for (int u = 0; u < XELL; ++u) len += eb[u] >= 0 ? 1 : 0;
+      const int most = wave_max_count<XELL>(len);
+#pragma unroll
+      for (int q = 0; q < XELL; q += XR) {
+        if (q >= most) break;
+        uint32_t o[XR];
+        int32_t b[XR];
+#pragma unroll
+        for (int u = 0; u < XR; ++u) {
+          o[u] = off[q + u];
+          b[u] = eb[q + u];
+        }
+        const int left = most - q < XR ? most - q : XR, mine = len - q < 0 ? 0 : len - q < XR ? len - q : XR;
+        xround_ops_pick<KT, TX, NV, XR>(left, S, vr, xin, v0, o, b, mine, md, mb, int(kd), r);
+      }
+      finish(i, r, w, in);
+      return;
     }
-    const int32_t* ptr = S.t.plan_ptr + int64_t(g) * D + d;
+    pointwise(i, w);
+    const RkIn in = rk.stage ? rk_stage_in(rk.stage, i, rk.y, rk.acc) : RkIn{0.0, 0.0};
+    const int32_t* ptr = S.ptr + int64_t(g) * S.D;
     const int32_t p0 = gld(ptr), p1 = gld(ptr + 1);
     for (int32_t pb = p0; pb < p1; pb += XR) {
       const int nvalid = p1 - pb < XR ? int(p1 - pb) : XR;
-      xround_pick<KT, TX, NV, XR>(wave_max_count<XR>(nvalid), S, vr, xin, N, v0, pb, 1, nvalid, md, mb, kd, r);
+      xround_pick<KT, TX, NV, XR>(wave_max_count<XR>(nvalid), S, vr, xin, v0, pb, 1, nvalid, md, mb, int(kd), r);
     }
     finish(i, r, w, in);
     return;
   }
-  if (end <= start) return;  // padding tile: the whole workgroup leaves before the barrier
-  const int t = threadIdx.x;
-  const int dof = t % KD;
-  const int pp = t / KD;
-  const int32_t g = int32_t(start / KD);
-  const int md = (dof / kd) % KT;
-  const uint32_t mb = uint32_t(dof - md * kd);
-  const int32_t* ptr = S.t.plan_ptr + int64_t(g) * D + d;
+  const int4* hp = S.heavy + blockIdx.x;
+  const int32_t p0 = sld(&hp->y), p1 = sld(&hp->z), parts = sld(&hp->w);
+  if (parts == 0) return;  // padding: the whole workgroup leaves before the barrier
+  const int64_t start = int64_t(sld(&hp->x)) * KD;
+  const uint32_t t = threadIdx.x;
+  const uint32_t pp = (t * (65536u / KD + 1)) >> 16;  // t / KD: exact for t < 256, KD <= 128
+  const uint32_t dof = t - pp * KD;
+  const int md = int((kd == 1 ? dof : __umulhi(dof, S.mkd)) % KT);
+  const uint32_t mb = dof - uint32_t(md) * kd;
   double r[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) r[v] = 0.0;
@@ -2300,12 +2328,11 @@ __global__ __launch_bounds__(TILE) void k_xsweep(LaunchArgs a, XComb cb, XRk rk,
     pointwise(start + dof, w);
     if (rk.stage) in = rk_stage_in(rk.stage, start + dof, rk.y, rk.acc);
   }
-  if (pp < parts) {
-    const int32_t p0 = gld(ptr), p1 = gld(ptr + 1);
-    for (int32_t pb = p0 + pp; pb < p1; pb += XR * parts) {
+  if (int(pp) < parts) {
+    for (int32_t pb = p0 + int(pp); pb < p1; pb += XR * parts) {
       const int32_t left = (p1 - pb + parts - 1) / parts;  // entries of this lane from pb on
       const int nvalid = left < XR ? int(left) : XR;
-      xround_pick<KT, TX, NV, XR>(wave_max_count<XR>(nvalid), S, vr, xin, N, v0, pb, parts, nvalid, md, mb, kd, r);
+      xround_pick<KT, TX, NV, XR>(wave_max_count<XR>(nvalid), S, vr, xin, v0, pb, parts, nvalid, md, mb, int(kd), r);
     }
   }
 #pragma unroll
@@ -2492,22 +2519,21 @@ static dim3 vec_grid(int64_t n) {
   return dim3(unsigned(blocks < 65536 ? blocks : 65536));
 }
 template <typename TX, int NC, int NL = 1>
-static hipError_t launch_xsweep_t(int K, int nvec, const LaunchArgs& a, const XComb& cb, const XRk& rk,
-                                  const int32_t* ell, hipStream_t s) {
-  const dim3 grid(unsigned(a.ntiles), unsigned(NC ? 1 : nvec / NL));
+static hipError_t launch_xsweep_t(int K, int nvec, const XDir& x, const void* xin, double* y, const XComb& cb,
+                                  const XRk& rk, hipStream_t s) {
+  const dim3 grid(unsigned(x.nheavy + NXCD * x.per), unsigned(NC ? 1 : nvec / NL));
   switch (K) {
-    case 2: hipLaunchKernelGGL((k_xsweep<2, TX, NC, NL>), grid, dim3(TILE), 0, s, a, cb, rk, ell); break;
-    case 3: hipLaunchKernelGGL((k_xsweep<3, TX, NC, NL>), grid, dim3(TILE), 0, s, a, cb, rk, nullptr); break;
-    case 5: hipLaunchKernelGGL((k_xsweep<5, TX, NC, NL>), grid, dim3(TILE), 0, s, a, cb, rk, nullptr); break;
+    case 2: hipLaunchKernelGGL((k_xsweep<2, TX, NC, NL>), grid, dim3(TILE), 0, s, x, xin, y, cb, rk); break;
+    case 3: hipLaunchKernelGGL((k_xsweep<3, TX, NC, NL>), grid, dim3(TILE), 0, s, x, xin, y, cb, rk); break;
+    case 5: hipLaunchKernelGGL((k_xsweep<5, TX, NC, NL>), grid, dim3(TILE), 0, s, x, xin, y, cb, rk); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
-hipError_t launch_xsweep(int K, int nvec, const LaunchArgs& a, hipStream_t s, bool in_f32, const XComb* comb,
-                         const XRk* rk, const int32_t* ell) {
-  static_assert(xround_len<2>() == XELL, "a row of the fixed-width table is one round");
-  if (a.ntiles <= 0 || nvec <= 0) return hipSuccess;
-  if (ell && K != 2) return hipErrorInvalidValue;  // the table exists for k = 2 only
+hipError_t launch_xsweep(int K, int nvec, const XDir& x, const void* xin, double* y, hipStream_t s, bool in_f32,
+                         const XComb* comb, const XRk* rk) {
+  if (x.N == 0 || nvec <= 0) return hipSuccess;
+  if (x.nheavy && (!x.ell || x.KD > TILE / 2)) return hipErrorInvalidValue;
   const XComb none{nullptr, nullptr, 0, 1};
   const XRk nork{0, 0.0, 0.0, nullptr, nullptr, nullptr, nullptr};
   if (rk && rk->stage && (comb || nvec != 1)) return hipErrorInvalidValue;  // one plain vector only
@@ -2516,21 +2542,21 @@ hipError_t launch_xsweep(int K, int nvec, const LaunchArgs& a, hipStream_t s, bo
     // the combination reads FP64 sweep results of Dx or 2 Dx vectors (Dx <= 4)
     if (comb->nv != nvec || in_f32) return hipErrorInvalidValue;
     switch (nvec) {
-      case 1: return launch_xsweep_t<double, 1>(K, nvec, a, *comb, r, ell, s);
-      case 2: return launch_xsweep_t<double, 2>(K, nvec, a, *comb, r, ell, s);
-      case 3: return launch_xsweep_t<double, 3>(K, nvec, a, *comb, r, ell, s);
-      case 4: return launch_xsweep_t<double, 4>(K, nvec, a, *comb, r, ell, s);
-      case 6: return launch_xsweep_t<double, 6>(K, nvec, a, *comb, r, ell, s);
-      case 8: return launch_xsweep_t<double, 8>(K, nvec, a, *comb, r, ell, s);
+      case 1: return launch_xsweep_t<double, 1>(K, nvec, x, xin, y, *comb, r, s);
+      case 2: return launch_xsweep_t<double, 2>(K, nvec, x, xin, y, *comb, r, s);
+      case 3: return launch_xsweep_t<double, 3>(K, nvec, x, xin, y, *comb, r, s);
+      case 4: return launch_xsweep_t<double, 4>(K, nvec, x, xin, y, *comb, r, s);
+      case 6: return launch_xsweep_t<double, 6>(K, nvec, x, xin, y, *comb, r, s);
+      case 8: return launch_xsweep_t<double, 8>(K, nvec, x, xin, y, *comb, r, s);
       default: return hipErrorInvalidValue;
     }
   }
   if (nvec % 2 == 0) {  // vector pairs: a lane runs both on the entries it loaded once
-    return in_f32 ? launch_xsweep_t<float, 0, 2>(K, nvec, a, none, r, ell, s)
-                  : launch_xsweep_t<double, 0, 2>(K, nvec, a, none, r, ell, s);
+    return in_f32 ? launch_xsweep_t<float, 0, 2>(K, nvec, x, xin, y, none, r, s)
+                  : launch_xsweep_t<double, 0, 2>(K, nvec, x, xin, y, none, r, s);
   }
-  return in_f32 ? launch_xsweep_t<float, 0>(K, nvec, a, none, r, ell, s)
-                : launch_xsweep_t<double, 0>(K, nvec, a, none, r, ell, s);
+  return in_f32 ? launch_xsweep_t<float, 0>(K, nvec, x, xin, y, none, r, s)
+                : launch_xsweep_t<double, 0>(K, nvec, x, xin, y, none, r, s);
 }
 
 hipError_t launch_fused(int pass, int stage, const FusedArgs& f, int grid, hipStream_t s) {
