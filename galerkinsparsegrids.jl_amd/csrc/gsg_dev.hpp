@@ -171,6 +171,7 @@ struct LaunchArgs {
   const void* xin2;  // APPLY_WAVE_SUM: the gradient buffer
   void* yout;
   int64_t instride;
+  int32_t gdirs;       // OP_APPLY_GRAD: only directions 0 .. gdirs - 1 are wanted (0: all)
   int64_t split;       // float OP_APPLY_GRAD: element offset of the input's lo part (0: none)
   int32_t lds_bytes;   // > 0: tiles are tile-plan tiles, run the LDS kernel with this LDS
   int32_t lds_xelems;  // LDS elements reserved for input cells (then the per-direction

@@ -286,6 +286,7 @@ __device__ __forceinline__ void plan_body(const LaunchArgs& a, int wg) {
 #pragma unroll
     for (int d = 0; d < DM; ++d) {
       if (d >= D) break;
+      if (a.op == OP_APPLY_GRAD && a.gdirs && d >= a.gdirs) break;
       const int md = (ml / kd) % K;
       const uint32_t mb = uint32_t(ml - md * kd);
       double r = plan_dir<KT, T, UNI>(S, xr, 0u, g, d, D, K, md, mb, kd);
@@ -371,6 +372,7 @@ __global__ __launch_bounds__(64 * DT) void k_plan_ds(LaunchArgs a) {
     T* w = a.op == OP_RK_WAVE_GRAD ? (T*)S.w : (T*)a.yout;
     const int64_t lo = sizeof(T) == 4 ? (a.op == OP_RK_WAVE_GRAD ? 2 * N : a.split) : 0;
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(x0, uint32_t((lo ? lo + N : N) * int64_t(sizeof(T))));
+    if (a.op == OP_APPLY_GRAD && a.gdirs && d >= a.gdirs) return;
     r = plan_dir<KT, T, UNI>(S, xr, 0u, g, d, D, K, md, mb, kd);
     if (lo) r += plan_dir<KT, T, UNI>(S, xr, uint32_t(lo * int64_t(sizeof(T))), g, d, D, K, md, mb, kd);
     if (real) gst(w + int64_t(d) * N + i, T(r));
@@ -959,6 +961,9 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
 #pragma unroll
   for (int dd = 0; dd < (DS ? 1 : D); ++dd) {
     const int d = DS ? wave : dd;
+    if constexpr (OPT == OP_APPLY_GRAD) {
+      if (a.gdirs && d >= a.gdirs) break;  // wave-uniform
+    }
     const int sd = ipow_rt(K, d);
     const bool fib = lane < F;
     const int fc = fib ? lane : 0;
@@ -1410,6 +1415,9 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
 #pragma unroll
   for (int dd = 0; dd < (DS ? 1 : D); ++dd) {
     const int d = DS ? wave : dd;  // the lists' index is dd
+    if constexpr (OPT == OP_APPLY_GRAD) {
+      if (a.gdirs && d >= a.gdirs) break;  // wave-uniform
+    }
     if constexpr (OPT == OP_APPLY_GRAD && !DS) {
       if (dsel >= 0 && d != dsel) {  // wave-uniform
         if (d < dsel) fetch(ewc, d + 1 < D ? d + 1 : d, 0);  // the next direction's first entries
@@ -1648,7 +1656,7 @@ static void launch_seg_op(const LaunchArgs& a, hipStream_t s) {
   // without the split, the gradient of a grid of fewer than 1024 workgroups (4 per CU)
   // runs one direction per grid row: measured on the 2 + 2 dimensional Vlasov derivative
   // (k = 2, n = 8)
-  const dim3 ggrid(grid.x, OPT == OP_APPLY_GRAD && grid.x < 1024 ? unsigned(DT) : 1u);
+  const dim3 ggrid(grid.x, OPT == OP_APPLY_GRAD && grid.x < 1024 ? unsigned(a.gdirs ? a.gdirs : DT) : 1u);
   if (a.dsplit)
     hipLaunchKernelGGL((k_seg_ds<DT, KT, OPT, STG>), dim3(unsigned(a.ntiles / seg_cpw(DT, KT))), dim3(64 * DT), 0, s, a);
   else
@@ -1785,6 +1793,9 @@ __device__ __forceinline__ void seg64_body(const LaunchArgs& a, int wg, unsigned
   int2 ewc = fetch(0, 0);
 #pragma unroll
   for (int d = 0; d < D; ++d) {
+    if constexpr (OPT == OP_APPLY_GRAD) {
+      if (a.gdirs && d >= a.gdirs) break;  // wave-uniform
+    }
     const int sd = ipow_rt(K, d);
     const int fc = fib ? fl : 0;
     const int vbd = fc % sd + (fc / sd) * sd * K;  // the fiber's element with digit d = 0

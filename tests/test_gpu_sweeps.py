@@ -24,3 +24,15 @@ def test_sweeps_match_the_assembled_matrix(g, gpu, D, k, n):
         op = g.transform(D, k, n, a, b)
         assert rel(op @ x, g.transform_csc(D, k, n, a, b) @ x) < 1e-12, (a, b)
         op.close()
+
+
+@pytest.mark.parametrize("Dx,k,n,prec", [(1, 2, 9, "fp32"), (1, 5, 5, "fp64"), (2, 2, 3, "fp32"), (2, 2, 9, "fp32"),
+                                         (2, 2, 9, "fp64"), (2, 3, 5, "fp32"), (2, 3, 6, "fp64"), (2, 5, 2, "fp64"),
+                                         (3, 2, 5, "fp32")])
+def test_without_a_force_only_space_is_differentiated(g, gpu, Dx, k, n, prec):
+    """The velocity derivatives are left out exactly where a zero force multiplies them."""
+    print(f"[gpu] vlasov Dx={Dx} k={k} n={n} {prec}", flush=True)
+    N = g.get_size(2 * Dx, k, n)
+    x = np.random.default_rng([Dx, k, n]).standard_normal(N)
+    free, zero = (g.vlasov_operator(Dx, k, n, F, precision=prec) for F in (None, [np.zeros(N)] * Dx))
+    np.testing.assert_array_equal(free @ x, zero @ x)
