@@ -748,32 +748,34 @@ struct SolveView {
     return (T*)(stage == 2 ? xs2 : xs1);
   }
   // rk for the two consecutive state entries idx, idx + 1 (idx even: 16-byte aligned)
-  // with their derivatives r0, r1, through 16-byte global accesses
-  __device__ __forceinline__ void rk2(int stage, int64_t idx, double r0, double r1) const {
-    typedef double d2 __attribute__((ext_vector_type(2)));
-    typedef T t2 __attribute__((ext_vector_type(2)));
-    typedef __attribute__((address_space(1))) d2 gd2;
-    typedef __attribute__((address_space(1))) t2 gt2;
+  // with their derivatives r0, r1, through 16-byte global accesses (lo even or negative)
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  typedef T t2 __attribute__((ext_vector_type(2)));
+  typedef __attribute__((address_space(1))) d2 gd2;
+  typedef __attribute__((address_space(1))) t2 gt2;
+  __device__ __forceinline__ static void put2(T* o, int64_t idx, int64_t lo, d2 x) {
+    const t2 h = {T(x.x), T(x.y)};
+    *(gt2*)(o + idx) = h;
+    if (sizeof(T) == 4 && lo >= 0) *(gt2*)(o + lo) = t2{T(x.x - double(h.x)), T(x.y - double(h.y))};
+  }
+  __device__ __forceinline__ void rk2(int stage, int64_t idx, double r0, double r1, int64_t lo = -1) const {
     const d2 r = {r0, r1};
     const d2 yi = stage <= 3 ? *(const gd2*)(y + idx) : d2{0.0, 0.0};
     const d2 ai = stage >= 2 ? *(const gd2*)(acc + idx) : d2{0.0, 0.0};
     T* o = out(stage);
     if (stage == 1) {
       *(gd2*)(acc + idx) = yi + dt6 * r;
-      const d2 x = yi + dt2 * r;
-      *(gt2*)(o + idx) = t2{T(x.x), T(x.y)};
+      put2(o, idx, lo, yi + dt2 * r);
     } else if (stage == 2) {
       *(gd2*)(acc + idx) = ai + dt3 * r;
-      const d2 x = yi + dt2 * r;
-      *(gt2*)(o + idx) = t2{T(x.x), T(x.y)};
+      put2(o, idx, lo, yi + dt2 * r);
     } else if (stage == 3) {
       *(gd2*)(acc + idx) = ai + dt3 * r;
-      const d2 x = yi + dt * r;
-      *(gt2*)(o + idx) = t2{T(x.x), T(x.y)};
+      put2(o, idx, lo, yi + dt * r);
     } else {
       const d2 yn = ai + dt6 * r;
       *(gd2*)(y + idx) = yn;
-      if (o) *(gt2*)(o + idx) = t2{T(yn.x), T(yn.y)};
+      if (o) put2(o, idx, lo, yn);
     }
   }
   // the next stage input at o[idx], and in float with lo >= 0 its rounding remainder at o[lo]
@@ -1135,23 +1137,42 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
-  if constexpr (OPT == OP_RK_SUM && FULL) {
-    // RK epilogue: lane l owns outputs 2l, 2l + 1 and 128 + 2l, 129 + 2l, so each
-    // 16-byte (2-double) access instruction covers 1 KiB contiguous across the wavefront
+  if constexpr (FULL) {
+    // lane l owns outputs 2l, 2l + 1 and 128 + 2l, 129 + 2l, so each 16-byte (2-double)
+    // access instruction covers 1 KiB contiguous across the wavefront.  The wave's second
+    // pass with outputs 4l .. 4l + 3 in 8-byte accesses took 94 us against 45 (n = 8, FP32)
+    using V2 = SolveView<T, D>;
+    typedef typename V2::d2 d2;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int m = h * 128 + 2 * lane;
-      V.rk2(STG, start + m, double(Y[m]), double(Y[m + 1]));
+      const int64_t i = start + m;
+      const double s0 = double(Y[m]), s1 = double(Y[m + 1]);
+      if constexpr (OPT == OP_RK_SUM) {
+        V.rk2(STG, i, s0, s1);
+      } else if constexpr (OPT == OP_RK_WAVE_SUM) {
+        const typename V2::t2 vN = *(const typename V2::gt2*)(V.in(STG) + N + i);
+        V.rk2(STG, i, double(vN.x), double(vN.y), 2 * N + i);
+        V.rk2(STG, N + i, s0, s1);
+      } else if constexpr (OPT == OP_APPLY_SUM) {
+        gst((double*)a.yout + i, s0);
+        gst((double*)a.yout + i + 1, s1);
+      } else {
+        const T* x = (const T*)a.xin;
+        gst((double*)a.yout + i, double(gld(x + N + i)));
+        gst((double*)a.yout + i + 1, double(gld(x + N + i + 1)));
+        gst((double*)a.yout + N + i, s0);
+        gst((double*)a.yout + N + i + 1, s1);
+      }
     }
     return;
   }
-  // epilogue: lane l owns the 4 consecutive outputs 4l .. 4l + 3 (smaller cells: outputs
-  // l and 64 + l of the k^D)
-  constexpr int NT = FULL ? 4 : (KD + 63) / 64;
+  // smaller cells: lane l owns outputs l and 64 + l of the k^D
+  constexpr int NT = (KD + 63) / 64;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const int m = FULL ? 4 * lane + t : 64 * t + lane;
-    if (!FULL && m >= KD) break;
+    const int m = 64 * t + lane;
+    if (m >= KD) break;
     const int64_t i = start + m;
     const T sum = Y[m];
     if constexpr (OPT == OP_APPLY_SUM) {
