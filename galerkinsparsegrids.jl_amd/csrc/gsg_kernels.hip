@@ -835,6 +835,14 @@ struct SolveView {
 #ifndef GSG_DSPLIT64_EB
 #define GSG_DSPLIT64_EB 1
 #endif
+// the operations whose float input has a rounding remainder that runs as a second part, in a
+// loop of its own: one loop with a branch around each product stopped the products from
+// being scheduled together (us a launch of the wave system, mean of both passes: D = 3, k = 4,
+// n = 8 19.4 / 15.4, n = 10 40.7 / 35.4; D = 4, k = 3, n = 9 61.6 / 57.7)
+template <typename T>
+constexpr bool parts_ok(int op) {
+  return sizeof(T) == 4 && (op == OP_RK_WAVE_GRAD || op == OP_APPLY_GRAD);
+}
 template <typename T, bool DS = false>
 constexpr int direct_eb() {
   return DS ? (sizeof(T) == 4 ? GSG_DSPLIT_EB : GSG_DSPLIT64_EB) : sizeof(T) == 4 ? DIRECT_EB : GSG_DIRECT64_EB;
@@ -932,7 +940,7 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
   int64_t lo = 0;
   if constexpr (MF && OPT == OP_RK_WAVE_GRAD) lo = 2 * N;
   if constexpr (MF && OPT == OP_APPLY_GRAD) lo = a.split;
-  const int npart = lo ? 2 : 1;
+  constexpr int NPART = parts_ok<T>(OPT) ? 2 : 1;
   const int64_t xelems = dstride ? dstride * D : (lo ? lo + N : N);
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(x0, uint32_t(xelems * int64_t(es)) & vmask);
   const __amdgpu_buffer_rsrc_t vr = make_rsrc(V.vals, uint32_t(V.val_elems * (MF ? 2 : 1) * int64_t(es)) & vmask);
@@ -977,7 +985,9 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
     v4f accv = {0.f, 0.f, 0.f, 0.f}, accl = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int q = 0; q < K; ++q) acc[q] = T(0);
-    for (int part = 0; part < npart; ++part)
+#pragma unroll
+    for (int part = 0; part < NPART; ++part) {  // a loop of its own for each part
+    if (part && !lo) break;
     for (int c0 = p0; c0 < p1; c0 += EB) {
       const int nb = p1 - c0;
       const uint32_t pbase = xbase + (part ? uint32_t(lo * int64_t(es)) : 0u);
@@ -1029,7 +1039,7 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
       }
       // next round's entry words (this direction's next round, its first again for the
       // second part, or the next direction's first), in flight during this round's math
-      const int nx = c0 + EB < p1 ? c0 + EB : (part + 1 < npart ? p0 : p1);
+      const int nx = c0 + EB < p1 ? c0 + EB : (part + 1 < NPART && lo ? p0 : p1);
 #pragma unroll
       for (int q = 0; q < 2 * EB; ++q) ew[q] = uni(sld(ep + 2 * nx + q));
       __builtin_amdgcn_s_waitcnt(0);  // the DMA into LDS (and everything else) has landed
@@ -1059,6 +1069,7 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
             for (int j = 0; j < K; ++j) acc[r] += (SB ? bs[u][r * K + j] : lane_bcast(bl[u], r * K + j)) * xv[j];
         }
       }
+    }
     }
     p0 = p1;
     if constexpr (MF) {
@@ -1325,7 +1336,7 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
   int64_t lo = 0;
   if constexpr (OPT == OP_RK_WAVE_GRAD) lo = 2 * N;
   if constexpr (OPT == OP_APPLY_GRAD) lo = a.split;
-  const int npart = lo ? 2 : 1;
+  constexpr int NPART = parts_ok<T>(OPT) ? 2 : 1;
   const int64_t xelems = dstride ? dstride * D : (lo ? lo + N : N);
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(x0, uint32_t(xelems * 4) & vmask);
   // the padded hi blocks, then the padded lo blocks
@@ -1452,7 +1463,9 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
     const int nr = nrd[dd];
     const uint32_t xbase = uint32_t(int64_t(d) * dstride * 4);
     v4f accv = {0.f, 0.f, 0.f, 0.f}, accl = {0.f, 0.f, 0.f, 0.f};
-    for (int part = 0; part < npart; ++part)
+#pragma unroll
+    for (int part = 0; part < NPART; ++part) {  // a loop of its own for each part
+    if (part && !lo) break;
     for (int c0 = 0; c0 < nr; c0 += EB) {
       const uint32_t pbase = xbase + (part ? uint32_t(lo * 4) : 0u);
       v4f bv[EB], bvl[EB];
@@ -1506,7 +1519,7 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
       // direction's first), in flight with this round's loads
       if (c0 + EB < nr)
         fetch(ewn, dd, c0 + EB);
-      else if (part + 1 < npart)
+      else if (part + 1 < NPART && lo)
         fetch(ewn, dd, 0);  // the direction's first entries again, for the second part
       else if (!DS && d + 1 < D)
         fetch(ewn, d + 1 < ND ? d + 1 : 0, 0);
@@ -1549,6 +1562,7 @@ __device__ __forceinline__ void seg_body(const LaunchArgs& a, int wg, int dsel, 
       for (int u = 0; u < EB; ++u) ewc[u] = ewn[u];
       // the next round's DMA rewrites the slots only after these reads (the MFMAs above
       // consumed them)
+    }
     }
     if (!DS && nr == 0 && d + 1 < D) fetch(ewc, d + 1 < ND ? d + 1 : 0, 0);  // no round ran
     // the hi and lo sums and the coefficient in double
