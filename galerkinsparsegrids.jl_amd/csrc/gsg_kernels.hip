@@ -989,7 +989,13 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
     for (int part = 0; part < NPART; ++part) {  // a loop of its own for each part
     if (part && !lo) break;
     for (int c0 = p0; c0 < p1; c0 += EB) {
-      const int nb = p1 - c0;
+#pragma unroll
+    for (int ne = EB; ne > (MF ? 0 : EB - 1); --ne) {
+      // MF: straight-line code for a round of ne entries: 85 instructions for ne = 4 against 145
+      // with a branch around each DMA and a mask on each operand.  D = 4, k = 4, us a stage:
+      // n = 7 16.7 / 16.0, n = 8 29.5 / 28.2, n = 9 62.5 / 60.0
+      if (MF && (ne == EB ? p1 - c0 < EB : p1 - c0 != ne)) continue;
+      const int nb = MF ? ne : p1 - c0;
       const uint32_t pbase = xbase + (part ? uint32_t(lo * int64_t(es)) : 0u);
       T bl[EB];
       T bs[SB ? EB : 1][SB ? KK : 1];
@@ -1045,9 +1051,9 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
       __builtin_amdgcn_s_waitcnt(0);  // the DMA into LDS (and everything else) has landed
       const v4s_t bwb = bf16x4(bw[0], bw[1], bw[2], bw[3]);  // MF: the block row as bf16 (lo correction)
 #pragma unroll
-      for (int u = 0; u < EB; ++u) {
-        // unused slots hold stale (or never written) data: read them anyway, branch-free,
-        // and clear the bits (a stale NaN times a zero block would still be NaN)
+      for (int u = 0; u < (MF ? ne : EB); ++u) {
+        // (MF: always in.)  Unused slots hold stale (or never written) data: read them anyway,
+        // branch-free, and clear the bits (a stale NaN times a zero block would still be NaN)
         const bool in = u < nb;
         const T* xs = Xs[wave][u] + sh[u] + vbd;
         T xv[K];
@@ -1069,6 +1075,7 @@ __device__ __forceinline__ void direct_body(const LaunchArgs& a, int wg, unsigne
             for (int j = 0; j < K; ++j) acc[r] += (SB ? bs[u][r * K + j] : lane_bcast(bl[u], r * K + j)) * xv[j];
         }
       }
+    }
     }
     }
     p0 = p1;
