@@ -123,8 +123,7 @@ struct SolveDesc {
   int32_t dir0;     // first direction in SUM mode
   int32_t pad;
   double coef[MAXD];
-  // the step and its fractions of the RK stages, divided on the host: a division in every
-  // lane's epilogue cost more than the epilogue's memory accesses
+  // the step and its fractions of the RK stages, divided once on the host
   double dt, dt2, dt3, dt6;
   void set_dt(double h) {
     dt = h;

@@ -1255,10 +1255,12 @@ constexpr int seg_lds_bytes(int D, int K) { return seg_lds_bytes(D, K, seg_eb(D,
 // With DS (one wavefront per direction) wg is the workgroup's one group of seg_cpw cells
 // and lds holds seg_split_lds_bytes(D, K) bytes: D wavefronts' input slots, then the D
 // directions' results in double.
-#ifndef GSG_SSPLIT_EB
-#define GSG_SSPLIT_EB seg_eb(D, K)
-#endif
-constexpr int seg_split_eb(int D, int K) { return GSG_SSPLIT_EB; }
+// Entries a round with DS: a small launch waits for its longest chain of rounds, so the
+// 4-lane shapes (D = 2, and D = 3 with k = 2) take 4 where the large launches take 2 (registers).
+// us a stage with 2 / 4 / 8: D = 2, k = 3, n = 9 13.4 / 11.2 / 10.8; D = 2, k = 4, n = 14 49.5 /
+// 46.2 / 53.6; D = 3, k = 2, n = 8 11.1 / 9.6 / 8.5, n = 11 21.8 / 20.7 / 23.9.  The other
+// shapes keep seg_eb (8: D = 3, k = 3, n = 7 8.6 / 8.4, n = 9 13.8 / 16.2).
+constexpr int seg_split_eb(int D, int K) { return seg_lanes(D, K) == 4 ? 4 : seg_eb(D, K); }
 constexpr int seg_split_lds_bytes(int D, int K) {
   return 1024 * D * seg_split_eb(D, K) + 8 * D * seg_cpw(D, K) * kpow(K, D);
 }
