@@ -131,7 +131,11 @@ int gsg_points_1d(int32_t k, int32_t n, double *x, int64_t len);
  * kernel (grids with D <= 6, k <= 5, k^D <= 256 and D k^(D-1) <= 256) and the
  * scalar-plan gather kernel (every grid).  gsg_tune_set records which one runs for a
  * grid and precision; GSG_KERNEL_AUTO restores the built-in rule.  Takes effect for
- * operators, batches and servers created afterwards.  Thread-safe. */
+ * operators, batches and servers created afterwards.  Thread-safe.  The choice is between
+ * the kernels of one launch a stage: RK4 solves small enough for one compute unit run
+ * resident in a workgroup, with the same sums, unless the environment's GSG_KERNEL asks
+ * for a stage kernel, and a small launch takes its kernel's form with a wavefront per
+ * direction (TILE_ALT: the rule's round there). */
 #define GSG_KERNEL_AUTO 0
 #define GSG_KERNEL_PLAN 1
 #define GSG_KERNEL_TILE 2
