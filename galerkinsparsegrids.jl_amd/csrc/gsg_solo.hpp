@@ -293,6 +293,18 @@ __device__ __forceinline__ void run(const SoloArgs& a, const SolveDesc& S, unsig
       lds_barrier();
     }
   }
+  // float: the stage launches read a step's first stage input from xs[0] (FP64: from y), so
+  // it is left there as their last stage leaves it, for a solve that goes on in stage launches
+  if constexpr (HL) {
+    T* const x0 = static_cast<T*>(S.xs[0]);
+    for (int i = tid; i < N; i += NT) {
+      gst(x0 + i, x[i]);
+      if (wave) {
+        gst(x0 + N + i, vv[i]);
+        gst(x0 + 2 * N + i, ulo[i]);
+      }
+    }
+  }
 }
 
 template <int D, int K, typename T, bool SEGR>
