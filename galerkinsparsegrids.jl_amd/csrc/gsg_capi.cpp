@@ -985,8 +985,8 @@ struct XForm {
       x.D = D;
       x.KD = uint32_t(KD);
       x.kd = uint32_t(Tables::ipow_i(k, d));
-      x.mKD = uint32_t((uint64_t(1) << 32) / x.KD);
-      x.mkd = x.kd == 1 ? 0u : uint32_t(((uint64_t(1) << 32) + x.kd - 1) / x.kd);
+      x.qKD = quot_mul(x.KD);
+      x.qkd = quot_mul(x.kd);
       x.nheavy = uint32_t(hv.size());
       x.per = uint32_t(((T->lt.N + TILE - 1) / TILE + NXCD - 1) / NXCD);
       x.vbytes = uint32_t(t.val_elems * int64_t(sizeof(double)));

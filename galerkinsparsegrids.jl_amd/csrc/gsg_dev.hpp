@@ -8,6 +8,8 @@
 
 #include <cstdint>
 
+#include "gsg_index.hpp"
+
 namespace gsg {
 
 // loads and stores through the global address space (the pointers are device
@@ -250,7 +252,7 @@ constexpr int NXCD = 8;  // workgroup b of a launch runs on XCD b % NXCD
 struct XDir {
   uint32_t N;          // elements of a vector
   uint32_t KD, kd;     // K^D, K^d
-  uint32_t mKD, mkd;   // floor(2^32 / KD), and ceil(2^32 / kd) (0 for kd = 1)
+  QuotMul qKD, qkd;    // division by KD, and by kd (not by kd = 1)
   uint32_t nheavy;     // workgroups of the cells with long lists, a multiple of NXCD, first in the grid
   uint32_t per;        // workgroups of TILE DoFs in an XCD's eighth of the grid
   uint32_t vbytes;     // of val

@@ -2295,7 +2295,7 @@ __global__ __launch_bounds__(TILE) void k_xsweep(XDir S, const void* xv, double*
     const uint32_t j = blockIdx.x - S.nheavy;  // XCD j % NXCD: its own eighth of the grid
     const uint32_t i = ((j % NXCD) * S.per + j / NXCD) * TILE + threadIdx.x;
     if (i >= S.N) return;
-    // the quotients by multiplication: of i one short at most, of ml exact (ml < 2^14)
+    // the quotients by multiplication (i < N < 2^31, ml < K^D)
     uint32_t g, ml;
     int md;
     if constexpr (KT == 2) {
@@ -2303,13 +2303,9 @@ __global__ __launch_bounds__(TILE) void k_xsweep(XDir S, const void* xv, double*
       g = i >> S.D;
       md = (ml & kd) ? 1 : 0;
     } else {
-      g = __umulhi(i, S.mKD);
+      g = quot(i, S.qKD);
       ml = i - g * KD;
-      if (ml >= KD) {
-        ml -= KD;
-        ++g;
-      }
-      md = int((kd == 1 ? ml : __umulhi(ml, S.mkd)) % KT);
+      md = int((kd == 1 ? ml : quot(ml, S.qkd)) % KT);
     }
     const uint32_t mb = ml - uint32_t(md) * kd;
     double w[NV], r[NV];
@@ -2370,9 +2366,9 @@ __global__ __launch_bounds__(TILE) void k_xsweep(XDir S, const void* xv, double*
   if (parts == 0) return;  // padding: the whole workgroup leaves before the barrier
   const int64_t start = int64_t(sld(&hp->x)) * KD;
   const uint32_t t = threadIdx.x;
-  const uint32_t pp = (t * (65536u / KD + 1)) >> 16;  // t / KD: exact for t < 256, KD <= 128
+  const uint32_t pp = quot(t, S.qKD);
   const uint32_t dof = t - pp * KD;
-  const int md = int((kd == 1 ? dof : __umulhi(dof, S.mkd)) % KT);
+  const int md = int((kd == 1 ? dof : quot(dof, S.qkd)) % KT);
   const uint32_t mb = dof - uint32_t(md) * kd;
   double r[NV];
 #pragma unroll
