@@ -1190,7 +1190,13 @@ static void op_apply_dev(gsg_op* op, const double* x, double* y, hipStream_t s) 
     return;
   }
   if (op->is_csr) {
-    HIPC(launch_csr(op->csr, op->fp32, x, y, s));
+    // FP32, y over x: through the float copy, as every other FP32 operator goes
+    float* x32 = nullptr;
+    if (op->fp32 && x < y + op->len && y < x + op->len) {
+      x32 = op->x32.as<float>();
+      HIPC(launch_to_f32(x, x32, op->len, s));
+    }
+    HIPC(launch_csr(op->csr, op->fp32, x, y, s, x32));
     return;
   }
   const Tables& T = *op->T;
@@ -1450,6 +1456,7 @@ int gsg_csc_create(int64_t m, int64_t n, const int64_t* colptr, const int64_t* r
       v32[v.size() + i] = float(v[i] - double(v32[i]));
     }
     upload(op->v32, v32);
+    if (op->fp32) op->x32.alloc(size_t(n) * 4);
     // row blocks of k_csr: consecutive rows, at most 256 of them and CSR_ENT entries, or one row
     std::vector<int32_t> blk{0};
     for (int64_t i = 1; i <= m; ++i)

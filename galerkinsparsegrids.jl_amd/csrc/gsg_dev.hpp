@@ -361,6 +361,8 @@ struct DevCsr {
   const int32_t* blk;  // nblk + 1 first rows of the row blocks (csr_blocks)
   int32_t nblk;
 };
-hipError_t launch_csr(const DevCsr& A, bool fp32, const double* x, double* y, hipStream_t s);
+// x32 (float only): the rounded vector, read in place of x
+hipError_t launch_csr(const DevCsr& A, bool fp32, const double* x, double* y, hipStream_t s,
+                      const float* x32 = nullptr);
 
 }  // namespace gsg

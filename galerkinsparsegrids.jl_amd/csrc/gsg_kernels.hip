@@ -2428,8 +2428,8 @@ __global__ void k_to_f64(const float* __restrict__ x, double* __restrict__ y, in
 // is read.  What bounded the thread per row was its own stride: 64 rows' entries a load
 // instruction, 64 cache lines.  Measured on the gradient of D = 3, k = 3, n = 6 (18,576 rows,
 // 0.93 M entries): 41.5 us before, 6.9 now; 3,000 rows with two dense ones: 365 / 55 us.
-template <typename T>
-__global__ __launch_bounds__(256) void k_csr(DevCsr A, const double* __restrict__ x, double* __restrict__ y) {
+template <typename T, typename TX>
+__global__ __launch_bounds__(256) void k_csr(DevCsr A, const TX* __restrict__ x, double* __restrict__ y) {
   constexpr bool HL = sizeof(T) == 4;
   __shared__ T sv[CSR_ENT], sl[HL ? CSR_ENT : 1], sx[CSR_ENT];
   const T* v = vals_of_csr<T>(A);
@@ -2820,12 +2820,14 @@ hipError_t launch_proj_pass(const ProjArgs& a, const double* wv, int d, int64_t 
   return hipGetLastError();
 }
 
-hipError_t launch_csr(const DevCsr& A, bool fp32, const double* x, double* y, hipStream_t s) {
+hipError_t launch_csr(const DevCsr& A, bool fp32, const double* x, double* y, hipStream_t s, const float* x32) {
   if (A.nblk <= 0) return hipSuccess;
-  if (fp32)
-    hipLaunchKernelGGL((k_csr<float>), dim3(unsigned(A.nblk)), dim3(256), 0, s, A, x, y);
+  if (fp32 && x32)
+    hipLaunchKernelGGL((k_csr<float, float>), dim3(unsigned(A.nblk)), dim3(256), 0, s, A, x32, y);
+  else if (fp32)
+    hipLaunchKernelGGL((k_csr<float, double>), dim3(unsigned(A.nblk)), dim3(256), 0, s, A, x, y);
   else
-    hipLaunchKernelGGL((k_csr<double>), dim3(unsigned(A.nblk)), dim3(256), 0, s, A, x, y);
+    hipLaunchKernelGGL((k_csr<double, double>), dim3(unsigned(A.nblk)), dim3(256), 0, s, A, x, y);
   return hipGetLastError();
 }
 
