@@ -1149,14 +1149,22 @@ static void on_op_stream(gsg_op* op, void* cs, F&& fn) {
   HIPC(hipEventRecord(out, op->stream));
   HIPC(hipStreamWaitEvent(c, out, 0));
 }
+// Whether cs (NULL: the current device's null stream) belongs to the handle's device.
+static bool on_op_device(const gsg_op* op, hipStream_t cs) {
+  int dev = -1;
+  const hipError_t e = cs ? hipStreamGetDevice(cs, &dev) : hipGetDevice(&dev);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e == hipSuccess && dev == op->device;
+}
 // Runs fn on the caller's stream itself, after the handle's earlier calls.  For work without
 // stream capture of its own (one application): the hop to the handle's stream and back cost
 // more than a small operator (two event records, two waits on the host and two
-// cross-stream dependencies on the device).
+// cross-stream dependencies on the device).  A stream of another device keeps the hop: the
+// kernels run where the handle's memory is, or the runtime refuses the event.
 template <typename F>
 static void on_caller_stream(gsg_op* op, void* cs, F&& fn) {
   hipStream_t c = static_cast<hipStream_t>(cs);
-  if (capturing(c)) {
+  if (capturing(c) || !on_op_device(op, c)) {
     on_op_stream(op, cs, fn);
     return;
   }
