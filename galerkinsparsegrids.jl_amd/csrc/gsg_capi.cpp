@@ -461,7 +461,13 @@ static std::shared_ptr<Tables> get_tables(int D, int k, int n, int full, int tki
 // kernel selection: built-in rule, tuning table, GSG_KERNEL environment override
 
 static std::mutex g_tune_mu;
-static std::map<std::tuple<int, int, int, int>, int> g_tune;
+// a grid's entry: `asked` by gsg_tune_set (that kernel runs in every launch), else measured (a
+// line of the tuning file, or GSG_KERNEL_TUNED: the kernel of launches that fill the chip)
+struct TuneEntry {
+  int variant = GSG_KERNEL_AUTO;
+  bool asked = false;
+};
+static std::map<std::tuple<int, int, int, int>, TuneEntry> g_tune;
 static std::once_flag g_tune_loaded;
 // the launch schedule of FP32 batches and servers whose own setting is GSG_SCHEDULE_AUTO
 // (a "schedule S" line of the tuning file, or gsg_tune_schedule); -1: not set
@@ -514,7 +520,7 @@ static void load_tune_file() {
     if (D < 1 || D > MAXD || k < 1 || k > KMAX || n < 0 || n > 20 || (prec != 0 && prec != 1)) continue;
     if (var != GSG_KERNEL_AUTO && var != GSG_KERNEL_PLAN && var != GSG_KERNEL_TILE && var != GSG_KERNEL_TILE_ALT)
       continue;
-    g_tune.emplace(std::make_tuple(D, k, n, prec), var);  // keeps entries set before the load
+    g_tune.emplace(std::make_tuple(D, k, n, prec), TuneEntry{var, false});  // keeps entries set before the load
   }
 }
 
@@ -547,23 +553,34 @@ static int resolve_schedule(int own) {
 // the segmented shapes only
 static bool tile_alt_ok(int D, int k, bool fp32) { return fp32 && seg_ok(D, k) && seg_cpw(D, k) > 1; }
 
-// The variant a grid runs: GSG_KERNEL_PLAN, GSG_KERNEL_TILE or GSG_KERNEL_TILE_ALT
-// (GSG_KERNEL=plan / tile in the environment, else the tuning table, else the built-in
-// rule: the tile variant wherever it applies).
-static int grid_variant(const Tables& T, bool fp32) {
-  if (!T.tile_ok) return GSG_KERNEL_PLAN;
+// How a grid's kernel was chosen: the variant, whether it was asked for (GSG_KERNEL in the
+// environment, gsg_tune_set) and runs in every launch, and whether an entry holds it.
+struct GridChoice {
+  int variant = GSG_KERNEL_PLAN;
+  bool asked = false, entry = false;
+};
+// GSG_KERNEL=plan / tile in the environment, else the tuning table, else the built-in rule:
+// the tile variant wherever it applies.
+static GridChoice grid_choice(const Tables& T, bool fp32) {
+  GridChoice c;
   if (const char* kv = std::getenv("GSG_KERNEL")) {
-    if (std::string(kv) == "plan") return GSG_KERNEL_PLAN;
-    if (std::string(kv) == "tile") return GSG_KERNEL_TILE;
+    c.asked = true;
+    if (T.tile_ok && std::string(kv) == "tile") c.variant = GSG_KERNEL_TILE;
+    if (std::string(kv) == "tile" || std::string(kv) == "plan") return c;
   }
   std::call_once(g_tune_loaded, load_tune_file);
   std::lock_guard<std::mutex> g(g_tune_mu);
   auto it = g_tune.find(std::make_tuple(T.D, T.k, T.n, fp32 ? 1 : 0));
-  if (it == g_tune.end() || it->second == GSG_KERNEL_AUTO) return GSG_KERNEL_TILE;
-  if (it->second == GSG_KERNEL_TILE_ALT && !tile_alt_ok(T.D, T.k, fp32)) return GSG_KERNEL_TILE;
-  return it->second;
+  if (it != g_tune.end() && it->second.variant != GSG_KERNEL_AUTO) {
+    c.entry = true;
+    c.asked = c.asked || it->second.asked;
+  }
+  if (!T.tile_ok) return c;
+  c.variant = c.entry ? it->second.variant : GSG_KERNEL_TILE;
+  if (c.variant == GSG_KERNEL_TILE_ALT && !tile_alt_ok(T.D, T.k, fp32)) c.variant = GSG_KERNEL_TILE;
+  return c;
 }
-static bool use_tile(const Tables& T, bool fp32) { return grid_variant(T, fp32) != GSG_KERNEL_PLAN; }
+static int grid_variant(const Tables& T, bool fp32) { return grid_choice(T, fp32).variant; }
 
 // ---------------------------------------------------------------------------------
 // one solve's device state
@@ -753,13 +770,16 @@ static int64_t dsplit_waves(int32_t kernel, int D, int K, bool fp32) {
 // 244; D = 1, k = 5, n = 9 254 / 1177; D = 5, k = 2, n = 6 137 / 202.  One solve (the plan
 // kernel with its directions split): D = 3, k = 5, n = 6 15.4 / 29.2; D = 2, k = 5, n = 9
 // 17.5 / 154; D = 6, k = 2, n = 5 10.8 / 12.8.
+// A measured entry stands for the launches that fill the chip (the tuner measures those); a
+// kernel that was asked for runs in every launch.
 constexpr int64_t FIBER_MIN_WAVES = 8192;
 // launch_waves: the wavefronts of every launch that runs beside this one
 static LdsShape lds_shape(const Tables& T, bool fp32, int64_t launch_cells, int64_t launch_waves) {
   LdsShape L = lds_shape(T, fp32);
   if (!fp32 && L.kernel == KERNEL_SEG && launch_cells < SEG64_MIN_CELLS) L = LdsShape{};
-  if (L.kernel == KERNEL_FIBER && !std::getenv("GSG_KERNEL") &&
-      (launch_waves <= FIBER_MIN_WAVES || T.D == 1 || T.D > 3 || (T.D == 2 && T.n > 6)))
+  const GridChoice c = grid_choice(T, fp32);
+  if (L.kernel == KERNEL_FIBER && !c.asked &&
+      (launch_waves <= FIBER_MIN_WAVES || (!c.entry && (T.D == 1 || T.D > 3 || (T.D == 2 && T.n > 6)))))
     L = LdsShape{};
   if (T.D > 1) L.dsplit = launch_waves <= dsplit_waves(L.kernel, T.D, T.k, fp32);
   return L;
@@ -813,7 +833,7 @@ struct SoloShape {
 };
 static SoloShape solo_shape(const Tables& T, const LdsShape& L, bool fp32, bool wave) {
   SoloShape q;
-  if (!T.solo_ent.p || std::getenv("GSG_KERNEL")) return q;  // a forced stage kernel runs as asked
+  if (!T.solo_ent.p || grid_choice(T, fp32).asked) return q;  // a stage kernel runs as asked
   if (fp32 && L.kernel == KERNEL_DIRECT) return q;           // its lo correction is the matrix cores' bf16 product
   const int es = fp32 ? 4 : 8;
   const int N = int(T.lt.N), ne = int(T.plan.ent.size() / 2);
@@ -1282,12 +1302,12 @@ int gsg_tune_set(int32_t D, int32_t k, int32_t n, int32_t precision, int32_t var
   return guarded([&] {
     require(D >= 1 && D <= MAXD && k >= 1 && k <= KMAX && n >= 0 && n <= 20, "invalid (D, k, n)");
     require(precision == GSG_PREC_FP64 || precision == GSG_PREC_FP32, "unknown precision");
-    require(variant == GSG_KERNEL_AUTO || variant == GSG_KERNEL_PLAN || variant == GSG_KERNEL_TILE ||
-                variant == GSG_KERNEL_TILE_ALT,
+    const int32_t v = variant & ~GSG_KERNEL_TUNED;
+    require(v == GSG_KERNEL_AUTO || v == GSG_KERNEL_PLAN || v == GSG_KERNEL_TILE || v == GSG_KERNEL_TILE_ALT,
             "unknown kernel variant");
     std::call_once(g_tune_loaded, load_tune_file);
     std::lock_guard<std::mutex> g(g_tune_mu);
-    g_tune[std::make_tuple(D, k, n, precision)] = variant;
+    g_tune[std::make_tuple(D, k, n, precision)] = TuneEntry{v, !(variant & GSG_KERNEL_TUNED)};
   });
 }
 

@@ -15,8 +15,10 @@ steps of a mixed workload.
 
 The choices are written to ``gsg_tune.txt`` beside libgsg.so: one line
 ``D k n precision variant`` per grid, ``lanes L`` and ``schedule S``; the library
-reads that file at first use, so C, Julia and Python callers all get the tuned choice.
-`set_variant` overrides one grid for the current process.  This has no counterpart in
+reads that file at first use, so C, Julia and Python callers all get the tuned choice for
+the launches that fill the GPU (small launches, and solves small enough to run resident in
+a workgroup, go by size).  `set_variant` makes one grid run one kernel in every launch of
+the current process.  This has no counterpart in
 the reference, which has a single SpMV path (SparseArrays' CSC product).
 """
 from __future__ import annotations
@@ -31,6 +33,7 @@ from ._lib import LIBPATH, PREC, check, lib
 from .solvers import Batch
 
 AUTO, PLAN, TILE, TILE_ALT = 0, 1, 2, 3
+TUNED = 16  # or-ed to a variant: recorded as a line of the tuning file is
 VARIANT = {"auto": AUTO, "plan": PLAN, "tile": TILE, "tile_alt": TILE_ALT}
 VARIANT_NAME = {AUTO: "auto", PLAN: "plan", TILE: "tile", TILE_ALT: "tile_alt"}
 SCHEDULE = {"auto": 0, "streams": 1, "fused": 2}
@@ -49,12 +52,13 @@ def tile_eligible(D: int, k: int) -> bool:
 
 def set_variant(D: int, k: int, n: int, precision: str, variant: str) -> None:
     """Use `variant` ('plan', 'tile', 'tile_alt' or 'auto') for operators and batches
-    created later."""
+    created later, in every launch (no resident solves, no choice by launch size)."""
     check(lib().gsg_tune_set(D, k, n, PREC[precision], VARIANT[variant]))
 
 
 def get_variant(D: int, k: int, n: int, precision: str) -> str:
-    """The variant ('plan', 'tile' or 'tile_alt') that runs for this grid and precision."""
+    """The variant ('plan', 'tile' or 'tile_alt') of this grid and precision, before the rules
+    that go by size."""
     return VARIANT_NAME[check(lib().gsg_tune_get(D, k, n, PREC[precision]))]
 
 

@@ -127,15 +127,19 @@ int gsg_points_1d(int32_t k, int32_t n, double *x, int64_t len);
 
 /* ---- kernel selection (autotuning) --------------------------------------------- */
 
-/* No counterpart in the reference.  Two kernels apply the operator: the LDS fiber
- * kernel (grids with D <= 6, k <= 5, k^D <= 256 and D k^(D-1) <= 256) and the
- * scalar-plan gather kernel (every grid).  gsg_tune_set records which one runs for a
- * grid and precision; GSG_KERNEL_AUTO restores the built-in rule.  Takes effect for
- * operators, batches and servers created afterwards.  Thread-safe.  The choice is between
- * the kernels of one launch a stage: RK4 solves small enough for one compute unit run
- * resident in a workgroup, with the same sums, unless the environment's GSG_KERNEL asks
- * for a stage kernel, and a small launch takes its kernel's form with a wavefront per
- * direction (TILE_ALT: the rule's round there). */
+/* No counterpart in the reference.  Two kernels apply the operator: the tile kernel (the
+ * direct, segmented or LDS fiber kernel by shape; grids with D <= 6, k <= 5, k^D <= 256 and
+ * D k^(D-1) <= 256) and the scalar-plan gather kernel (every grid).  gsg_tune_set records
+ * which one runs for a grid and precision, in every launch; GSG_KERNEL_AUTO restores the
+ * built-in rule.  Takes effect for operators, batches and servers created afterwards.
+ * Thread-safe.
+ *   Without such a call the rule goes by size as well: RK4 solves small enough for one compute
+ * unit run resident in a workgroup, with the same sums, and the FP64 fiber kernel runs in
+ * launches of more than 8192 wavefronts only, and, unless an entry of gsg_tune.txt says so,
+ * not for D = 1, D > 3 or D = 2 with n > 6 (the plan kernel does).
+ *   In every case a small launch takes its kernel's form with a wavefront per direction
+ * (TILE_ALT: the rule's round there), and the FP64 segmented kernel (k = 2) needs 65,536
+ * cells in a launch. */
 #define GSG_KERNEL_AUTO 0
 #define GSG_KERNEL_PLAN 1
 #define GSG_KERNEL_TILE 2
@@ -143,9 +147,12 @@ int gsg_points_1d(int32_t k, int32_t n, double *x, int64_t len);
  * other number of coupled input cells moved per load round (4 where the rule takes 2,
  * 2 where it takes 4) in the RK stages; elsewhere it means GSG_KERNEL_TILE. */
 #define GSG_KERNEL_TILE_ALT 3
+/* Or-ed to a variant: recorded as a line of gsg_tune.txt is, for the launches that fill the
+ * chip; the size rules above stay in force. */
+#define GSG_KERNEL_TUNED 16
 int gsg_tune_set(int32_t D, int32_t k, int32_t n, int32_t precision, int32_t variant);
-/* The variant that runs for (D, k, n, precision): GSG_KERNEL_PLAN, GSG_KERNEL_TILE or
- * GSG_KERNEL_TILE_ALT. */
+/* The variant of (D, k, n, precision), before the size rules: GSG_KERNEL_PLAN,
+ * GSG_KERNEL_TILE or GSG_KERNEL_TILE_ALT. */
 int gsg_tune_get(int32_t D, int32_t k, int32_t n, int32_t precision);
 /* Streams (1..8) a batch or server spreads its (D, k) classes over under the streams
  * schedule (0: the tuned count, a "lanes L" line of gsg_tune.txt, else 4).  Takes effect
