@@ -96,8 +96,9 @@ def autotune(grids=None, precisions=("fp32", "fp64"), steps=6, min_dofs=3_000_00
     """Time the variants of every tile-eligible grid in `grids` ((D, k, n) tuples): plan,
     tile, and tile_alt where the segmented kernel serves the grid; keep the fastest.  Each
     measurement advances enough copies of a transport solve to cover at least `min_dofs`
-    DoFs, so the launch fills the GPU as in a busy batch; tile_alt must also beat tile on
-    one copy alone (a grid's entry also serves its single solves).
+    DoFs, so the launch fills the GPU as in a busy batch; tile_alt must also not lose to tile
+    on one copy alone (a grid's entry also serves its single solves).  The choices are in
+    force in this process too, as the file's lines would be.
 
     Returns a list of dicts (D, k, n, precision, variant and the <variant>_ms timed).  With
     `write`, the table is written to `path` (default: beside libgsg.so), merged with
@@ -119,15 +120,16 @@ def autotune(grids=None, precisions=("fp32", "fp64"), steps=6, min_dofs=3_000_00
         best = min(t, key=t.get)
         if best == "tile_alt":
             # the table is keyed by grid, and a grid also runs as a single solve: the other
-            # round size is kept only if it also wins on one copy of the grid alone
+            # round size is dropped where it clearly loses on one copy of the grid alone (a
+            # small launch runs the same code for both, a wavefront per direction)
             one = {}
             for v in ("tile", "tile_alt"):
                 set_variant(D, k, n, prec, v)
                 one[v] = _class_ms(prec, D, k, n, 1, steps, seed=D * 100 + k * 10 + n)
             t.update({f"{v}_single": ms for v, ms in one.items()})
-            if one["tile_alt"] >= one["tile"]:
+            if one["tile_alt"] > 1.03 * one["tile"]:
                 best = "tile"
-        set_variant(D, k, n, prec, best)
+        check(lib().gsg_tune_set(D, k, n, PREC[prec], VARIANT[best] | TUNED))
         rows.append(dict(D=D, k=k, n=n, precision=prec, variant=best, **{f"{v}_ms": ms for v, ms in t.items()}))
         if verbose:
             print(f"tune D={D} k={k} n={n} {prec}: " + ", ".join(f"{v} {ms:.4f} ms" for v, ms in t.items()) +

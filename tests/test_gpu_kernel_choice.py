@@ -1,5 +1,5 @@
 """Which kernel runs: one that gsg_tune_set asks for runs in every launch, a tuned entry in the
-launches that fill the chip."""
+launches that fill the chip, and the tuner times launches of the kernels it names."""
 import numpy as np
 import pytest
 
@@ -54,5 +54,21 @@ def test_a_tuned_entry_goes_by_size(g, gpu):
             check(lib().gsg_tune_set(D, k, n, 0, tune.VARIANT[v] | tune.TUNED))
             assert _run(g, D, k, n, "fp64")[1] == [(one, 12)]
             assert _run(g, D, k, n, "fp64", copies=40)[1] == [(many, 12)]
+    finally:
+        tune.set_variant(D, k, n, "fp64", "auto")
+
+
+def test_tuner_times_stage_launches(g, gpu, tmp_path):
+    """A grid small enough to run resident: the tuner's times are of a stage launch of each
+    kernel, and its choice leaves the grid's solves resident."""
+    from galerkinsparsegrids_jl_amd import tune
+    print("[gpu] tuner on a small grid", flush=True)
+    D, k, n = 2, 3, 4
+    try:
+        rows = tune.autotune([(D, k, n)], ("fp64",), steps=3, min_dofs=500_000, path=tmp_path / "t.txt")
+        assert set(rows[0]) >= {"plan_ms", "tile_ms"} and rows[0]["variant"] in ("plan", "tile")
+        assert tune.read_table(tmp_path / "t.txt") == {(D, k, n, "fp64"): rows[0]["variant"]}
+        assert [launches for _, launches in _run(g, D, k, n, "fp64")[1]] == [1]  # all steps in one
+        assert tune.get_variant(D, k, n, "fp64") == rows[0]["variant"]
     finally:
         tune.set_variant(D, k, n, "fp64", "auto")
