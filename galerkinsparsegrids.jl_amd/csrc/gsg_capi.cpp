@@ -1975,6 +1975,7 @@ struct Group {
   std::vector<Tile> tiles;
   DevMem dtiles;
   int64_t dofs = 0;  // component DoFs covered per launch
+  int64_t active = 0;  // those of its unfinished solves
   LdsShape lds;      // kernel; for the fiber kernel the LDS layout (maxima over the group)
   SoloShape solo;    // resident solves: all steps of a call in one launch (maxima over the group)
   std::vector<int32_t> ids;  // resident: the group's solves
@@ -1988,6 +1989,7 @@ struct Scheduler {
   std::vector<SolveDesc> descs;
   DevMem ddescs;
   std::vector<Group> groups;
+  std::vector<size_t> group_of;  // of each solve of descs
   // kernel timing
   bool profile = false;
   std::vector<hipEvent_t> evpool;
@@ -2082,6 +2084,7 @@ struct Scheduler {
     reset_graph();
     descs.clear();
     groups.clear();
+    group_of.clear();
     std::map<std::tuple<int, int, int, int, int>, size_t> gidx;
     std::vector<std::vector<size_t>> members;
     auto solo_of = [&](const SolveState& S) {
@@ -2116,7 +2119,7 @@ struct Scheduler {
       auto it = gidx.find(key);
       if (it == gidx.end()) {
         gidx[key] = groups.size();
-        groups.push_back(Group{S.T->D, S.T->k, S.desc.sys, {}, {}, 0, L, q, {}, {}});
+        groups.push_back(Group{S.T->D, S.T->k, S.desc.sys, {}, {}, 0, 0, L, q, {}, {}});
         members.emplace_back();
         it = gidx.find(key);
       }
@@ -2128,6 +2131,8 @@ struct Scheduler {
         g.solo.us = std::max(g.solo.us, q.us);
       }
       groups[it->second].dofs += S.N;
+      groups[it->second].active += S.N;
+      group_of.push_back(it->second);
       members[it->second].push_back(s);
     }
     for (size_t gi = 0; gi < groups.size(); ++gi) {
@@ -2228,6 +2233,7 @@ struct Scheduler {
   void deactivate(size_t s) {
     if (s >= descs.size() || !descs[s].active) return;
     descs[s].active = 0;
+    groups[group_of[s]].active -= descs[s].N;
     CaptureGuard cg(g_capture_mu);
     HIPC(hipMemcpy(reinterpret_cast<unsigned char*>(ddescs.p) + s * sizeof(SolveDesc) + offsetof(SolveDesc, active),
                    &descs[s].active, sizeof(int32_t), hipMemcpyHostToDevice));
@@ -2237,6 +2243,7 @@ struct Scheduler {
   void switch_off(size_t s) {
     if (s >= descs.size() || !descs[s].active) return;
     descs[s].active = 0;
+    groups[group_of[s]].active -= descs[s].N;
     HIPC(launch_switch_off(ddescs.as<SolveDesc>() + s, stream));
   }
 
@@ -2268,7 +2275,8 @@ struct Scheduler {
     HIPC(hipEventRecord(next_event(), stream));
     HIPC(launch_op(g.D, g.K, fp32, a, stream));
     HIPC(hipEventRecord(next_event(), stream));
-    pend.push_back(Pending{g.D, g.K, g.sys, g.tiled(), g.dofs, double(g.dofs) * stage_bytes(g.sys, op, stage, fp32, g.D), e0});
+    pend.push_back(Pending{g.D, g.K, g.sys, g.tiled(), g.active,
+                           double(g.active) * stage_bytes(g.sys, op, stage, fp32, g.D), e0});
   }
 
   // all k steps of a resident group
@@ -2283,7 +2291,7 @@ struct Scheduler {
       if (g.sys == SYS_WAVE) b += stage_bytes(g.sys, OP_RK_WAVE_GRAD, stage, fp32, g.D);
       b += stage_bytes(g.sys, g.sys == SYS_WAVE ? OP_RK_WAVE_SUM : OP_RK_SUM, stage, fp32, g.D);
     }
-    pend.push_back(Pending{g.D, g.K, g.sys, g.tiled(), g.dofs, double(g.dofs) * b * double(k), e0});
+    pend.push_back(Pending{g.D, g.K, g.sys, g.tiled(), g.active, double(g.active) * b * double(k), e0});
   }
 
   // GSG_STREAMS=1 runs every launch on the batch stream (for kernel-trace profiles whose
@@ -2315,7 +2323,7 @@ struct Scheduler {
   void enqueue(int64_t n) {
     if (schedule == GSG_SCHEDULE_FUSED && !profile) {
       for (const Group& g : groups)
-        if (g.solo.on) launch_solo_group(g, n, stream);
+        if (g.solo.on && g.active) launch_solo_group(g, n, stream);
       for (int64_t st = 0; st < n; ++st)
         for (int stage = 1; stage <= 4; ++stage) {
           if (fused[0].nseg) HIPC(launch_fused(fused_pass_a, stage, fused[0], fused[0].items, stream));
@@ -2334,11 +2342,11 @@ struct Scheduler {
       for (int l = 0; l < nlanes; ++l) HIPC(hipStreamWaitEvent(lanes[l], fork, 0));
     }
     for (size_t gi = 0; gi < groups.size(); ++gi)
-      if (groups[gi].solo.on) launch_solo_group(groups[gi], n, par ? lanes[lane_of[gi]] : stream);
+      if (groups[gi].solo.on && groups[gi].active) launch_solo_group(groups[gi], n, par ? lanes[lane_of[gi]] : stream);
     for (int64_t st = 0; st < n; ++st)
       for (size_t gi = 0; gi < groups.size(); ++gi) {
         const Group& g = groups[gi];
-        if (g.solo.on) continue;
+        if (g.solo.on || !g.active) continue;
         hipStream_t s = par ? lanes[lane_of[gi]] : stream;
         for (int stage = 1; stage <= 4; ++stage) {
           if (g.sys == SYS_WAVE) {

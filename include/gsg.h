@@ -277,7 +277,7 @@ typedef struct gsg_kernel_stat {
     int64_t launches;             /* kernel launches timed */
     double total_ms;              /* summed launch durations */
     double algo_bytes;            /* summed algorithmic HBM bytes of those launches */
-    int64_t dofs;                 /* state DoFs of the class (per launch) */
+    int64_t dofs;                 /* state DoFs of the class's unfinished solves (last launch) */
 } gsg_kernel_stat;
 
 int gsg_batch_profile(gsg_batch *b, int32_t enable);

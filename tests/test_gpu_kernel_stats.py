@@ -1,0 +1,30 @@
+"""A batch's kernel statistics count the unfinished solves of a class."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _batch(g, prec, solves):
+    b = g.Batch(prec)
+    for kind, D, k, n, steps in solves:
+        y0 = np.random.default_rng(n).standard_normal(g.get_size(D, k, n) * (2 if kind == "wave" else 1))
+        b.add(kind, D, k, n, y0, 0.02 * 2.0 ** -n, steps, a=[0.3, -0.8, 0.5][:D] if kind == "transport" else None)
+    b.profile(True)
+    b.run()
+    st = {(s["D"], s["k"], s["sys"], s["variant"]): s for s in b.kernel_stats()}
+    b.close()
+    return st
+
+
+def test_finished_solves_are_not_counted(g, gpu):
+    print("[gpu] statistics of finished solves", flush=True)
+    N5, N8 = g.get_size(3, 3, 5), g.get_size(3, 3, 8)
+    # no rebuild: the solves that finish hold less than a quarter of the batch
+    st = _batch(g, "fp32", [("transport", 3, 3, 8, 10), ("transport", 3, 3, 5, 4), ("transport", 3, 4, 5, 3)])
+    # per entry and step: the float input, and the stage's reads and writes
+    per = sum(4 + e for e in (8 + 8 + 4, 8 + 16 + 4, 8 + 16 + 4, 8 + 8 + 4))
+    a, c = st[(3, 3, 0, 2)], st[(3, 4, 0, 2)]
+    assert a["launches"] == 4 * 10 and a["dofs"] == N8
+    assert a["algo_bytes"] == per * (10 * N8 + 4 * N5)
+    assert c["launches"] == 4 * 3 and c["algo_bytes"] == per * 3 * g.get_size(3, 4, 5)
