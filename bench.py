@@ -46,10 +46,13 @@ def log(msg):
 def kernel_name(stat):
     """Source name of the kernel a (D, k) class ran: the scalar-plan gather kernel, or
     the tile variant: the direct kernel for D = 4, k = 4; in float the segmented
-    kernel for the other D <= 4, k <= 4 shapes; the LDS fiber kernel otherwise."""
+    kernel for the other D <= 4, k <= 4 shapes; the LDS fiber kernel otherwise; or the
+    resident kernel of small solves."""
     D, k = stat["D"], stat["k"]
     fp32 = stat["precision"] == 1
     dtype = "float" if fp32 else "double"
+    if stat["variant"] == 4:  # resident in a workgroup
+        return f"k_solo<{D},{k},{dtype}>"
     if stat["variant"] != 2:
         return f"k_plan<{D},{k},{dtype}>"
     if (D, k) == (4, 4):

@@ -854,16 +854,16 @@ static SoloShape solo_shape(const Tables& T, const LdsShape& L, bool fp32, bool 
 }
 // nsteps RK4 steps of nsolve solves of one shape (ids: their indices, null: 0, 1, ...),
 // cut into launches of a few milliseconds
+constexpr int64_t SOLO_STEPS = 256;
 static void launch_solo_steps(int D, int K, bool fp32, const SoloShape& q, const SolveDesc* solves, const int32_t* ids,
                               int nsolve, int64_t nsteps, hipStream_t s) {
-  constexpr int64_t STEPS = 256;
   SoloArgs a{};
   a.solves = solves;
   a.ids = ids;
   a.vals_lds = q.vals ? 1 : 0;
   a.small_map = q.small ? 1 : 0;
   for (; nsteps > 0; nsteps -= a.nsteps) {
-    a.nsteps = std::min(nsteps, STEPS);
+    a.nsteps = std::min(nsteps, SOLO_STEPS);
     HIPC(launch_solo(D, K, fp32, q.segr, a, nsolve, q.threads, q.lds, s));
   }
 }
@@ -1969,6 +1969,14 @@ static double stage_bytes(int sys, int op, int stage, bool fp32, int D) {
   return D * es + es + 2.0 * epi_noinput + (stage == 1 && !fp32 ? 16.0 : 0.0);
 }
 
+// The same of k resident steps in `launches` launches: the operator's vectors stay in LDS, the
+// RK registers y and acc are read and written by each stage (80 bytes an entry and step), y
+// is read and, in float, the next stage input left at the ends of a launch.
+static double solo_bytes(int sys, bool fp32, int64_t k, int64_t launches) {
+  const double ends = sys == SYS_WAVE ? 16.0 + (fp32 ? 12.0 : 0.0) : 8.0 + (fp32 ? 4.0 : 0.0);
+  return (sys == SYS_WAVE ? 160.0 : 80.0) * double(k) + ends * double(launches);
+}
+
 // Device-side grouping of resident solves into (D, K, sys) classes with tile lists.
 struct Group {
   int D, K, sys;
@@ -1980,7 +1988,8 @@ struct Group {
   SoloShape solo;    // resident solves: all steps of a call in one launch (maxima over the group)
   std::vector<int32_t> ids;  // resident: the group's solves
   DevMem dids;
-  bool tiled() const { return lds.kernel != KERNEL_PLAN; }
+  // the kernel of the group's statistics (gsg_kernel_stat::variant)
+  int variant() const { return solo.on ? GSG_KERNEL_RESIDENT : lds.kernel == KERNEL_PLAN ? GSG_KERNEL_PLAN : GSG_KERNEL_TILE; }
 };
 
 struct Scheduler {
@@ -1995,14 +2004,13 @@ struct Scheduler {
   std::vector<hipEvent_t> evpool;
   size_t evused = 0;
   struct Pending {
-    int D, K, sys;
-    bool tiled;
-    int64_t dofs;
+    int D, K, sys, variant;
+    int64_t dofs, launches;
     double bytes;
     size_t ev;
   };
   std::vector<Pending> pend;
-  std::map<std::tuple<int, int, int, bool>, gsg_kernel_stat> stats;
+  std::map<std::tuple<int, int, int, int>, gsg_kernel_stat> stats;
   // Solves of different classes are independent, so each class runs its stages on one
   // of NLANE streams (default priority) and the classes overlap on the GPU: the small
   // classes fill the gaps the large ones leave.  The batch stream forks to the lanes
@@ -2275,7 +2283,7 @@ struct Scheduler {
     HIPC(hipEventRecord(next_event(), stream));
     HIPC(launch_op(g.D, g.K, fp32, a, stream));
     HIPC(hipEventRecord(next_event(), stream));
-    pend.push_back(Pending{g.D, g.K, g.sys, g.tiled(), g.active,
+    pend.push_back(Pending{g.D, g.K, g.sys, g.variant(), g.active, 1,
                            double(g.active) * stage_bytes(g.sys, op, stage, fp32, g.D), e0});
   }
 
@@ -2286,12 +2294,9 @@ struct Scheduler {
     launch_solo_steps(g.D, g.K, fp32, g.solo, ddescs.as<SolveDesc>(), g.dids.as<int32_t>(), int(g.ids.size()), k, st);
     if (!profile) return;
     HIPC(hipEventRecord(next_event(), st));
-    double b = 0;
-    for (int stage = 1; stage <= 4; ++stage) {
-      if (g.sys == SYS_WAVE) b += stage_bytes(g.sys, OP_RK_WAVE_GRAD, stage, fp32, g.D);
-      b += stage_bytes(g.sys, g.sys == SYS_WAVE ? OP_RK_WAVE_SUM : OP_RK_SUM, stage, fp32, g.D);
-    }
-    pend.push_back(Pending{g.D, g.K, g.sys, g.tiled(), g.active, double(g.active) * b * double(k), e0});
+    const int64_t launches = (k + SOLO_STEPS - 1) / SOLO_STEPS;
+    pend.push_back(Pending{g.D, g.K, g.sys, g.variant(), g.active, launches,
+                           double(g.active) * solo_bytes(g.sys, fp32, k, launches), e0});
   }
 
   // GSG_STREAMS=1 runs every launch on the batch stream (for kernel-trace profiles whose
@@ -2370,13 +2375,13 @@ struct Scheduler {
     for (const Pending& p : pend) {
       float ms = 0.f;
       HIPC(hipEventElapsedTime(&ms, evpool[p.ev], evpool[p.ev + 1]));
-      gsg_kernel_stat& s = stats[std::make_tuple(p.D, p.K, p.sys, p.tiled)];
+      gsg_kernel_stat& s = stats[std::make_tuple(p.D, p.K, p.sys, p.variant)];
       s.D = p.D;
       s.k = p.K;
       s.precision = fp32 ? GSG_PREC_FP32 : GSG_PREC_FP64;
       s.sys = p.sys;
-      s.variant = p.tiled ? GSG_KERNEL_TILE : GSG_KERNEL_PLAN;
-      s.launches += 1;
+      s.variant = p.variant;
+      s.launches += p.launches;
       s.total_ms += ms;
       s.algo_bytes += p.bytes;
       s.dofs = p.dofs;

@@ -272,13 +272,16 @@ int64_t gsg_batch_dofs(const gsg_batch *b);
  * and its duration is accumulated per (D, k, system, kernel variant) class. */
 typedef struct gsg_kernel_stat {
     int32_t D, k, precision, sys; /* sys: 0 sum-form (transport), 1 wave */
-    int32_t variant;              /* GSG_KERNEL_PLAN or GSG_KERNEL_TILE */
+    int32_t variant;              /* GSG_KERNEL_PLAN, GSG_KERNEL_TILE or GSG_KERNEL_RESIDENT */
     int32_t reserved;
     int64_t launches;             /* kernel launches timed */
     double total_ms;              /* summed launch durations */
     double algo_bytes;            /* summed algorithmic HBM bytes of those launches */
     int64_t dofs;                 /* state DoFs of the class's unfinished solves (last launch) */
 } gsg_kernel_stat;
+/* Statistics only: solves resident in a workgroup, many RK4 steps a launch; algo_bytes counts
+ * the RK registers, the operator's vectors stay in LDS. */
+#define GSG_KERNEL_RESIDENT 4
 
 int gsg_batch_profile(gsg_batch *b, int32_t enable);
 

@@ -1,4 +1,5 @@
-"""A batch's kernel statistics count the unfinished solves of a class."""
+"""A batch's kernel statistics count the unfinished solves of a class, and resident solves in
+an entry of their own."""
 import numpy as np
 import pytest
 
@@ -28,3 +29,16 @@ def test_finished_solves_are_not_counted(g, gpu):
     assert a["launches"] == 4 * 10 and a["dofs"] == N8
     assert a["algo_bytes"] == per * (10 * N8 + 4 * N5)
     assert c["launches"] == 4 * 3 and c["algo_bytes"] == per * 3 * g.get_size(3, 4, 5)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_resident_solves_have_their_own_entry(g, gpu, prec):
+    print(f"[gpu] statistics of resident solves {prec}", flush=True)
+    N5, N4 = g.get_size(2, 3, 5), g.get_size(2, 3, 4)
+    st = _batch(g, prec, [("transport", 2, 3, 5, 300), ("wave", 2, 3, 4, 300), ("transport", 2, 3, 9, 300)])
+    r, w = st[(2, 3, 0, 4)], st[(2, 3, 1, 4)]
+    lo = 4 if prec == "fp32" else 0
+    assert r["launches"] == 2 and r["dofs"] == N5 and r["algo_bytes"] == N5 * (80 * 300 + 2 * (8 + lo))
+    assert w["launches"] == 2 and w["algo_bytes"] == N4 * (160 * 300 + 2 * (16 + 3 * lo))
+    staged = [s for key, s in st.items() if key[3] != 4]
+    assert len(staged) == 1 and staged[0]["launches"] == 4 * 300 and staged[0]["dofs"] == g.get_size(2, 3, 9)
