@@ -2229,13 +2229,6 @@ struct Scheduler {
     }
   }
 
-  // change the schedule of a built batch (the captured steps are recorded anew)
-  void set_schedule(int s) {
-    schedule_own = s;
-    reset_graph();
-    build_fused();
-  }
-
   // stop advancing solve s of the last build (its launches then skip it); call with the
   // stream idle.  The captured step graphs stay valid: they read the descriptors.
   void deactivate(size_t s) {
@@ -2543,11 +2536,12 @@ int gsg_batch_schedule(gsg_batch* b, int32_t schedule) {
     require(b != nullptr, "NULL batch");
     require(schedule == GSG_SCHEDULE_AUTO || schedule == GSG_SCHEDULE_STREAMS || schedule == GSG_SCHEDULE_FUSED,
             "unknown schedule");
-    if (b->built) {
+    b->sched.schedule_own = schedule;
+    // built for another schedule: the kernels' forms are chosen with it (fused launches do not
+    // split directions)
+    if (b->built && !b->active.empty()) {
       HIPC(hipStreamSynchronize(b->stream));
-      b->sched.set_schedule(schedule);
-    } else {
-      b->sched.schedule_own = schedule;
+      batch_reschedule(b);
     }
   });
 }
