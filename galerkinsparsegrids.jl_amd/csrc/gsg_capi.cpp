@@ -2104,13 +2104,16 @@ struct Scheduler {
     double busy = 0;
     for (SolveState* S : solves)
       if (!solo_of(*S).on) busy += stage_us(double(S->N), S->T->D, S->T->k, S->desc.sys);
-    const bool solo_ok = busy <= SOLO_BATCH_US;
+    // The fused launches follow resident steps in stream order, so there only alone.  FP32,
+    // uneven transport solves, fused, us a step with resident ones first / without: 12 solves
+    // 109 / 84, 48 solves 319 / 231.
+    const bool whole = fp32 && resolve_schedule(schedule_own) == GSG_SCHEDULE_FUSED;  // fused launches do not split
+    const bool solo_ok = whole ? busy == 0 : busy <= SOLO_BATCH_US;
     // cells and wavefronts per (D, k, system) class: a launch of too few cells runs the plan
     // kernel (FP64, SEG64_MIN_CELLS), one of few wavefronts splits directions (a class's own
     // count, its launches follow each other whatever runs beside them, but doubled: what
     // runs beside them fills the chip as well)
     std::map<std::tuple<int, int, int>, std::pair<int64_t, int64_t>> launch_of;
-    const bool whole = fp32 && resolve_schedule(schedule_own) == GSG_SCHEDULE_FUSED;  // fused launches do not split
     for (SolveState* S : solves)
       if (!(solo_ok && solo_of(*S).on)) {
         auto& q = launch_of[std::make_tuple(S->T->D, S->T->k, S->desc.sys)];

@@ -42,3 +42,24 @@ def test_resident_solves_have_their_own_entry(g, gpu, prec):
     assert w["launches"] == 2 and w["algo_bytes"] == N4 * (160 * 300 + 2 * (16 + 3 * lo))
     staged = [s for key, s in st.items() if key[3] != 4]
     assert len(staged) == 1 and staged[0]["launches"] == 4 * 300 and staged[0]["dofs"] == g.get_size(2, 3, 9)
+
+
+@pytest.mark.parametrize("when", ["before", "after"])
+def test_fused_batches_keep_small_solves_in_the_launch(g, gpu, when):
+    """Beside others a small solve runs in the fused launch, resident only alone; a schedule
+    set after the first steps counts from then on."""
+    print(f"[gpu] fused batch, schedule set {when} the first steps", flush=True)
+    for solves, resident in (([(2, 3, 5), (2, 3, 9)], False), ([(2, 3, 5), (2, 3, 4)], True)):
+        b = g.Batch("fp32")
+        if when == "before":
+            b.schedule("fused")
+        for D, k, n in solves:
+            y0 = np.random.default_rng(n).standard_normal(g.get_size(D, k, n))
+            b.add("transport", D, k, n, y0, 0.02 * 2.0 ** -n, 20, a=[0.3, -0.8])
+        b.step(4)
+        b.schedule("fused")
+        b.profile(True)
+        b.step(4)
+        assert ([s["variant"] for s in b.kernel_stats()] == [4]) == resident
+        assert all((s["variant"] == 4) == resident for s in b.kernel_stats())
+        b.close()
