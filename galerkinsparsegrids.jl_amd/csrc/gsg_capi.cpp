@@ -908,9 +908,12 @@ static bool graphs_enabled() {
 // Captured RK4 steps: a graph of CHUNK steps and one of a single step, replayed to cover
 // any step count (CHUNK steps per graph launch amortise the launch cost of small
 // grids).  The first call after a reset captures at once when it has at least `first_min`
-// steps and runs eagerly otherwise.  For a batch that is CHUNK steps: 17 classes on four
-// streams took 1.9 ms to capture and 0.83 ms a replayed step, 1.40 an eager one.  The graphs hold kernel
-// and event nodes only (no memset or copy nodes).
+// steps and runs eagerly otherwise.  A batch captures at once when 4 CHUNK steps are to come:
+// capturing and releasing the graphs costs milliseconds.  A whole batch of FP64 solves with wave systems,
+// us eager / captured: 6 solves, 8 steps 1237 / 1510, 32 steps 2653 / 2574; 16 solves, 8 steps
+// 3998 / 6988, 32 steps 11159 / 11434, 64 steps 20456 / 17008; 48 solves, 16 steps 7371 /
+// 8817, 32 steps 12593 / 12700.  The graphs hold kernel and event nodes only (no memset or
+// copy nodes).
 struct StepGraphs {
   static constexpr int CHUNK = 8;
   hipGraph_t g[2] = {nullptr, nullptr};
@@ -2310,7 +2313,8 @@ struct Scheduler {
   StepGraphs graphs;
   void reset_graph() { graphs.reset(); }
 
-  void steps(int64_t n) {
+  // n steps; ahead: at least so many, these among them, are known to come before a rebuild
+  void steps(int64_t n, int64_t ahead) {
     if (n <= 0) return;
     if (profile) {
       enqueue(n);
@@ -2318,7 +2322,7 @@ struct Scheduler {
     }
     if (groups.size() > 1 && lanes_enabled() && schedule != GSG_SCHEDULE_FUSED)
       init_lanes();  // no stream creation inside a capture
-    graphs.run(n, stream, StepGraphs::CHUNK, [&](int64_t k, hipStream_t) { enqueue(k); });
+    graphs.run(n, stream, ahead >= 4 * StepGraphs::CHUNK ? 0 : n + 1, [&](int64_t k, hipStream_t) { enqueue(k); });
   }
 
   void enqueue(int64_t n) {
@@ -2438,7 +2442,7 @@ static void batch_advance(gsg_batch* b, int64_t steps) {
   while (steps > 0 && !b->active.empty()) {
     int64_t phase = steps;
     for (size_t i : b->active) phase = std::min(phase, b->solves[i]->nsteps - b->solves[i]->done);
-    b->sched.steps(phase);
+    b->sched.steps(phase, phase);
     if (b->sched.profile) {
       HIPC(hipStreamSynchronize(b->stream));
       b->sched.collect();
@@ -2767,8 +2771,9 @@ static void server_loop(gsg_server* S) {
       res = S->resident;
     }
     if (res.empty()) continue;
-    int64_t tick = std::max<int32_t>(1, S->cfg.steps_per_tick);
-    for (Request* r : res) tick = std::min(tick, r->nsteps - r->done);
+    int64_t left = INT64_MAX;  // until the first of the requests finishes
+    for (Request* r : res) left = std::min(left, r->nsteps - r->done);
+    const int64_t tick = std::min<int64_t>(std::max<int32_t>(1, S->cfg.steps_per_tick), left);
     const auto t0 = Clock::now();
     try {  // nothing may escape the worker thread: a failure fails the resident requests
       if (S->dirty) {
@@ -2788,7 +2793,7 @@ static void server_loop(gsg_server* S) {
           S->retired.clear();
         }
       }
-      if (tick > 0) S->sched.steps(tick);
+      if (tick > 0) S->sched.steps(tick, left);
       HIPC(hipStreamSynchronize(S->stream));
     } catch (const std::exception& e) {
       std::lock_guard<std::mutex> g(S->mu);
