@@ -757,11 +757,23 @@ constexpr int64_t SEG64_MIN_CELLS = 65536;
 // D = 4, k = 3: 5248 25.1 / 21.6, 10496 34.0 / 35.9; D = 4, k = 4: 3040 12.4 / 11.4,
 // 6080 17.1 / 19.3; FP64 D = 4, k = 4: 20992 72.7 / 70.2, 41984 150 / 158; D = 3, k = 4:
 // 688 14.4 / 9.6, 9728 26.5 / 26.5.
-static int64_t dsplit_waves(int32_t kernel, int D, int K, bool fp32) {
+//   The plan kernel serves shapes whose lists are short (D = 5, 6 at small n): the longest
+// direction saves little there, and the D-fold wavefronts, each with its own indexing, cost
+// more the more an entry moves.  So its line is k wavefronts <= 3500 (FP32) or 5400 (FP64)
+// mean entries of a list, and at most 8192 wavefronts.  Over its 245 grids of 60 to 3 M
+// coefficients that gives 0.96 or better everywhere and passes by 1.03 at most.  us an FP64 RK
+// stage without / with: D = 6, k = 5, n = 1 (1709 wavefronts, 1.3 entries) 13.6 / 17.0; D = 5, k =
+// 5, n = 3 (4688, 2.3) 29.7 / 40.9; D = 6, k = 3, n = 3 (1572, 2.1) 16.9 / 13.9; D = 3, k = 5, n = 7
+// (3313, 5.9) 43 / 29.
+static int64_t dsplit_waves(const Tables& T, int32_t kernel, bool fp32) {
   if (fp32 && (kernel == KERNEL_SEG || kernel == KERNEL_SEG_ALT)) return 8192;
-  if (kernel == KERNEL_PLAN) return D <= 6 && K <= 5 ? 8192 : -1;
+  if (kernel == KERNEL_PLAN) {
+    if (T.D > 6 || T.k > 5) return -1;
+    const double list = double(T.plan.ent.size() / 2) / double(T.plan.ptr.size() - 1);
+    return std::min<int64_t>(8192, int64_t((fp32 ? 3500.0 : 5400.0) * list / T.k));
+  }
   if (kernel != KERNEL_DIRECT) return -1;
-  return fp32 ? 4096 : direct_ok(D, K) ? 24576 : 8192;
+  return fp32 ? 4096 : direct_ok(T.D, T.k) ? 24576 : 8192;
 }
 // The FP64 fiber kernel walks its tile's batches with barriers between them: it wins in
 // launches bound by throughput at D = 3 and on the coarse grids of D = 2, and loses where the
@@ -781,7 +793,7 @@ static LdsShape lds_shape(const Tables& T, bool fp32, int64_t launch_cells, int6
   if (L.kernel == KERNEL_FIBER && !c.asked &&
       (launch_waves <= FIBER_MIN_WAVES || (!c.entry && (T.D == 1 || T.D > 3 || (T.D == 2 && T.n > 6)))))
     L = LdsShape{};
-  if (T.D > 1) L.dsplit = launch_waves <= dsplit_waves(L.kernel, T.D, T.k, fp32);
+  if (T.D > 1) L.dsplit = launch_waves <= dsplit_waves(T, L.kernel, fp32);
   return L;
 }
 static int64_t grid_cells(const Tables& T) { return T.lt.N / Tables::ipow_i(T.k, T.D); }
