@@ -531,9 +531,9 @@ __global__ __launch_bounds__(TILE) void k_fiber(LaunchArgs a) {
     const int32_t E0 = uni(sld(lb));
     const int32_t ne = uni(sld(lb + CPT * D)) - E0;
     for (int32_t q = tid; q < ns; q += TILE)
-      soff[q] = uint32_t(gld(S.t.slot_off + s0 + q)) + uint32_t(gld(S.t.slot_dir + s0 + q) * dstride);
-    for (int32_t q = tid; q < ne; q += TILE) entl[q] = gld(S.t.tile_ent + E0 + q);
-    for (int32_t q = tid; q <= CPT * D; q += TILE) lptl[q] = gld(lb + q) - E0;
+      soff[q] = uint32_t(S.t.slot_off[s0 + q]) + uint32_t(S.t.slot_dir[s0 + q] * dstride);
+    for (int32_t q = tid; q < ne; q += TILE) entl[q] = S.t.tile_ent[E0 + q];
+    for (int32_t q = tid; q <= CPT * D; q += TILE) lptl[q] = lb[q] - E0;
     __syncthreads();
     // input cells: chunk w of the batch -> chunk w % XCH of slot w / XCH, from the
     // 16-byte boundary at or below the slot's cell
@@ -611,13 +611,13 @@ __global__ __launch_bounds__(TILE) void k_fiber(LaunchArgs a) {
 #pragma unroll
       for (int e = 0; e < D; ++e) s += T(S.coef[e]) * yq[e * KD];
       if (a.op == OP_APPLY_SUM)
-        gst((double*)a.yout + i, double(s));
+        ((double*)a.yout)[i] = double(s);
       else
         rk_update<T>(S, a.stage, i, double(s));
     } else if (a.op == OP_APPLY_GRAD || a.op == OP_RK_WAVE_GRAD) {
       T* w = a.op == OP_RK_WAVE_GRAD ? (T*)S.w : (T*)a.yout;
 #pragma unroll
-      for (int e = 0; e < D; ++e) gst(w + int64_t(e) * N + i, yq[e * KD]);
+      for (int e = 0; e < D; ++e) w[int64_t(e) * N + i] = yq[e * KD];
     } else {
       T s = T(0);
 #pragma unroll
