@@ -1500,11 +1500,16 @@ int gsg_csc_create(int64_t m, int64_t n, const int64_t* colptr, const int64_t* r
     }
     upload(op->v32, v32);
     if (op->fp32) op->x32.alloc(size_t(n) * 4);
-    // row blocks of k_csr: consecutive rows, at most 256 of them and CSR_ENT entries, or one row
+    // row blocks of k_csr: consecutive rows, at most 256 of them and CSR_ENT entries, or one
+    // row; a thread a row where the rows have about one entry and none has many
+    int64_t longest = 0;
     std::vector<int32_t> blk{0};
-    for (int64_t i = 1; i <= m; ++i)
+    for (int64_t i = 1; i <= m; ++i) {
+      longest = std::max(longest, rp[i] - rp[i - 1]);
       if (i == m || i - blk.back() == 256 || rp[i + 1] - rp[blk.back()] > CSR_ENT) blk.push_back(int32_t(i));
-    upload(op->blk, blk);
+    }
+    const bool rows = 2 * nnz <= 3 * m && longest <= 8;
+    if (!rows) upload(op->blk, blk);
     op->csr = DevCsr{m,
                      n,
                      nnz,
@@ -1513,7 +1518,7 @@ int gsg_csc_create(int64_t m, int64_t n, const int64_t* colptr, const int64_t* r
                      op->v64.as<double>(),
                      op->v32.as<float>(),
                      op->blk.as<int32_t>(),
-                     int32_t(blk.size() - 1)};
+                     int32_t(rows ? (m + 255) / 256 : int64_t(blk.size()) - 1)};
     *out = op.release();
   });
 }

@@ -358,7 +358,7 @@ struct DevCsr {
   const int32_t* ci;
   const double* v64;
   const float* v32;  // 2 nnz: hi values, then lo values (v64 - hi)
-  const int32_t* blk;  // nblk + 1 first rows of the row blocks (csr_blocks)
+  const int32_t* blk;  // nblk + 1 first rows of the row blocks (null: nblk blocks of 256 rows, a thread a row)
   int32_t nblk;
 };
 // x32 (float only): the rounded vector, read in place of x

@@ -2428,12 +2428,26 @@ __global__ void k_to_f64(const float* __restrict__ x, double* __restrict__ y, in
 // is read.  What bounded the thread per row was its own stride: 64 rows' entries a load
 // instruction, 64 cache lines.  Measured on the gradient of D = 3, k = 3, n = 6 (18,576 rows,
 // 0.93 M entries): 41.5 us before, 6.9 now; 3,000 rows with two dense ones: 365 / 55 us.
+// Rows of about one entry each gain nothing from it and wait for the block's bounds and the
+// LDS: they stay on a thread a row (A.blk null; 50,000 rows of one entry 2.9 / 2.5 us).
 template <typename T, typename TX>
 __global__ __launch_bounds__(256) void k_csr(DevCsr A, const TX* __restrict__ x, double* __restrict__ y) {
   constexpr bool HL = sizeof(T) == 4;
   __shared__ T sv[CSR_ENT], sl[HL ? CSR_ENT : 1], sx[CSR_ENT];
   const T* v = vals_of_csr<T>(A);
   const int tid = threadIdx.x;
+  if (!A.blk) {
+    const int64_t i = blockIdx.x * int64_t(blockDim.x) + tid;
+    if (i >= A.m) return;
+    T s = T(0), l = T(0);
+    for (int64_t p = A.rp[i]; p < A.rp[i + 1]; ++p) {
+      const T xv = T(x[A.ci[p]]);
+      s += v[p] * xv;
+      if constexpr (HL) l += v[A.nnz + p] * xv;
+    }
+    y[i] = HL ? double(s) + double(l) : double(s);
+    return;
+  }
   const int64_t r0 = A.blk[blockIdx.x], r1 = A.blk[blockIdx.x + 1];
   const int64_t e0 = A.rp[r0], e1 = A.rp[r1];
   const int64_t row = r0 + tid;
