@@ -1701,10 +1701,13 @@ static void launch_seg_op(const LaunchArgs& a, hipStream_t s) {
   // runs one direction per grid row: measured on the 2 + 2 dimensional Vlasov derivative
   // (k = 2, n = 8)
   const dim3 ggrid(grid.x, OPT == OP_APPLY_GRAD && grid.x < 1024 ? unsigned(a.gdirs ? a.gdirs : DT) : 1u);
-  if (a.dsplit)
-    hipLaunchKernelGGL((k_seg_ds<DT, KT, OPT, STG>), dim3(unsigned(a.ntiles / seg_cpw(DT, KT))), dim3(64 * DT), 0, s, a);
-  else
-    hipLaunchKernelGGL((k_seg<DT, KT, OPT, STG, EBX>), ggrid, dim3(TILE), 0, s, a);
+  if constexpr (DT > 1) {  // one direction does not split
+    if (a.dsplit) {
+      hipLaunchKernelGGL((k_seg_ds<DT, KT, OPT, STG>), dim3(unsigned(a.ntiles / seg_cpw(DT, KT))), dim3(64 * DT), 0, s, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_seg<DT, KT, OPT, STG, EBX>), ggrid, dim3(TILE), 0, s, a);
 }
 template <int DT, int KT, int OPT, int EBX = 0>
 static void launch_seg_stage(const LaunchArgs& a, hipStream_t s) {
@@ -1720,7 +1723,7 @@ static void launch_seg_stage(const LaunchArgs& a, hipStream_t s) {
 // the rule's)
 template <int DT, int KT>
 static hipError_t launch_seg_alt(const LaunchArgs& a, hipStream_t s) {
-  if (a.ntiles % ((a.dsplit ? 1 : SEG_WAVES) * seg_cpw(DT, KT))) return hipErrorInvalidValue;  // the host pads
+  if (a.ntiles % ((DT > 1 && a.dsplit ? 1 : SEG_WAVES) * seg_cpw(DT, KT))) return hipErrorInvalidValue;  // the host pads
   constexpr int E = seg_eb_alt(DT, KT);
   switch (a.op) {
     case OP_RK_SUM: launch_seg_stage<DT, KT, OP_RK_SUM, E>(a, s); break;
@@ -1733,7 +1736,7 @@ static hipError_t launch_seg_alt(const LaunchArgs& a, hipStream_t s) {
 
 template <int DT, int KT>
 static hipError_t launch_seg(const LaunchArgs& a, hipStream_t s) {
-  if (a.ntiles % ((a.dsplit ? 1 : SEG_WAVES) * seg_cpw(DT, KT))) return hipErrorInvalidValue;  // the host pads
+  if (a.ntiles % ((DT > 1 && a.dsplit ? 1 : SEG_WAVES) * seg_cpw(DT, KT))) return hipErrorInvalidValue;  // the host pads
   switch (a.op) {
     case OP_APPLY_SUM: launch_seg_op<DT, KT, OP_APPLY_SUM, 0>(a, s); break;
     case OP_APPLY_GRAD: launch_seg_op<DT, KT, OP_APPLY_GRAD, 0>(a, s); break;
