@@ -625,6 +625,12 @@ def main():
     if "plain_fp64_solve_by_solve_dof_updates_per_s" in extras:
         out["fp32_batched_over_plain_fp64"] = value / extras["plain_fp64_solve_by_solve_dof_updates_per_s"]
     print(json.dumps(out), flush=True)
+    # the metric's precision: a rate of results further off than that is none
+    errs = {"batched": rel_max}
+    if "max" in extras.get("serving", {}).get("fp32_rel_l2_vs_fp64", {}):
+        errs["served"] = extras["serving"]["fp32_rel_l2_vs_fp64"]["max"]
+    if any(not e <= 1e-6 for e in errs.values()):
+        sys.exit(f"FP32 results further than 1e-6 from FP64 (relative L2): {errs}")
 
 
 if __name__ == "__main__":
