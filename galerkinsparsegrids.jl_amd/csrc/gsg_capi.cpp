@@ -919,18 +919,14 @@ static bool graphs_enabled() {
 
 // Captured RK4 steps: a graph of CHUNK steps and one of a single step, replayed to cover
 // any step count (CHUNK steps per graph launch amortise the launch cost of small
-// grids).  The first call after a reset captures at once when it has at least `first_min`
-// steps and runs eagerly otherwise.  A batch captures at once when 4 CHUNK steps are to come:
-// capturing and releasing the graphs costs milliseconds.  A whole batch of FP64 solves with wave systems,
-// us eager / captured: 6 solves, 8 steps 1237 / 1510, 32 steps 2653 / 2574; 16 solves, 8 steps
-// 3998 / 6988, 32 steps 11159 / 11434, 64 steps 20456 / 17008; 48 solves, 16 steps 7371 /
-// 8817, 32 steps 12593 / 12700.  The graphs hold kernel and event nodes only (no memset or
-// copy nodes).
+// grids).  The caller says whether a call is worth capturing for, as capturing and releasing the
+// graphs costs milliseconds; once captured, every call replays.  The graphs hold kernel and
+// event nodes only (no memset or copy nodes).
 struct StepGraphs {
   static constexpr int CHUNK = 8;
   hipGraph_t g[2] = {nullptr, nullptr};
   hipGraphExec_t e[2] = {nullptr, nullptr};  // [0]: 1 step, [1]: CHUNK steps
-  bool used = false;
+  bool used = false;  // since the last reset
   void reset() {
     CaptureGuard cg(g_capture_mu);
     for (int i = 0; i < 2; ++i) {
@@ -942,13 +938,13 @@ struct StepGraphs {
     used = false;
   }
   ~StepGraphs() { reset(); }
+  bool captured() const { return e[1] != nullptr; }
   // run `n` steps on stream s; enqueue(k, stream) issues k steps eagerly
   template <typename F>
-  void run(int64_t n, hipStream_t s, int64_t first_min, F&& enqueue) {
+  void run(int64_t n, hipStream_t s, bool capture, F&& enqueue) {
     if (n <= 0) return;
-    const bool first = !used;
     used = true;
-    if (!graphs_enabled() || (first && n < first_min)) {
+    if (!graphs_enabled() || (!captured() && !capture)) {
       enqueue(n, s);
       return;
     }
@@ -1145,7 +1141,7 @@ static void vlasov_rk_steps(gsg_op* op, double dt, int64_t n, hipStream_t s) {
   // FP32: the stage update also writes the float copy of the next stage input (and of
   // the new state), so only the first stage of a run converts
   float* x32 = op->fp32 ? op->x32.as<float>() : nullptr;
-  op->vgraphs.run(n, s, 2 * StepGraphs::CHUNK, [&](int64_t k, hipStream_t st) {
+  op->vgraphs.run(n, s, op->vgraphs.used || n >= 2 * StepGraphs::CHUNK, [&](int64_t k, hipStream_t st) {
     for (int64_t i = 0; i < k; ++i)
       for (int stage = 1; stage <= 4; ++stage) {
         // the last n2m sweep applies the stage update (no right-hand-side vector)
@@ -1762,7 +1758,7 @@ static void op_rk_steps(gsg_op* op, int64_t nsteps, hipStream_t s) {
     launch_solo_steps(T.D, T.k, op->fp32, op->solo, op->d_rkdesc.as<SolveDesc>(), nullptr, 1, nsteps, s);
     return;
   }
-  op->rkgraphs.run(nsteps, s, 2 * StepGraphs::CHUNK, [&](int64_t k, hipStream_t st) {
+  op->rkgraphs.run(nsteps, s, op->rkgraphs.used || nsteps >= 2 * StepGraphs::CHUNK, [&](int64_t k, hipStream_t st) {
     for (int64_t i = 0; i < k; ++i)
       launch_rk_step(T.D, T.k, op->fp32, sys, op->d_rkdesc.as<SolveDesc>(), op->d_tiles.as<Tile>(), op->n_tiles,
                      op->shape, st);
@@ -2330,8 +2326,23 @@ struct Scheduler {
   StepGraphs graphs;
   void reset_graph() { graphs.reset(); }
 
-  // n steps; ahead: at least so many, these among them, are known to come before a rebuild
-  void steps(int64_t n, int64_t ahead) {
+  // Whether to capture the steps when `horizon` of them will run before the next rebuild (the
+  // first call also goes by its own count, as no other may follow).  A whole batch of FP64 solves
+  // with wave systems, us eager / captured: 6 solves, 8 steps 1237 / 1510, 32 steps 2653 / 2574;
+  // 16 solves, 8 steps 3998 / 6988, 32 steps 11159 / 11434, 64 steps 20456 / 17008; 48 solves, 16
+  // steps 7371 / 8817, 32 steps 12593 / 12700.
+  bool worth_capture(int64_t horizon, int64_t call) const {
+    return std::min(horizon, graphs.used ? horizon : call) >= 4 * StepGraphs::CHUNK;
+  }
+  // steps until the solves that finish hold more than 1 / share of the built DoFs, of which `idle`
+  // do already: the next rebuild (left: steps to go and length of the others)
+  static int64_t horizon(std::vector<std::pair<int64_t, int64_t>> left, int64_t idle, int64_t built, int64_t share) {
+    std::sort(left.begin(), left.end());
+    for (const auto& q : left)
+      if (share * (idle += q.second) > built) return q.first;
+    return left.empty() ? 0 : left.back().first;
+  }
+  void steps(int64_t n, bool capture) {
     if (n <= 0) return;
     if (profile) {
       enqueue(n);
@@ -2339,7 +2350,7 @@ struct Scheduler {
     }
     if (groups.size() > 1 && lanes_enabled() && schedule != GSG_SCHEDULE_FUSED)
       init_lanes();  // no stream creation inside a capture
-    graphs.run(n, stream, ahead >= 4 * StepGraphs::CHUNK ? 0 : n + 1, [&](int64_t k, hipStream_t) { enqueue(k); });
+    graphs.run(n, stream, capture, [&](int64_t k, hipStream_t) { enqueue(k); });
   }
 
   void enqueue(int64_t n) {
@@ -2459,7 +2470,21 @@ static void batch_advance(gsg_batch* b, int64_t steps) {
   while (steps > 0 && !b->active.empty()) {
     int64_t phase = steps;
     for (size_t i : b->active) phase = std::min(phase, b->solves[i]->nsteps - b->solves[i]->done);
-    b->sched.steps(phase, phase);
+    bool capture = false;
+    if (!b->sched.graphs.captured()) {
+      std::vector<std::pair<int64_t, int64_t>> left;
+      int64_t built = 0, idle = 0;
+      for (size_t i : b->scheduled) {
+        const BatchSolve& s = *b->solves[i];
+        built += s.st.len;
+        if (s.done < s.nsteps)
+          left.emplace_back(s.nsteps - s.done, s.st.len);
+        else
+          idle += s.st.len;
+      }
+      capture = b->sched.worth_capture(b->sched.horizon(left, idle, built, 4), steps);
+    }
+    b->sched.steps(phase, capture);
     if (b->sched.profile) {
       HIPC(hipStreamSynchronize(b->stream));
       b->sched.collect();
@@ -2788,9 +2813,8 @@ static void server_loop(gsg_server* S) {
       res = S->resident;
     }
     if (res.empty()) continue;
-    int64_t left = INT64_MAX;  // until the first of the requests finishes
-    for (Request* r : res) left = std::min(left, r->nsteps - r->done);
-    const int64_t tick = std::min<int64_t>(std::max<int32_t>(1, S->cfg.steps_per_tick), left);
+    int64_t tick = std::max<int32_t>(1, S->cfg.steps_per_tick);
+    for (Request* r : res) tick = std::min(tick, r->nsteps - r->done);
     const auto t0 = Clock::now();
     try {  // nothing may escape the worker thread: a failure fails the resident requests
       if (S->dirty) {
@@ -2810,7 +2834,14 @@ static void server_loop(gsg_server* S) {
           S->retired.clear();
         }
       }
-      if (tick > 0) S->sched.steps(tick, left);
+      bool capture = false;
+      if (!S->sched.graphs.captured()) {
+        std::vector<std::pair<int64_t, int64_t>> to_go;
+        for (Request* r : res) to_go.emplace_back(r->nsteps - r->done, r->len);
+        const int64_t h = S->sched.horizon(to_go, S->idle_dofs, S->built_dofs, 10);
+        capture = S->sched.worth_capture(h, h);
+      }
+      if (tick > 0) S->sched.steps(tick, capture);
       HIPC(hipStreamSynchronize(S->stream));
     } catch (const std::exception& e) {
       std::lock_guard<std::mutex> g(S->mu);

@@ -8,6 +8,9 @@
         the Vlasov workload to profile: free streaming on the 2 + 2 dimensional phase
         space, k = 2, n = 8, f0 = Maxwellian in v times (1 + 0.1 cos 2 pi x1), RK4 steps
         on the device
+    python galerkinsparsegrids.jl_amd/rocprof_summary.py solve transport 4 4 9 fp64 [--steps 64]
+        one solve to profile: RK4 steps of a transport or wave system of (D, k, n) on the
+        device, random state
     python galerkinsparsegrids.jl_amd/rocprof_summary.py projection [--n 9]
         the initial-data projection to profile: vcoeffs_DG on the device at D = 4, k = 4
         (default rule q = 8, 16^4 nodes per cell) of a non-separable f evaluated by
@@ -88,6 +91,23 @@ def cmd_vlasov(a):
         torch.cuda.synchronize()
         print(f"vlasov {prec}: {1e3 * (time.perf_counter() - t0) / a.steps:.3f} ms per RK4 step", flush=True)
         op.close()
+
+
+def cmd_solve(a):
+    from pathlib import Path
+
+    import torch
+    sys.path.insert(0, str(Path(__file__).resolve().parent.parent))
+    import __graft_entry__ as ge
+    g = ge.load_package()
+    torch.cuda.set_device(0)
+    op = (g.wave_matrix(a.D, a.k, a.n, precision=a.precision) if a.kind == "wave" else
+          g.transport_matrix(a.D, a.k, a.n, [0.7, -0.3, 0.5, 0.2, 0.9, -0.4][:a.D], precision=a.precision))
+    y = torch.randn(op.len, dtype=torch.float64, device="cuda")
+    op.rk4(y, 1e-5, a.steps)
+    torch.cuda.synchronize()
+    op.close()
+    print(f"{a.kind} D={a.D} k={a.k} n={a.n} {a.precision}: {a.steps} steps", flush=True)
 
 
 def cmd_projection(a):
@@ -197,6 +217,12 @@ def main():
     v = sub.add_parser("vlasov")
     v.add_argument("--steps", type=int, default=50)
     v.add_argument("precision", nargs="*", choices=["fp32", "fp64"])
+    so = sub.add_parser("solve")
+    so.add_argument("kind", choices=["transport", "wave"])
+    for name in ("D", "k", "n"):
+        so.add_argument(name, type=int)
+    so.add_argument("precision", choices=["fp64", "fp32"])
+    so.add_argument("--steps", type=int, default=64)
     pj = sub.add_parser("projection")
     pj.add_argument("--n", type=int, default=9)
     s = sub.add_parser("stats")
@@ -215,7 +241,7 @@ def main():
     m.add_argument("--cus", type=int, default=256)
     m.add_argument("--xcds", type=int, default=8)
     a = ap.parse_args()
-    {"copy": cmd_copy, "vlasov": cmd_vlasov, "projection": cmd_projection, "stats": cmd_stats,
+    {"copy": cmd_copy, "vlasov": cmd_vlasov, "solve": cmd_solve, "projection": cmd_projection, "stats": cmd_stats,
      "traffic": cmd_traffic, "pmc": cmd_pmc}[a.cmd](a)
 
 
