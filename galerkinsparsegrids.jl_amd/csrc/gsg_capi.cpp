@@ -236,6 +236,8 @@ static std::vector<Tile> xcd_split(const std::vector<Tile>& tiles, size_t chunk 
 // D = 3, k = 4, n = 9, wave: 29.6 / 23.8; FP32 D = 4, k = 4, n = 8: 33.4 / 30.3.  Launches of
 // more than 64 K wavefronts keep the old order (256-solve batch in FP64: 2% slower in the new).
 constexpr size_t LONG_FIRST_WAVES = 65536;
+// The classes count rounds of four entries for every kernel: the FP64 direct kernel takes its
+// entries one by one, but the classes only have to rank the wavefronts.
 static std::vector<Tile> xcd_split_work(const std::vector<Tile>& tiles, int D, size_t chunk, size_t unit, int per_round) {
   const size_t nu = tiles.size() / unit, per = (nu + NXCD - 1) / NXCD;
   std::vector<uint8_t> cls(nu);
@@ -609,6 +611,8 @@ struct SolveState {
     const int64_t len = kind == GSG_OP_WAVE ? 2 * N : N;
     return len + (fp32 && kind == GSG_OP_WAVE ? N : 0);
   }
+  // the vectors' bytes; the 256-byte starts of init() add less than 1.5 KB a solve, which is less
+  // than the allocator's own rounding
   static size_t footprint(int kind, int D, int64_t N, bool fp32) {
     const int64_t len = kind == GSG_OP_WAVE ? 2 * N : N;
     const size_t es = fp32 ? 4 : 8;
@@ -2114,9 +2118,12 @@ struct Scheduler {
     auto solo_of = [&](const SolveState& S) {
       return solo_shape(*S.T, lds_shape(*S.T, fp32), fp32, S.desc.sys == SYS_WAVE);
     };
-    // Resident solves only beside little else: every other class's launches of a large batch
-    // cover its small solves as well, and a resident solve holds a compute unit (256 uneven
-    // solves: 1.98 ms a step with the small ones resident, 1.91 without).
+    // Resident solves only beside little else (SOLO_BATCH_US of stage_us): every other class's
+    // launches of a large batch cover its small solves as well, and a resident solve holds a
+    // compute unit.  us a step staged / resident, 8 or 64 small solves beside D = 4, k = 4, n = 5
+    // ones of 45 us 151 / 67 (FP32) and 146 / 69 (FP64), 124 us 182 / 102 and 174 / 141, 400 us 332 /
+    // 318 and 454 / 440; beside D = 3, k = 3, n = 7 ones of 40 to 400 us 0.95 to 1.02 times; 256
+    // uneven solves 1.91 / 1.98 ms.  The line is on the safe side of where they meet.
     double busy = 0;
     for (SolveState* S : solves)
       if (!solo_of(*S).on) busy += stage_us(double(S->N), S->T->D, S->T->k, S->desc.sys);
